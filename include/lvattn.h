@@ -106,7 +106,8 @@ int lv_store_latents(const void* latent, int64_t latent_stride_t, int32_t num_to
  * Query j of a row with lq queries and lk keys sees keys 0 .. lk-lq+j (bottom-right causal).
  * A row with no keys gets a zero output.
  * max_seqlen_k (at most 2^30) bounds every row's key length (block-table width * block_size will do); it sizes the
- * split-K grid so a captured graph needs no length read back. num_tokens is T (it sizes the work list).
+ * split-K grid and workspace so a captured graph needs no length read back (the splits themselves are sized on the
+ * device, from the lengths). num_tokens is T (it sizes the work list).
  * workspace: caller-owned device memory of at least lv_paged_attention_workspace_bytes(...) bytes for the same
  * arguments; its contents need no initialisation.
  * schedule (a step with prompt rows): LV_SCHEDULE_OVERLAP runs the prompt tiles on part of the CUs beside the
@@ -164,8 +165,8 @@ typedef struct lv_launch_info {
   int32_t prompt_workgroups;
   int32_t kv_heads_per_item;  /* 1, or 2: a decode item reads two adjacent kv heads of each token */
   int32_t two_streams;
-  int32_t keys_per_split;     /* keys per decode item */
-  int32_t max_splits;         /* the most decode items one row is split into */
+  int32_t keys_per_split;     /* keys per decode item at least (the plan sizes them from the rows' lengths) */
+  int32_t max_splits;         /* the most decode items one row may be split into */
   int32_t splitk_merge;       /* 1: rows are split over several items; each row's last split to finish merges
                                  them (log-sum-exp) inside the decode launch */
 } lv_launch_info;

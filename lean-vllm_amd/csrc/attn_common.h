@@ -8,6 +8,15 @@ namespace lv {
 constexpr int kPrefillKeys = 64;  // keys per prompt tile
 constexpr int kPrefillRows = 128;  // (position, head) query rows per prompt item, 32 per wave
 
+// Counts of a work list, as plan_kernel leaves them.
+enum : int {
+  kPlanDecodes = 0,  // decode items
+  kPlanPrompts = 1,  // prompt items
+  kPlanTicket = 2,   // next decode item of a persistent launch
+  kPlanDone = 3,     // and its count of workgroups done
+  kPlanSplit = 4,    // keys per decode item
+};
+
 struct AttnParams {
   const char* q;
   int64_t q_st, q_sh;  // bytes
@@ -29,13 +38,13 @@ struct AttnParams {
   int64_t o_st, o_sh;  // bytes
   float* lse;          // optional natural log-sum-exp of prompt rows [T, Hq]
   int64_t lse_st, lse_sh;  // elements
-  int32_t split;       // S: keys per decode item
-  int32_t max_splits;
-  float* part_o;    // [rows][hq][max_splits][D] normalised partial outputs
-  float* part_lse;  // [rows][hq][max_splits] log2-sum-exp2 of the partials
-  const int2* items;
-  const int32_t* n_items;  // [0]: list length, [1]: prompt items at its head
-  int32_t* ticket;         // next decode item of a persistent launch (zeroed by the plan kernel)
+  const int32_t* part_base;  // [rows] first partial slot of a split row
+  float* part_o;             // [slots][hq][D] normalised partial outputs
+  float* part_lse;           // [slots][hq] log2-sum-exp2 of the partials
+  const int2* prompts;       // the work lists: prompt items, decode items
+  const int2* items;         // and their counts (kPlan*); null in a step without a list
+  const int32_t* n_items;
+  int32_t* ticket;           // &n_items[kPlanTicket]
   // Split rows (listed steps only): per (row, item head group), the count of its splits that have written their
   // partials (zeroed by the plan kernel); the last to arrive merges them and puts the count back to zero.
   int32_t* merge_count;

@@ -30,8 +30,10 @@ constexpr int kOverlapCusMaxPct = 75;  // at most this percent when the caller s
 constexpr int kDecodeWgs = 2;         // persistent decode workgroups per CU outside the overlap
 constexpr int kOverlapDecodeWgs = 3;  // persistent decode workgroups per CU beside a mixed step's prompt workgroups
                                       // (at most: pair items at D = 128 fit two)
-constexpr int kSplitTarget = 4096;    // decode items (x kv heads x query-head groups) a split-K grid aims for
+constexpr int kSplitTarget = 4096;    // decode items (x kv heads x query-head groups) a step with split rows aims for
+constexpr int kMaxRowSplits = 128;    // and splits per row on average at most
 constexpr int kMinSplit = 256;        // keys per decode item at least
+constexpr int kSplitStep = 64;        // and a multiple of this: one tile of every wave
 constexpr int kSmallStepRounds = 8;   // a mixed step of at most this many GPU-fulls of workgroups is one launch
 
 // ---------------------------------------------------------------------------------------------------------
@@ -71,34 +73,41 @@ __device__ __forceinline__ void coherent_store(float* ptr, float v) {
 __device__ __forceinline__ float coherent_load(const float* ptr) {
   return __hip_atomic_load(ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Two adjacent floats (8-byte aligned) in one access.
+__device__ __forceinline__ void coherent_store2(float* ptr, float a, float b) {
+  const uint64_t v = (uint64_t)__float_as_uint(a) | (uint64_t)__float_as_uint(b) << 32;
+  __hip_atomic_store(reinterpret_cast<uint64_t*>(ptr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void coherent_load2(const float* ptr, float& a, float& b) {
+  const uint64_t v =
+      __hip_atomic_load(reinterpret_cast<const uint64_t*>(ptr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  a = __uint_as_float((uint32_t)v);
+  b = __uint_as_float((uint32_t)(v >> 32));
+}
 
-// Merge of a split row's partial outputs for dims d0 .. d0 + PER - 1 of query head `head`, written to the output row
-// `tok`: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M). The partials are read kMergeBatch splits at a time, every
-// load of a batch issued before the first is used, with the max and the sums carried from batch to batch (a long
-// row's 32 splits are two round trips to memory, not 64). Each output element's arithmetic depends only on its own
-// head and dim, so any spread of the elements over threads gives the same bits.
-constexpr int kMergeBatch = 16;
-template <typename T, int D, int PER>
-__device__ __forceinline__ void merge_split_partials(const AttnParams& p, int row, int tok, int head, int nsplit,
+// Merge of a split row's partial outputs (slots slot0 .. slot0 + nsplit - 1) for dims d0, d0 + 1 of query head `head`,
+// written to the output row `tok`: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M). The partials are read
+// kMergeBatch splits at a time, every load of a batch issued before the first is used, with the max and the sums
+// carried from batch to batch: the merge is the serial end of a long row's step, one round trip past the L2 per batch.
+// Each output element's arithmetic depends only on its own head and dim, so any spread of the elements over threads
+// gives the same bits.
+constexpr int kMergeBatch = 32;
+template <typename T, int D>
+__device__ __forceinline__ void merge_split_partials(const AttnParams& p, int slot0, int tok, int head, int nsplit,
                                                      int d0) {
   using E = Elem<T>;
-  static_assert(PER == 1 || PER == 2, "one or two dims per thread");
-  const int64_t slot0 = ((int64_t)row * p.hq + head) * p.max_splits;
-  float m = -INFINITY, den = 0.f, o[PER];
-#pragma unroll
-  for (int e = 0; e < PER; ++e) o[e] = 0.f;
+  float m = -INFINITY, den = 0.f, o0 = 0.f, o1 = 0.f;
+  const int64_t first = (int64_t)slot0 * p.hq + head;
   for (int s0 = 0; s0 < nsplit; s0 += kMergeBatch) {
-    float ls[kMergeBatch], x[kMergeBatch][PER];
+    float ls[kMergeBatch], x[kMergeBatch][2];
 #pragma unroll
     for (int i = 0; i < kMergeBatch; ++i) {
       ls[i] = -INFINITY;
-#pragma unroll
-      for (int e = 0; e < PER; ++e) x[i][e] = 0.f;
+      x[i][0] = x[i][1] = 0.f;
       if (s0 + i < nsplit) {  // uniform over the threads of a row
-        ls[i] = coherent_load(p.part_lse + slot0 + s0 + i);
-        const float* src = p.part_o + (slot0 + s0 + i) * D;
-#pragma unroll
-        for (int e = 0; e < PER; ++e) x[i][e] = coherent_load(src + d0 + e);
+        const int64_t at = first + (int64_t)(s0 + i) * p.hq;
+        ls[i] = coherent_load(p.part_lse + at);
+        coherent_load2(p.part_o + at * D + d0, x[i][0], x[i][1]);
       }
     }
     float bm = m;
@@ -107,30 +116,25 @@ __device__ __forceinline__ void merge_split_partials(const AttnParams& p, int ro
     if (bm == -INFINITY) continue;
     const float alpha = fast_exp2(m - bm);  // 0 while m is -inf
     den *= alpha;
-#pragma unroll
-    for (int e = 0; e < PER; ++e) o[e] *= alpha;
+    o0 *= alpha;
+    o1 *= alpha;
 #pragma unroll
     for (int i = 0; i < kMergeBatch; ++i) {
       const float w = fast_exp2(ls[i] - bm);  // 0 past the last split
       den += w;
-#pragma unroll
-      for (int e = 0; e < PER; ++e) o[e] = fmaf(w, x[i][e], o[e]);
+      o0 = fmaf(w, x[i][0], o0);
+      o1 = fmaf(w, x[i][1], o1);
     }
     m = bm;
   }
   const float inv = den > 0.f ? 1.f / den : 0.f;
-  char* dst = p.out + tok * p.o_st + head * p.o_sh + (int64_t)d0 * 2;
-  if constexpr (PER == 2) {
-    *reinterpret_cast<uint32_t*>(dst) = E::pack(o[0] * inv, o[1] * inv);
-  } else {
-    *reinterpret_cast<uint16_t*>(dst) = (uint16_t)(E::pack(o[0] * inv, 0.f) & 0xffffu);
-  }
+  *reinterpret_cast<uint32_t*>(p.out + tok * p.o_st + head * p.o_sh + (int64_t)d0 * 2) = E::pack(o0 * inv, o1 * inv);
 }
 
 // publish (persistent launches): thread 0 stores publish_value there before the item's merge barrier, and the
 // barrier is met even by an item with nothing to do, so the whole workgroup reads the value after the call.
 template <typename T, int D, int GS, int HP, int US = 0>
-__device__ void decode_item(const AttnParams& p, int row, int split, int kvh, int qg, char* smem,
+__device__ void decode_item(const AttnParams& p, int row, int split, int per, int kvh, int qg, char* smem,
                             int* publish = nullptr, int publish_value = 0) {
   using E = Elem<T>;
   static_assert(D == 64 || D == 128, "head_dim 64 or 128");
@@ -145,14 +149,21 @@ __device__ void decode_item(const AttnParams& p, int row, int split, int kvh, in
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int grp = lane / LPH, hs = (lane / LPT) % HP, part = lane % LPT;
 
-  const int lk = key_len(p, row);
-  const int kbeg = split * p.split;
-  // Past the row's end (the grid is sized for the longest row), or past the bound the caller gave.
-  const bool valid = !((split > 0 && kbeg >= lk) || split >= p.max_splits);
+  // The row's key length, its first query and the page of the item's first key, in one round trip (the page exists: the
+  // plan lists splits that hold keys, and a row of none has a table all the same).
+  const int kbeg = split * per;  // per: keys per split
+  const int32_t* table = p.tables + (int64_t)row * p.t_stride;
+  const int pg0 = (int)p.bs.div(kbeg);
+  const int32_t* len = p.lens_k ? p.lens_k + row : p.cu_k + row;
+  const int32_t* const where[4] = {len, p.lens_k ? len : len + 1, p.cu_q ? p.cu_q + row : len, table + pg0};
+  int got[4];
+  sload_n<4>(where, got);
+  const int lk = p.lens_k ? got[0] : got[1] - got[0];
+  const int tok = p.cu_q ? got[2] : row;
+  const bool valid = split == 0 || kbeg < lk;  // else past the row's end: the row has shrunk since the plan
   if (!valid && !publish) return;
-  const int kend = valid ? min(lk, kbeg + p.split) : kbeg;
-  const int nsplit = min((lk + p.split - 1) / p.split, p.max_splits);
-  const int tok = p.cu_q ? p.cu_q[row] : row;
+  const int kend = valid ? min(lk, kbeg + per) : kbeg;
+  const int nsplit = lk > per ? (lk + per - 1) / per : 1;
   const int head0 = (kvh + hs) * p.group + qg * GS;  // this lane's query heads (kvh: the item's first kv head)
   const float c = p.scale_log2;
 
@@ -173,12 +184,11 @@ __device__ void decode_item(const AttnParams& p, int row, int split, int kvh, in
   uint32_t loff[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) loff[u] = (uint32_t)((u * TPI + grp) * p.c_st + hs * p.c_sh + part * 16);
-  const int32_t* table = p.tables + (int64_t)row * p.t_stride;
 
   // Page numbers come through the scalar cache, once per page this wave enters: a vector load of the table would
   // be waited for in order with the K/V loads already in flight.
-  int cached_pg = -1;
-  int64_t cached_base = 0;
+  int cached_pg = pg0;
+  int64_t cached_base = (int64_t)got[3] * p.c_sb + (int64_t)kvh * p.c_sh;
   auto tile_base = [&](int t0) {
     const int pg = (int)p.bs.div(t0);
     if (pg != cached_pg) {
@@ -324,59 +334,66 @@ __device__ void decode_item(const AttnParams& p, int row, int split, int kvh, in
   if (publish && threadIdx.x == 0) *publish = publish_value;
   __syncthreads();
   if (!valid) return;
-  // One thread per 8 output elements.
-  for (int c = threadIdx.x; c < HG * D / 8; c += blockDim.x) {
-    const int g = c / (D / 8), d0 = (c % (D / 8)) * 8;  // g: query head of the item, hs-major
-    float mmax = -INFINITY;
+  // The waves' sums of the item's query head g, dims d0 .. d0 + N - 1, merged; returns the log2-sum-exp2.
+  auto merge_waves = [&](int g, int d0, auto& o) {
+    constexpr int N = sizeof(o) / sizeof(o[0]);
+    float mmax = -INFINITY, den = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) mmax = fmaxf(mmax, wm[w * HG + g]);
-    float o[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    float den = 0.f;
-    if (mmax != -INFINITY) {
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float wt = fast_exp2(wm[w * HG + g] - mmax);
-        den += wt * wl[w * HG + g];
+    for (int e = 0; e < N; ++e) o[e] = 0.f;
+    if (mmax == -INFINITY) return mmax;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] += wt * wacc[(w * HG + g) * D + d0 + e];
-      }
-      const float inv = 1.f / den;
+    for (int w = 0; w < kWaves; ++w) {
+      const float wt = fast_exp2(wm[w * HG + g] - mmax);
+      den += wt * wl[w * HG + g];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] *= inv;
+      for (int e = 0; e < N; ++e) o[e] += wt * wacc[(w * HG + g) * D + d0 + e];
     }
-    const int head = (kvh + g / GS) * p.group + qg * GS + g % GS;
-    if (nsplit <= 1) {
+    const float inv = 1.f / den;
+#pragma unroll
+    for (int e = 0; e < N; ++e) o[e] *= inv;
+    return mmax + fast_log2(den);
+  };
+  auto head_of = [&](int g) { return (kvh + g / GS) * p.group + qg * GS + g % GS; };  // g: hs-major
+  if (nsplit <= 1) {
+    // One thread per 8 output elements.
+    for (int c = threadIdx.x; c < HG * D / 8; c += blockDim.x) {
+      const int g = c / (D / 8), d0 = (c % (D / 8)) * 8;
+      float o[8];
+      merge_waves(g, d0, o);
       u32x4 packed;
 #pragma unroll
       for (int w = 0; w < 4; ++w) packed[w] = E::pack(o[2 * w], o[2 * w + 1]);
-      st16(p.out + tok * p.o_st + head * p.o_sh + (int64_t)d0 * 2, packed);
-    } else {
-      const int64_t slot = ((int64_t)row * p.hq + head) * p.max_splits + split;
-      float* dst = p.part_o + slot * D + d0;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) coherent_store(dst + e, o[e]);
-      if (d0 == 0) coherent_store(p.part_lse + slot, mmax == -INFINITY ? -INFINITY : mmax + fast_log2(den));
+      st16(p.out + tok * p.o_st + head_of(g) * p.o_sh + (int64_t)d0 * 2, packed);
     }
+    return;
   }
-  // A split row: the split that counts in last merges the item's heads. Each wave waits until its partial stores
-  // are complete (written through to memory) before the barrier that precedes the count, so every split's partials
-  // are in memory before its count; the merger reads them past its L2 after its own count has returned.
-  if (nsplit > 1 && p.merge_count) {
-    __shared__ int s_last;
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    int32_t* count = p.merge_count + (row * (p.hkv / HP) + kvh / HP) * p.qgroups + qg;
-    if (threadIdx.x == 0)
-      s_last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
-    __syncthreads();
-    if (s_last) {
-      for (int c = threadIdx.x; c < HG * D / 2; c += blockDim.x) {
-        const int g = c / (D / 2), d0 = (c % (D / 2)) * 2;
-        merge_split_partials<T, D, 2>(p, row, tok, (kvh + g / GS) * p.group + qg * GS + g % GS, nsplit, d0);
-      }
-      // Back to zero for the next layer on this plan.
-      if (threadIdx.x == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+  // One thread per two elements of the partial: a wave writes 512 consecutive bytes.
+  const int slot0 = p.part_base[row];  // the row's partial slots
+  for (int c = threadIdx.x; c < HG * D / 2; c += blockDim.x) {
+    const int g = c / (D / 2), d0 = (c % (D / 2)) * 2;
+    float o[2];
+    const float lse = merge_waves(g, d0, o);
+    const int64_t slot = (int64_t)(slot0 + split) * p.hq + head_of(g);
+    coherent_store2(p.part_o + slot * D + d0, o[0], o[1]);
+    if (d0 == 0) coherent_store(p.part_lse + slot, lse);
+  }
+  // The split that counts in last merges the item's heads. Each wave waits until its partial stores are complete
+  // (written through to memory) before the barrier that precedes the count, so every split's partials are in memory
+  // before its count; the merger reads them past its L2 after its own count has returned.
+  __shared__ int s_last;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  int32_t* count = p.merge_count + (row * (p.hkv / HP) + kvh / HP) * p.qgroups + qg;
+  if (threadIdx.x == 0)
+    s_last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
+  __syncthreads();
+  if (s_last) {
+    for (int c = threadIdx.x; c < HG * D / 2; c += blockDim.x)
+      merge_split_partials<T, D>(p, slot0, tok, head_of(c / (D / 2)), nsplit, (c % (D / 2)) * 2);
+    // Back to zero for the next layer on this plan.
+    if (threadIdx.x == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -389,19 +406,36 @@ struct SmemBytes {
 };
 
 // Work-list kernels. blockIdx.x walks the device work list with the query-head groups innermost, so workgroups
-// are dispatched in list order (longest first). The list holds a step's prompt items first (n_items[1] of them),
-// then its decode items (n_items[0] in all). Decode items run in decode_list_kernel at the decode item's register
-// budget; prompt items in prompt_list_kernel, whose MFMA tile needs more registers and LDS.
+// are dispatched in list order (longest first). The step's prompt items and its decode items are two lists. Decode
+// items run in decode_list_kernel at the decode item's register budget; prompt items in prompt_list_kernel, whose MFMA
+// tile needs more registers and LDS.
+
+// Decode item i (below the launch's bound, so inside the list's memory), the number of decode items and the keys per
+// split, in one round trip: a decode workgroup's start is a chain of dependent loads (item, then lengths and page,
+// then keys), and a step of a few short rows is little more than that chain.
+struct DecodeWork {
+  int row, split, count, per;
+};
+__device__ __forceinline__ DecodeWork decode_work(const AttnParams& p, int i) {
+  DecodeWork w;
+  int64_t item;
+  asm volatile("s_load_dwordx2 %0, %3, 0x0\n\ts_load_dword %1, %4, %5\n\ts_load_dword %2, %4, %6\n\ts_waitcnt lgkmcnt(0)"
+               : "=&s"(item), "=&s"(w.count), "=&s"(w.per)
+               : "s"(p.items + i), "s"(p.n_items), "n"(4 * kPlanDecodes), "n"(4 * kPlanSplit));
+  w.row = (int)(uint32_t)item;
+  w.split = (int)(item >> 32);
+  return w;
+}
+
 template <typename T, int D, int GS, int HP, int US = 0>
 __global__ __launch_bounds__(256) void decode_list_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) char smem[SmemBytes<D, GS, HP>::kDecode];
   const int ny = p.hkv / HP * p.qgroups;
   const int bx = blockIdx.x / ny, by = blockIdx.x - bx * ny;
   const int kh = by / p.qgroups, qg = by - kh * p.qgroups;
-  const int i = bx + p.n_items[1];
-  if (i >= p.n_items[0]) return;
-  const int2 it = p.items[i];
-  decode_item<T, D, GS, HP, US>(p, it.x, it.y, kh * HP, qg, smem);
+  const DecodeWork w = decode_work(p, bx);
+  if (bx >= w.count) return;
+  decode_item<T, D, GS, HP, US>(p, w.row, w.split, w.per, kh * HP, qg, smem);
 }
 
 // Decode items of the work list on a persistent grid beside a mixed step's prompt workgroups: each workgroup takes
@@ -417,8 +451,7 @@ __device__ __forceinline__ void decode_persistent(const AttnParams& p) {
   __shared__ __attribute__((aligned(16))) char smem[2][SmemBytes<D, GS, HP>::kDecode];
   __shared__ int s_ticket[2];
   const int ny = p.hkv / HP * p.qgroups;
-  const int first = p.n_items[1];
-  const int total = (p.n_items[0] - first) * ny;
+  const int total = p.n_items[kPlanDecodes] * ny;
   if (threadIdx.x == 0) s_ticket[0] = atomicAdd(p.ticket, 1);
   __syncthreads();
   int f = __builtin_amdgcn_readfirstlane(s_ticket[0]);
@@ -427,8 +460,8 @@ __device__ __forceinline__ void decode_persistent(const AttnParams& p) {
     if (threadIdx.x == 0) next = atomicAdd(p.ticket, 1);
     const int bx = f / ny, by = f - bx * ny;
     const int kh = by / p.qgroups, qg = by - kh * p.qgroups;
-    const int2 it = p.items[first + bx];
-    decode_item<T, D, GS, HP, US>(p, it.x, it.y, kh * HP, qg, smem[k & 1], &s_ticket[(k + 1) & 1], next);
+    const DecodeWork w = decode_work(p, bx);
+    decode_item<T, D, GS, HP, US>(p, w.row, w.split, w.per, kh * HP, qg, smem[k & 1], &s_ticket[(k + 1) & 1], next);
     f = __builtin_amdgcn_readfirstlane(s_ticket[(k + 1) & 1]);
   }
   if (threadIdx.x == 0 && atomicAdd(p.ticket + 1, 1) == (int)gridDim.x - 1) {
@@ -461,8 +494,8 @@ __global__ __launch_bounds__(256, 2) void prompt_list_kernel(AttnParams p) {
   constexpr int RING = kRingOf<TP>;
   __shared__ __attribute__((aligned(16))) char smem[(RING > 0 ? RING : 1) * PromptSmem<D, D, (TP > 1)>::kBytes];
   const int bx = blockIdx.x / p.hkv, kvh = blockIdx.x - bx * p.hkv;
-  if (bx >= p.n_items[1]) return;
-  const int2 it = p.items[bx];
+  if (bx >= p.n_items[kPlanPrompts]) return;
+  const int2 it = p.prompts[bx];
   prefill_item<T, D, D, true, false, RING, 4, false, (TP > 0 ? TP : 1)>(p, it.x, -1 - it.y, kvh, smem);
 }
 
@@ -478,10 +511,10 @@ __global__ __launch_bounds__(256, 2) void prompt_overlap_kernel(AttnParams p) {
   // The prompt tiles are the step's critical path beside the decode waves, which need few issue slots: the prompt
   // waves win the SIMD's issue arbitration (1% on the Qwen3-8B mixed step; favouring the decode waves costs 15%).
   __builtin_amdgcn_s_setprio(1);
-  const int n = p.n_items[1] * p.hkv;
+  const int n = p.n_items[kPlanPrompts] * p.hkv;
   for (int f = blockIdx.x; f < n; f += gridDim.x) {
     const int bx = f / p.hkv, kvh = f - bx * p.hkv;
-    const int2 it = p.items[bx];
+    const int2 it = p.prompts[bx];
     prefill_item<T, D, D, true, true, RING, 4, false, (TP > 0 ? TP : 1)>(p, it.x, -1 - it.y, kvh, smem);
     __syncthreads();  // the next item restages the LDS tiles
   }
@@ -501,27 +534,26 @@ __global__ __launch_bounds__(256, 2) void mixed_small_kernel(AttnParams p, int32
   const int b = blockIdx.x;
   if (b < prompt_wgs) {
     const int bx = b / p.hkv, kvh = b - bx * p.hkv;
-    if (bx >= p.n_items[1]) return;
-    const int2 it = p.items[bx];
+    if (bx >= p.n_items[kPlanPrompts]) return;
+    const int2 it = p.prompts[bx];
     prefill_item<T, D, D, true, false, RING, 4, false, (TP > 0 ? TP : 1)>(p, it.x, -1 - it.y, kvh, smem);
   } else {
     const int ny = p.hkv / HP * p.qgroups;
     const int f = b - prompt_wgs, bx = f / ny, by = f - bx * ny;
     const int kh = by / p.qgroups, qg = by - kh * p.qgroups;
-    const int i = bx + p.n_items[1];
-    if (i >= p.n_items[0]) return;
-    const int2 it = p.items[i];
-    decode_item<T, D, GS, HP>(p, it.x, it.y, kh * HP, qg, smem);
+    const DecodeWork w = decode_work(p, bx);
+    if (bx >= w.count) return;
+    decode_item<T, D, GS, HP>(p, w.row, w.split, w.per, kh * HP, qg, smem);
   }
 }
 
-// Decode of more rows than the planner holds: blockIdx.x is (row, split), blockIdx.y the query-head group. Such a
-// step is planned unsplit (max_splits 1): a split row's partials need the merge counters of a work list.
+// Decode of more rows than the planner holds: blockIdx.x is the row, blockIdx.y the kv head (or pair) and query-head
+// group. Such a step's rows are not split: a split row's partials need the slots and merge counters of a work list.
 template <typename T, int D, int GS, int HP>
 __global__ __launch_bounds__(256) void decode_grid_kernel(AttnParams p) {
   __shared__ __attribute__((aligned(16))) char smem[SmemBytes<D, GS, HP>::kDecode];
   const int kh = blockIdx.y / p.qgroups, qg = blockIdx.y % p.qgroups;
-  decode_item<T, D, GS, HP>(p, blockIdx.x / p.max_splits, blockIdx.x % p.max_splits, kh * HP, qg, smem);
+  decode_item<T, D, GS, HP>(p, blockIdx.x, 0, INT32_MAX, kh * HP, qg, smem);
 }
 
 constexpr int kLenBuckets = 64;
@@ -531,37 +563,98 @@ __device__ inline int len_bucket(int keys, int split) {
   return b < kLenBuckets - 1 ? b : kLenBuckets - 1;
 }
 
-// Work list of a step, longest work first: prompt items (row, -1 - tile), then every full decode split (row, s),
-// then each decode row's last split (row, n - 1) by decreasing key count (counting sort over length buckets).
+// Work lists of a step, longest work first: the prompt items (row, -1 - tile); and the decode items, every full split
+// (row, s), then each row's last split (row, n - 1) by decreasing key count (counting sort over length buckets).
 // In-order dispatch of that list approximates longest-processing-time scheduling, so the launch ends with short
 // items instead of a tail of full ones. A prompt row's tiles go last tile first (most keys) when the prompt items
 // have the GPU to themselves (last_first: a step of prompts, or the serial schedule): the Qwen3-8B chunks 5-6%
 // faster than first tile first. Beside the decode rows (the overlapped schedule) the order made no measurable
 // difference, and the first tile goes first there as before. The split rows' merge counters start at zero.
+//
+// Keys per decode split: the decode rows' own keys over `pieces`, at least kMinSplit and a multiple of kSplitStep, so
+// that a step is cut into about the same number of items whatever its lengths (at most pieces + rows). The caller's
+// bound on key lengths only sizes the buffers: a captured graph's bound is the longest context it may ever serve, and
+// a batch of a few rows far apart in length has most of its keys in one of them. pieces 0: rows are not split, and
+// one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]; a split
+// that needs more slots than there are (lengths past the caller's bound) is doubled until they fit.
+struct PlanOut {
+  int2* prompts;    // the prompt items
+  int2* items;      // the decode items
+  int32_t* counts;  // kPlan* entries
+  int32_t* part_base;
+  int32_t* merge_count;
+};
+
 __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __restrict__ cu_q,
                                                             const int32_t* __restrict__ lens_k,
                                                             const int32_t* __restrict__ cu_k, int32_t rows,
-                                                            int32_t split, int32_t qp, int32_t max_items,
-                                                            int32_t last_first, int2* __restrict__ items,
-                                                            int32_t* __restrict__ n_items,
-                                                            int32_t* __restrict__ merge_count, int32_t n_merge) {
+                                                            int32_t pieces, int32_t max_slots, int32_t qp,
+                                                            int32_t max_prompts, int32_t max_items,
+                                                            int32_t last_first, int32_t n_merge,
+                                                            PlanOut out) {
   __shared__ int pre[kPlanMaxRows + 1];
   __shared__ int full[kPlanMaxRows + 1];
+  __shared__ int slots[kPlanMaxRows + 1];
   __shared__ int bucket[kLenBuckets + 1];
   __shared__ int wave_tot[kScanThreads / 64 + 1];
+  __shared__ int64_t wave_keys[kScanThreads / 64];
+  __shared__ int wave_max[kScanThreads / 64];
   const int tid = threadIdx.x;
   for (int b = tid; b <= kLenBuckets; b += kScanThreads) bucket[b] = 0;
-  for (int i = tid; i < n_merge; i += kScanThreads) merge_count[i] = 0;
-  __syncthreads();
+  for (int i = tid; i < n_merge; i += kScanThreads) out.merge_count[i] = 0;
+  // The decode rows' keys in all and at most.
+  int64_t keys = 0;
+  int longest = 1;
   for (int r = tid; r < rows; r += kScanThreads) {
     const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
-    pre[r] = lq > 1 ? (lq + qp - 1) / qp : 0;
-    full[r] = 0;
     if (lq == 1) {
-      const int n = lk > 0 ? (lk + split - 1) / split : 1;
-      full[r] = n - 1;
+      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+      keys += max(lk, 0);
+      longest = max(longest, lk);
+    }
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    keys += __shfl_xor(keys, d, 64);
+    longest = max(longest, __shfl_xor(longest, d, 64));
+  }
+  if ((tid & 63) == 0) {
+    wave_keys[tid >> 6] = keys;
+    wave_max[tid >> 6] = longest;
+  }
+  __syncthreads();
+  keys = 0;
+  longest = 1;
+#pragma unroll
+  for (int w = 0; w < kScanThreads / 64; ++w) {
+    keys += wave_keys[w];
+    longest = max(longest, wave_max[w]);
+  }
+  int64_t want = longest;
+  if (pieces > 0) want = min(want, max((int64_t)kMinSplit, (keys + pieces - 1) / pieces));
+  int split = (int)min((want + kSplitStep - 1) / kSplitStep * kSplitStep, (int64_t)INT32_MAX);
+  for (;;) {  // every thread leaves together: slots[rows] is the same for all, and split reaches the longest row
+    for (int r = tid; r < rows; r += kScanThreads) {
+      const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
+      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+      const int n = lq == 1 ? (lk > split ? (lk + split - 1) / split : 1) : 0;  // the row's decode items
+      pre[r] = lq > 1 ? (lq + qp - 1) / qp : 0;
+      full[r] = max(n - 1, 0);
+      slots[r] = n > 1 ? n : 0;
+    }
+    __syncthreads();
+    block_scan(slots, rows, wave_tot);
+    if (slots[rows] <= max_slots || split >= longest) break;
+    split = split < (1 << 29) ? 2 * split : INT32_MAX;
+    __syncthreads();  // every thread has read slots[rows]
+  }
+  for (int r = tid; r < rows; r += kScanThreads) {
+    const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
+    if (lq == 1) {
+      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+      const int n = lk > split ? (lk + split - 1) / split : 1;
       atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
+      if (n > 1) out.part_base[r] = slots[r];
     }
   }
   __syncthreads();
@@ -575,24 +668,32 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   block_scan(pre, rows, wave_tot);  // its barriers also publish the bucket offsets
   block_scan(full, rows, wave_tot);
   const int npre = pre[rows], nfull = full[rows], npart = bucket[kLenBuckets];
+  // Full splits, one thread each (a few long rows hold hundreds: a thread per row would write them one by one).
+  for (int i = tid; i < nfull; i += kScanThreads) {
+    int lo = 0, hi = rows - 1;  // the last row whose first full split is at or before i
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (full[mid] <= i) lo = mid; else hi = mid - 1;
+    }
+    if (i < max_items) out.items[i] = make_int2(lo, i - full[lo]);
+  }
   for (int r = tid; r < rows; r += kScanThreads) {
     for (int i = pre[r]; i < pre[r + 1]; ++i)
-      if (i < max_items) items[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
-    for (int i = full[r]; i < full[r + 1]; ++i)
-      if (npre + i < max_items) items[npre + i] = make_int2(r, i - full[r]);
+      if (i < max_prompts) out.prompts[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
     const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
     if (lq == 1) {
       const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
-      const int n = lk > 0 ? (lk + split - 1) / split : 1;
-      const int pos = npre + nfull + atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
-      if (pos < max_items) items[pos] = make_int2(r, n - 1);
+      const int n = lk > split ? (lk + split - 1) / split : 1;
+      const int pos = nfull + atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
+      if (pos < max_items) out.items[pos] = make_int2(r, n - 1);
     }
   }
   if (tid == 0) {
-    n_items[0] = min(npre + nfull + npart, max_items);
-    n_items[1] = min(npre, max_items);
-    n_items[2] = 0;  // the persistent decode launch's ticket counter
-    n_items[3] = 0;  // and its count of workgroups done
+    out.counts[kPlanDecodes] = min(nfull + npart, max_items);
+    out.counts[kPlanPrompts] = min(npre, max_prompts);
+    out.counts[kPlanTicket] = 0;
+    out.counts[kPlanDone] = 0;
+    out.counts[kPlanSplit] = split;
   }
 }
 
@@ -600,9 +701,12 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
 // Host side.
 
 struct Shape {
-  int32_t split, max_splits, max_items, max_prompt_items, max_decode_items, gs;
-  int64_t merges;  // split rows' merge counters (rows x kv heads x query-head groups), listed steps only
-  size_t items_off, count_off, lse_off, o_off, merge_off, bytes;
+  int32_t max_items, max_prompt_items, max_decode_items, gs;
+  int32_t pieces;      // the plan cuts the decode rows' keys into this many (0: rows are not split)
+  int32_t max_splits;  // the most items one row may be split into
+  int32_t slots;       // split rows' partial slots
+  int64_t merges;      // split rows' merge counters (rows x kv heads x query-head groups)
+  size_t items_off, count_off, base_off, lse_off, o_off, merge_off, bytes;
 };
 
 static int pick_gs(int group) {
@@ -616,36 +720,49 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   Shape s{};
   const int group = hq / hkv;
   s.gs = pick_gs(group);
-  const int64_t units = (int64_t)rows * hkv * (group / s.gs);
+  const int64_t per_split = (int64_t)hkv * (group / s.gs);  // decode items per row and split
   const int64_t keys = max_k > 0 ? max_k : 1;
-  // Keys per decode item: enough items to fill the chip several times over, at least 256 keys each. Rows split only
-  // in a listed step (whose workspace holds the merge counters); a step of more rows has units beyond the target
-  // anyway.
-  const int64_t target = kSplitTarget;
-  int64_t split = kMinSplit;
-  while (split < keys && (!listed || units * ((keys + split - 1) / split) > target)) split *= 2;
-  s.split = (int32_t)split;
-  s.max_splits = (int32_t)((keys + split - 1) / split);
+  // Rows split only in a listed step (whose workspace holds the partial slots and merge counters) whose unsplit items
+  // are at most half the target: with more, the longest-first list balances them as they are.
+  //
+  // The number of splits weighs the list's balance against the merge of a row, one round trip past the L2 per
+  // kMergeBatch splits after its last split: 4096 one-head items for many rows, fewer for a few long ones. 32/8 heads,
+  // d128, contexts U[32K, 128K], 1024 / 2048 / 3072 / 4096 items (before, 4096 with batches of 16): 1 row
+  // 93 / 113 / 125 / 132 us (166), 2 rows 174 / 181 / 192 / 190 (219), 3 rows 252 / 250 / 256 / 261 (272), 8 rows
+  // 594 / 557 / 567 / 569 (585), 24 rows 1494 / 1399 / 1372 / 1384 (1452); 48 rows U[4K, 64K] 1431 / 1283 / 1237 / 1241
+  // (1309).
+  const int64_t items = rows <= 2 ? kSplitTarget / 4 : rows <= 16 ? kSplitTarget / 2 : kSplitTarget;
+  const int64_t target =  // splits of all rows
+      std::min<int64_t>((items + per_split - 1) / per_split, (int64_t)kMaxRowSplits * rows);
+  const bool split = listed && 2 * (int64_t)rows <= target && keys > kMinSplit;
+  s.pieces = split ? (int32_t)(target - rows) : 0;
+  const int64_t most = split ? (keys + kMinSplit - 1) / kMinSplit : 1;  // of one row
+  const int64_t splits = split ? std::min(rows * most, target) : rows;
+  s.max_splits = (int32_t)std::min(most, splits);
   const int qp = kPrefillRows / (group > 0 ? group : 1);
   // In 64 bits, saturated: a count past INT32_MAX is far past what one launch holds (check_grids refuses it).
   auto sat = [](int64_t x) { return (int32_t)std::min<int64_t>(x, INT32_MAX); };
   s.max_prompt_items = listed ? sat(((int64_t)tokens + qp - 1) / qp + rows) : 0;
-  s.max_decode_items = listed ? sat((int64_t)rows * s.max_splits) : 0;
+  s.max_decode_items = listed ? sat(splits) : 0;
   s.max_items = sat((int64_t)s.max_prompt_items + s.max_decode_items);
+  s.slots = s.max_splits > 1 ? sat(splits) : 0;
   size_t off = 0;
   s.items_off = off;
   off += (size_t)s.max_items * sizeof(int2);
   off = (off + 255) / 256 * 256;
   s.count_off = off;
   off += 256;
-  const size_t parts = s.max_splits > 1 ? (size_t)rows * hq * s.max_splits : 0;
+  s.base_off = off;
+  off += s.slots > 0 ? (size_t)rows * sizeof(int32_t) : 0;
+  off = (off + 255) / 256 * 256;
+  const size_t parts = (size_t)s.slots * hq;
   s.lse_off = off;
   off += parts * sizeof(float);
   off = (off + 255) / 256 * 256;
   s.o_off = off;
   off += parts * d * sizeof(float);
   off = (off + 255) / 256 * 256;
-  s.merges = listed && s.max_splits > 1 ? (int64_t)rows * hkv * (group / s.gs) : 0;
+  s.merges = s.slots > 0 ? (int64_t)rows * per_split : 0;
   s.merge_off = off;
   off += (size_t)s.merges * sizeof(int32_t);
   s.bytes = off;
@@ -745,8 +862,8 @@ static Route route_of(const AttnParams& p, const Shape& s, const StepKind& k) {
   const int ny = p.hkv / HP * p.qgroups;
   const int cus = device_cus();
   const int64_t pw = k.listed && k.mixed ? (int64_t)s.max_prompt_items * p.hkv : 0;
-  const int64_t dw = k.listed ? (int64_t)s.max_decode_items * ny : (int64_t)p.rows * p.max_splits * ny;
-  r.merge = p.max_splits > 1 && !k.prompts_only;
+  const int64_t dw = k.listed ? (int64_t)s.max_decode_items * ny : (int64_t)p.rows * ny;
+  r.merge = s.max_splits > 1 && !k.prompts_only;
   if (k.prompts_only) {
     r.prompt = LV_KERNEL_PROMPT_LIST;
     r.prompt_grid = (int)pw;
@@ -782,7 +899,7 @@ static void launch_decode(const AttnParams& p, const Route& r, hipStream_t strea
   if (r.decode == LV_KERNEL_DECODE_BESIDE)
     hipLaunchKernelGGL((decode_beside_kernel<T, D, GS, HP>), dim3(r.decode_grid), dim3(256), 0, stream, p);
   else if (r.decode == LV_KERNEL_DECODE_GRID)
-    hipLaunchKernelGGL((decode_grid_kernel<T, D, GS, HP>), dim3(p.rows * p.max_splits, p.hkv / HP * p.qgroups),
+    hipLaunchKernelGGL((decode_grid_kernel<T, D, GS, HP>), dim3(p.rows, p.hkv / HP * p.qgroups),
                        dim3(256), 0, stream, p);
   else if (r.decode == LV_KERNEL_DECODE_LIST)
     hipLaunchKernelGGL((decode_list_kernel<T, D, GS, HP, kWideSteps<D, HP>>), dim3(r.decode_grid), dim3(256), 0,
@@ -873,7 +990,7 @@ static int launch_tp(const AttnParams& p, const Shape& s, const StepKind& k, hip
 constexpr int kPairItems = 8;
 template <typename T, int D, int GS>
 static int launch_hp(const AttnParams& p, const Shape& s, const StepKind& k, hipStream_t stream, Route* info) {
-  const int64_t items = (int64_t)(k.listed ? s.max_decode_items : p.rows * p.max_splits) * p.hkv * p.qgroups;
+  const int64_t items = (int64_t)(k.listed ? s.max_decode_items : p.rows) * p.hkv * p.qgroups;
   if (p.hkv % 2 == 0 && p.c_sh >= 0 && p.c_sh < ((int64_t)1 << 30) && items >= (int64_t)kPairItems * device_cus())
     return launch_tp<T, D, GS, 2>(p, s, k, stream, info);
   return launch_tp<T, D, GS, 1>(p, s, k, stream, info);
@@ -942,11 +1059,11 @@ static void* scratch_on_current_device() {
 struct PlanSig {
   const void* ws = nullptr;
   const int32_t *cu_q = nullptr, *lens = nullptr, *cu_k = nullptr;
-  int64_t rows = 0, tokens = 0, max_k = 0, split = 0, qp = 0, max_items = 0, bytes = 0;
+  int64_t rows = 0, tokens = 0, max_k = 0, pieces = 0, qp = 0, max_items = 0, bytes = 0;
   bool mixed = false, last_first = false;
   bool operator==(const PlanSig& o) const {
     return ws == o.ws && cu_q == o.cu_q && lens == o.lens && cu_k == o.cu_k && rows == o.rows &&
-           tokens == o.tokens && max_k == o.max_k && split == o.split && qp == o.qp && max_items == o.max_items &&
+           tokens == o.tokens && max_k == o.max_k && pieces == o.pieces && qp == o.qp && max_items == o.max_items &&
            bytes == o.bytes && mixed == o.mixed && last_first == o.last_first;
   }
 };
@@ -1031,11 +1148,8 @@ static StepKind step_kind(int32_t num_rows, bool has_cu_q, int32_t max_seqlen_q,
 
 // A launch counts its work-items (workgroups x 256) in 32 bits: the step's largest grid must stay below that.
 static int check_grids(const Shape& s, int32_t num_rows, int32_t num_heads, int32_t num_kv_heads) {
-  // Split rows are merged through the work list's counters: a step without the list must not split.
-  LV_REQUIRE(s.max_splits == 1 || s.merges > 0, "paged_attention: %d rows split over %d items without a work list",
-             num_rows, s.max_splits);
   const int64_t prompt = (int64_t)s.max_prompt_items * num_kv_heads;
-  const int64_t decode = std::max<int64_t>(s.max_decode_items, (int64_t)num_rows * s.max_splits) * num_heads;
+  const int64_t decode = std::max<int64_t>(s.max_decode_items, num_rows) * num_heads;
   LV_REQUIRE(fits_one_launch(prompt + decode, 256),
              "paged_attention: the step needs %lld + %lld workgroups, more than one launch holds", (long long)prompt,
              (long long)decode);
@@ -1052,8 +1166,6 @@ static void shape_params(AttnParams& p, const Shape& s, int32_t num_rows, int32_
   p.hkv = num_kv_heads;
   p.group = num_heads / num_kv_heads;
   p.qgroups = p.group / s.gs;
-  p.split = s.split;
-  p.max_splits = s.max_splits;
 }
 
 // One step, with the workspace given (workspace != nullptr or an empty shape) or, for static_ws, the device's
@@ -1114,8 +1226,10 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   p.v_sh = p.c_sh;
   p.paged = true;
   p.causal = 1;
-  p.tables = block_tables;
-  p.t_stride = table_stride;
+  // Decode items read their row's first page before its length; with no keys at all a table may hold no entry, so the
+  // lengths (any readable ints) stand in for it.
+  p.tables = max_seqlen_k > 0 ? block_tables : seqlens_k ? seqlens_k : cu_seqlens_k;
+  p.t_stride = max_seqlen_k > 0 ? table_stride : 0;
   p.cu_q = cu_seqlens_q;
   p.lens_k = seqlens_k;
   p.cu_k = cu_seqlens_k;
@@ -1124,11 +1238,13 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   p.o_st = out_stride_t * 2;
   p.o_sh = out_stride_h * 2;
   char* ws = (char*)workspace;
-  p.part_lse = s.max_splits > 1 ? reinterpret_cast<float*>(ws + s.lse_off) : nullptr;
-  p.part_o = s.max_splits > 1 ? reinterpret_cast<float*>(ws + s.o_off) : nullptr;
-  p.items = kind.listed ? reinterpret_cast<const int2*>(ws + s.items_off) : nullptr;
+  p.part_base = s.slots > 0 ? reinterpret_cast<const int32_t*>(ws + s.base_off) : nullptr;
+  p.part_lse = s.slots > 0 ? reinterpret_cast<float*>(ws + s.lse_off) : nullptr;
+  p.part_o = s.slots > 0 ? reinterpret_cast<float*>(ws + s.o_off) : nullptr;
+  p.prompts = kind.listed ? reinterpret_cast<const int2*>(ws + s.items_off) : nullptr;
+  p.items = kind.listed ? p.prompts + s.max_prompt_items : nullptr;
   p.n_items = kind.listed ? reinterpret_cast<const int32_t*>(ws + s.count_off) : nullptr;
-  p.ticket = kind.listed ? reinterpret_cast<int32_t*>(ws + s.count_off) + 2 : nullptr;
+  p.ticket = kind.listed ? reinterpret_cast<int32_t*>(ws + s.count_off) + kPlanTicket : nullptr;
   p.merge_count = s.merges > 0 ? reinterpret_cast<int32_t*>(ws + s.merge_off) : nullptr;
 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -1141,7 +1257,7 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   sig.rows = num_rows;
   sig.tokens = num_tokens;
   sig.max_k = max_seqlen_k;
-  sig.split = s.split;
+  sig.pieces = s.pieces;
   sig.qp = qp;
   sig.max_items = s.max_items;
   sig.bytes = (int64_t)s.bytes;
@@ -1150,10 +1266,12 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   bool planned = false;
   if (kind.listed && !plan_is_current(sig, (flags & LV_ATTN_REUSE_PLAN) != 0)) {
     record_plan(workspace, nullptr);  // until this plan's launch is accepted, the workspace holds no plan
+    int2* lists = reinterpret_cast<int2*>(ws + s.items_off);
+    const PlanOut out{lists, lists + s.max_prompt_items, reinterpret_cast<int32_t*>(ws + s.count_off),
+                      reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kScanThreads), 0, st, kind.mixed ? cu_seqlens_q : nullptr,
-                       seqlens_k, cu_seqlens_k, num_rows, s.split, qp, s.max_items, (int32_t)sig.last_first,
-                       reinterpret_cast<int2*>(ws + s.items_off), reinterpret_cast<int32_t*>(ws + s.count_off),
-                       p.merge_count, (int32_t)s.merges);
+                       seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
+                       s.max_decode_items, (int32_t)sig.last_first, (int32_t)s.merges, out);
     LV_LAUNCH_CHECK("plan_kernel");
     planned = true;
   }
@@ -1211,7 +1329,7 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
   info->prompt_workgroups = r.prompt_grid;
   info->kv_heads_per_item = r.hp;
   info->two_streams = r.two_streams;
-  info->keys_per_split = s.split;
+  info->keys_per_split = kMinSplit;
   info->max_splits = s.max_splits;
   info->splitk_merge = r.merge;
   return LV_OK;

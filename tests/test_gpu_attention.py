@@ -733,3 +733,33 @@ def test_huge_values_with_scores_above_the_first_tile(cuda, dim):
     assert torch.isfinite(out).all()
     # The path's bf16 bar (2e-2 absolute, 1e-2 relative) at the values' scale.
     torch.testing.assert_close(out.float().cpu(), want.float(), atol=2e-2 * 2.0 ** 100, rtol=1e-2)
+
+
+@pytest.mark.parametrize("lens", [[40_000], [3, 20_000], [5_000, 0, 9_000] + [700] * 13, [12_000] + [257] * 16],
+                         ids=["one-row", "two-rows", "16-rows", "17-rows"])
+def test_splits_are_sized_from_the_rows_lengths(cuda, lens):
+    """Decode rows far apart in length, under a table twice as wide as the longest needs: the plan sizes the splits
+    from the keys there are. The row counts sit on both sides of the rules that bound the number of splits (2 and 16
+    rows; one row's splits capped). Against the oracle."""
+    bs, heads, kv_heads, dim = 16, 8, 2, 64
+    need = [-(-n // bs) for n in lens]
+    width, at, tables = 2 * max(need), 0, []
+    for k in need:
+        tables.append(list(range(at, at + k)) + [-1] * (width - k))
+        at += k
+    b = MI355XAttention(heads, dim, 1 / math.sqrt(dim), kv_heads)
+    qs, kf, vf, kn, vn, kc, vc, slots = paged_step([max(n - 1, 0) for n in lens], [min(n, 1) for n in lens], tables, at,
+                                                   heads=heads, kv_heads=kv_heads, dim=dim, bs=bs, device=cuda,
+                                                   dtype=torch.bfloat16, seed=9)
+    b.store_kvcache(kn, vn, kc, vc, slots)
+    live = [i for i, n in enumerate(lens) if n]
+    q = torch.randn(len(lens), heads, dim, generator=torch.Generator().manual_seed(10)).to(torch.bfloat16).to(cuda)
+    ctx = Context(context_lens=torch.tensor(lens, dtype=torch.int32, device=cuda),
+                  block_tables=torch.tensor(tables, dtype=torch.int32, device=cuda))
+    b.launch_trace = []
+    out = b.decode(q, kc, vc, ctx)
+    torch.cuda.synchronize()
+    assert b.launch_trace[-1]["splitk_merge"]
+    want = dense_expected([q[i:i + 1] for i in live], [kf[i] for i in live], [vf[i] for i in live], 1 / math.sqrt(dim))
+    torch.testing.assert_close(out[live].float().cpu(), want, atol=2e-2, rtol=1e-2)
+    assert not out[[i for i, n in enumerate(lens) if not n]].any()
