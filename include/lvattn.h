@@ -128,7 +128,8 @@ int lv_store_latents(const void* latent, int64_t latent_stride_t, int32_t num_to
  * them at zero again, so a later layer finds them as the plan left them. */
 #define LV_ATTN_REUSE_PLAN 1
 /* flags, also: LV_ATTN_PROMPTS_ONLY -- every row of the step has more than one query (the caller's host lengths say
- * so), so no decode launch and no split-K merge are made. Needs cu_seqlens_q and max_seqlen_q > 1. */
+ * so), so no decode launch and no split-K merge are made; a step whose rows all have few queries (drafted tokens) runs
+ * as decode items with or without it. Needs cu_seqlens_q and max_seqlen_q > 1. */
 #define LV_ATTN_PROMPTS_ONLY 2
 size_t lv_paged_attention_workspace_bytes(int32_t num_rows, int32_t num_tokens, int32_t num_heads,
                                           int32_t num_kv_heads, int32_t head_dim, int32_t max_seqlen_k,
@@ -181,7 +182,7 @@ int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t
  * allocation. The work list, its counters and the split-K partials live in a static device array of
  * LV_STATIC_WORKSPACE_BYTES that each GPU the library runs on holds until the process ends; a step needing more
  * (lv_paged_attention_workspace_bytes larger than that; the split-K sizing keeps steps of up to 4096 rows at any
- * context length under 9 MiB) is refused with LV_EINVAL. The kernels clear what must start at zero themselves
+ * context length under 9 MiB, of few queries per row under 15 MiB) is refused with LV_EINVAL. The kernels clear what must start at zero themselves
  * (the plan kernel zeroes the persistent grid's ticket and the split rows' merge counters), so no memset is recorded
  * into a captured graph. Every call
  * on one GPU shares that GPU's array, which keeps the last call's contents: calls that overlap on one GPU (two

@@ -8,6 +8,8 @@
 //                  16-lane row; online softmax per tile; p.v on the VALU in fp32. The four waves and, for long
 //                  rows, the splits are merged by log-sum-exp (a row's splits by whichever finishes last).
 //   prompt item  = (row, q tile, kv head): a row with several queries; the MFMA tile of attn_common.h.
+// A step whose rows all have few queries (drafted tokens, or decode of GQA groups other than 1, 2 and 4) runs on the
+// items of few_query.hip instead, listed as decode items.
 // Launches read a work list built on the device by plan_kernel from the key lengths (and cu_seqlens_q), longest
 // work first; its workspace also holds the split rows' partials and their merge counters.
 //
@@ -16,12 +18,11 @@
 #include <algorithm>
 #include <mutex>
 
-#include "attn_common.h"
+#include "split_rows.h"
 
 namespace lv {
 
 constexpr int kTile = 16;          // decode tokens per tile; block sizes are multiples of 16, so a tile sits in one block
-constexpr int kWaves = 4;          // waves per workgroup
 constexpr int kPlanMaxRows = 4096;  // rows of a step with prompts (the work-list scan lives in LDS)
 
 constexpr int kPromptRing = 2;        // LDS stages of the prompt tiles' ring
@@ -33,6 +34,8 @@ constexpr int kOverlapDecodeWgs = 3;  // persistent decode workgroups per CU bes
 constexpr int kSplitTarget = 4096;    // decode items (x kv heads x query-head groups) a step with split rows aims for
 constexpr int kMaxRowSplits = 128;    // and splits per row on average at most
 constexpr int kMinSplit = 256;        // keys per decode item at least
+constexpr int kFewRound = 512;        // workgroups that the GPU holds at once, two per CU
+constexpr int64_t kFewPartBytes = 14 << 20;  // partials of a step of few queries per row at most (within the static workspace)
 constexpr int kSplitStep = 64;        // and a multiple of this: one tile of every wave
 constexpr int kSmallStepRounds = 8;   // a mixed step of at most this many GPU-fulls of workgroups is one launch
 
@@ -62,73 +65,6 @@ __device__ inline float groups_sum(float x) {
   if constexpr (LPH == 8) x += dpp_ror8(x);
   if constexpr (LPH <= 16) x = xor16_sum(x);
   return xor32_sum(x);
-}
-
-// A split row's partials pass between workgroups that may run on different XCDs, whose L2 caches are not coherent
-// with each other. They are stored and loaded as device-scope relaxed atomics (global_store / global_load with sc1:
-// written through to memory, read past the L2), so neither side needs a whole-L2 writeback or invalidate.
-__device__ __forceinline__ void coherent_store(float* ptr, float v) {
-  __hip_atomic_store(ptr, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float coherent_load(const float* ptr) {
-  return __hip_atomic_load(ptr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Two adjacent floats (8-byte aligned) in one access.
-__device__ __forceinline__ void coherent_store2(float* ptr, float a, float b) {
-  const uint64_t v = (uint64_t)__float_as_uint(a) | (uint64_t)__float_as_uint(b) << 32;
-  __hip_atomic_store(reinterpret_cast<uint64_t*>(ptr), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void coherent_load2(const float* ptr, float& a, float& b) {
-  const uint64_t v =
-      __hip_atomic_load(reinterpret_cast<const uint64_t*>(ptr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  a = __uint_as_float((uint32_t)v);
-  b = __uint_as_float((uint32_t)(v >> 32));
-}
-
-// Merge of a split row's partial outputs (slots slot0 .. slot0 + nsplit - 1) for dims d0, d0 + 1 of query head `head`,
-// written to the output row `tok`: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M). The partials are read
-// kMergeBatch splits at a time, every load of a batch issued before the first is used, with the max and the sums
-// carried from batch to batch: the merge is the serial end of a long row's step, one round trip past the L2 per batch.
-// Each output element's arithmetic depends only on its own head and dim, so any spread of the elements over threads
-// gives the same bits.
-constexpr int kMergeBatch = 32;
-template <typename T, int D>
-__device__ __forceinline__ void merge_split_partials(const AttnParams& p, int slot0, int tok, int head, int nsplit,
-                                                     int d0) {
-  using E = Elem<T>;
-  float m = -INFINITY, den = 0.f, o0 = 0.f, o1 = 0.f;
-  const int64_t first = (int64_t)slot0 * p.hq + head;
-  for (int s0 = 0; s0 < nsplit; s0 += kMergeBatch) {
-    float ls[kMergeBatch], x[kMergeBatch][2];
-#pragma unroll
-    for (int i = 0; i < kMergeBatch; ++i) {
-      ls[i] = -INFINITY;
-      x[i][0] = x[i][1] = 0.f;
-      if (s0 + i < nsplit) {  // uniform over the threads of a row
-        const int64_t at = first + (int64_t)(s0 + i) * p.hq;
-        ls[i] = coherent_load(p.part_lse + at);
-        coherent_load2(p.part_o + at * D + d0, x[i][0], x[i][1]);
-      }
-    }
-    float bm = m;
-#pragma unroll
-    for (int i = 0; i < kMergeBatch; ++i) bm = fmaxf(bm, ls[i]);
-    if (bm == -INFINITY) continue;
-    const float alpha = fast_exp2(m - bm);  // 0 while m is -inf
-    den *= alpha;
-    o0 *= alpha;
-    o1 *= alpha;
-#pragma unroll
-    for (int i = 0; i < kMergeBatch; ++i) {
-      const float w = fast_exp2(ls[i] - bm);  // 0 past the last split
-      den += w;
-      o0 = fmaf(w, x[i][0], o0);
-      o1 = fmaf(w, x[i][1], o1);
-    }
-    m = bm;
-  }
-  const float inv = den > 0.f ? 1.f / den : 0.f;
-  *reinterpret_cast<uint32_t*>(p.out + tok * p.o_st + head * p.o_sh + (int64_t)d0 * 2) = E::pack(o0 * inv, o1 * inv);
 }
 
 // publish (persistent launches): thread 0 stores publish_value there before the item's merge barrier, and the
@@ -390,8 +326,9 @@ __device__ void decode_item(const AttnParams& p, int row, int split, int per, in
     s_last = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nsplit - 1;
   __syncthreads();
   if (s_last) {
-    for (int c = threadIdx.x; c < HG * D / 2; c += blockDim.x)
-      merge_split_partials<T, D>(p, slot0, tok, head_of(c / (D / 2)), nsplit, (c % (D / 2)) * 2);
+    merge_item<T, D>(p, HG * D / 2, 1, nsplit, [&](int c) {
+      return MergePiece{slot0, tok, head_of(c / (D / 2)), (c % (D / 2)) * 2};
+    });
     // Back to zero for the next layer on this plan.
     if (threadIdx.x == 0) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
@@ -409,23 +346,6 @@ struct SmemBytes {
 // are dispatched in list order (longest first). The step's prompt items and its decode items are two lists. Decode
 // items run in decode_list_kernel at the decode item's register budget; prompt items in prompt_list_kernel, whose MFMA
 // tile needs more registers and LDS.
-
-// Decode item i (below the launch's bound, so inside the list's memory), the number of decode items and the keys per
-// split, in one round trip: a decode workgroup's start is a chain of dependent loads (item, then lengths and page,
-// then keys), and a step of a few short rows is little more than that chain.
-struct DecodeWork {
-  int row, split, count, per;
-};
-__device__ __forceinline__ DecodeWork decode_work(const AttnParams& p, int i) {
-  DecodeWork w;
-  int64_t item;
-  asm volatile("s_load_dwordx2 %0, %3, 0x0\n\ts_load_dword %1, %4, %5\n\ts_load_dword %2, %4, %6\n\ts_waitcnt lgkmcnt(0)"
-               : "=&s"(item), "=&s"(w.count), "=&s"(w.per)
-               : "s"(p.items + i), "s"(p.n_items), "n"(4 * kPlanDecodes), "n"(4 * kPlanSplit));
-  w.row = (int)(uint32_t)item;
-  w.split = (int)(item >> 32);
-  return w;
-}
 
 template <typename T, int D, int GS, int HP, int US = 0>
 __global__ __launch_bounds__(256) void decode_list_kernel(AttnParams p) {
@@ -576,7 +496,8 @@ __device__ inline int len_bucket(int keys, int split) {
 // bound on key lengths only sizes the buffers: a captured graph's bound is the longest context it may ever serve, and
 // a batch of a few rows far apart in length has most of its keys in one of them. pieces 0: rows are not split, and
 // one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]; a split
-// that needs more slots than there are (lengths past the caller's bound) is doubled until they fit.
+// that needs more slots than there are (lengths past the caller's bound, rows of unequal query counts) is doubled until
+// they fit. few: rows of several queries are streamed as decode items too, one slot per query.
 struct PlanOut {
   int2* prompts;    // the prompt items
   int2* items;      // the decode items
@@ -590,7 +511,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
                                                             const int32_t* __restrict__ cu_k, int32_t rows,
                                                             int32_t pieces, int32_t max_slots, int32_t qp,
                                                             int32_t max_prompts, int32_t max_items,
-                                                            int32_t last_first, int32_t n_merge,
+                                                            int32_t last_first, int32_t few, int32_t n_merge,
                                                             PlanOut out) {
   __shared__ int pre[kPlanMaxRows + 1];
   __shared__ int full[kPlanMaxRows + 1];
@@ -600,6 +521,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   __shared__ int64_t wave_keys[kScanThreads / 64];
   __shared__ int wave_max[kScanThreads / 64];
   const int tid = threadIdx.x;
+  auto streamed = [&](int lq) { return few ? lq > 0 : lq == 1; };  // a row of decode items
   for (int b = tid; b <= kLenBuckets; b += kScanThreads) bucket[b] = 0;
   for (int i = tid; i < n_merge; i += kScanThreads) out.merge_count[i] = 0;
   // The decode rows' keys in all and at most.
@@ -607,7 +529,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   int longest = 1;
   for (int r = tid; r < rows; r += kScanThreads) {
     const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    if (lq == 1) {
+    if (streamed(lq)) {
       const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
       keys += max(lk, 0);
       longest = max(longest, lk);
@@ -637,10 +559,10 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     for (int r = tid; r < rows; r += kScanThreads) {
       const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
       const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
-      const int n = lq == 1 ? (lk > split ? (lk + split - 1) / split : 1) : 0;  // the row's decode items
-      pre[r] = lq > 1 ? (lq + qp - 1) / qp : 0;
+      const int n = streamed(lq) ? (lk > split ? (lk + split - 1) / split : 1) : 0;  // the row's decode items
+      pre[r] = lq > 1 && !few ? (lq + qp - 1) / qp : 0;
       full[r] = max(n - 1, 0);
-      slots[r] = n > 1 ? n : 0;
+      slots[r] = n > 1 ? n * lq : 0;
     }
     __syncthreads();
     block_scan(slots, rows, wave_tot);
@@ -650,7 +572,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   }
   for (int r = tid; r < rows; r += kScanThreads) {
     const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    if (lq == 1) {
+    if (streamed(lq)) {
       const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
       const int n = lk > split ? (lk + split - 1) / split : 1;
       atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
@@ -681,7 +603,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     for (int i = pre[r]; i < pre[r + 1]; ++i)
       if (i < max_prompts) out.prompts[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
     const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    if (lq == 1) {
+    if (streamed(lq)) {
       const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
       const int n = lk > split ? (lk + split - 1) / split : 1;
       const int pos = nfull + atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
@@ -715,37 +637,66 @@ static int pick_gs(int group) {
   return 1;
 }
 
+// Queries per row that a step of few queries may have (0: the GQA group is too wide). Past 32 query rows per kv head an
+// item at D = 128 streams its keys into LDS twice, and the prompt items (128 query rows, unsplit) are as fast once they
+// fill the GPU: 16 queries a row of 32/8 heads, two layers, 8 rows 162 against 398 us, 48 rows 758 against 492. At D = 64
+// it stays with one copy: 48 rows 231 against 308 us, 8 rows 83 against 256. (A decode row of a group that wide is a few-query
+// row all the same: the VALU items would read its keys once per four heads.)
+static int few_queries(int64_t rows, int32_t hkv, int32_t d, int group) {
+  const int most = d == 64 || group > 32 || rows * hkv <= kFewRound / 4 ? kFewMaxRows : kFewMaxRows / 2;
+  return std::min(kFewMaxQueries, most / group);
+}
+
 static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, int32_t d, int32_t max_k,
-                        bool listed) {
+                        bool listed, bool few) {
   Shape s{};
   const int group = hq / hkv;
   s.gs = pick_gs(group);
-  const int64_t per_split = (int64_t)hkv * (group / s.gs);  // decode items per row and split
+  const int64_t per_split = few ? hkv : (int64_t)hkv * (group / s.gs);  // decode items per row and split
   const int64_t keys = max_k > 0 ? max_k : 1;
-  // Rows split only in a listed step (whose workspace holds the partial slots and merge counters) whose unsplit items
-  // are at most half the target: with more, the longest-first list balances them as they are.
+  // Rows split only in a listed step (whose workspace holds the partial slots and merge counters). The number of pieces
+  // weighs the list's balance against the merge of a row, its round trips past the L2 after its last split.
   //
-  // The number of splits weighs the list's balance against the merge of a row, one round trip past the L2 per
-  // kMergeBatch splits after its last split: 4096 one-head items for many rows, fewer for a few long ones. 32/8 heads,
-  // d128, contexts U[32K, 128K], 1024 / 2048 / 3072 / 4096 items (before, 4096 with batches of 16): 1 row
+  // Where unsplit items fill the GPU (VALU: more than half the items aimed for; few queries: more than one round), the
+  // longest-first list balances them as they are, and only a row of more than two workgroups' share of all keys is split.
+  //
+  // VALU decode items: 4096 one-head items for many rows, fewer for a few long ones. 32/8 heads, d128, contexts
+  // U[32K, 128K], 1024 / 2048 / 3072 / 4096 items (before, 4096 of sizes set by the longest row): 1 row
   // 93 / 113 / 125 / 132 us (166), 2 rows 174 / 181 / 192 / 190 (219), 3 rows 252 / 250 / 256 / 261 (272), 8 rows
-  // 594 / 557 / 567 / 569 (585), 24 rows 1494 / 1399 / 1372 / 1384 (1452); 48 rows U[4K, 64K] 1431 / 1283 / 1237 / 1241
-  // (1309).
-  const int64_t items = rows <= 2 ? kSplitTarget / 4 : rows <= 16 ? kSplitTarget / 2 : kSplitTarget;
-  const int64_t target =  // splits of all rows
-      std::min<int64_t>((items + per_split - 1) / per_split, (int64_t)kMaxRowSplits * rows);
-  const bool split = listed && 2 * (int64_t)rows <= target && keys > kMinSplit;
-  s.pieces = split ? (int32_t)(target - rows) : 0;
-  const int64_t most = split ? (keys + kMinSplit - 1) / kMinSplit : 1;  // of one row
-  const int64_t splits = split ? std::min(rows * most, target) : rows;
+  // 594 / 557 / 567 / 569 (585), 24 rows 1494 / 1399 / 1372 / 1384 (1452); 48 rows U[4K, 64K] 1431 / 1283 / 1237 / 1241 (1309).
+  //
+  // Steps of few queries (few_query.hip, two workgroups per CU whatever the group): a full piece is one workgroup's share
+  // of all keys, so the full pieces run in one round and the rows' remainders pack beside them; up to kFewRound / 8
+  // rows' remainders are counted in, so that all run at once. More pieces cost more than they balance, their partials
+  // being several query rows each. 32/8 heads, d128, 4 queries a row, contexts U[512, 8192], two layers, pieces of half
+  // a share / two thirds / one: 12 rows 121 / 117 / 110 us, 24 rows 193 / 192 / 182, 48 rows 346 / 353 / 336; 4 rows with
+  // their remainders beside the round 66.7, in it 57.9; 100 rows split by shares 631, unsplit 624.
+  const int64_t units = rows * per_split;
+  const int64_t row_queries = few ? ((int64_t)tokens + rows - 1) / rows : 1;  // partial slots per split
+  const int64_t share = std::max<int64_t>(1, kFewRound / per_split);  // splits of one round of workgroups
+  int64_t pieces = std::max<int64_t>(1, share / 2);
+  if (few && row_queries * group > 4) {
+    if (units <= kFewRound) pieces = std::min(share - (8 * rows <= share ? rows : 0), (int64_t)kMaxRowSplits * rows);
+    const int64_t max_slots = kFewPartBytes / ((int64_t)hq * (d + 1) * (int64_t)sizeof(float));
+    if ((pieces + std::min<int64_t>(rows, pieces)) * row_queries > max_slots) pieces = max_slots / row_queries / 2;
+  } else {  // up to four query rows an item weighs no more than a VALU item and splits as one
+    const int64_t items = rows <= 2 ? kSplitTarget / 4 : rows <= 16 ? kSplitTarget / 2 : kSplitTarget;
+    const int64_t splits = std::min<int64_t>((items + per_split - 1) / per_split, (int64_t)kMaxRowSplits * rows);
+    if (2 * (int64_t)rows <= splits) pieces = splits - rows;
+  }
+  if (!listed || keys <= kMinSplit) pieces = 0;
+  s.pieces = (int32_t)pieces;
+  const int64_t most = pieces > 0 ? (keys + kMinSplit - 1) / kMinSplit : 1;  // splits of one row
+  const int64_t splits = std::min(rows * most, pieces + rows);  // of all rows
   s.max_splits = (int32_t)std::min(most, splits);
   const int qp = kPrefillRows / (group > 0 ? group : 1);
   // In 64 bits, saturated: a count past INT32_MAX is far past what one launch holds (check_grids refuses it).
   auto sat = [](int64_t x) { return (int32_t)std::min<int64_t>(x, INT32_MAX); };
-  s.max_prompt_items = listed ? sat(((int64_t)tokens + qp - 1) / qp + rows) : 0;
+  s.max_prompt_items = listed && !few ? sat(((int64_t)tokens + qp - 1) / qp + rows) : 0;
   s.max_decode_items = listed ? sat(splits) : 0;
   s.max_items = sat((int64_t)s.max_prompt_items + s.max_decode_items);
-  s.slots = s.max_splits > 1 ? sat(splits) : 0;
+  // Rows of more than one split hold more keys than a split, so there are at most `pieces` of them.
+  s.slots = s.max_splits > 1 ? sat(std::min(splits, pieces + std::min<int64_t>(rows, pieces)) * row_queries) : 0;
   size_t off = 0;
   s.items_off = off;
   off += (size_t)s.max_items * sizeof(int2);
@@ -825,6 +776,9 @@ struct StepKind {
   bool mixed;         // some row has more than one query
   bool overlap;       // the caller's schedule lets prompt tiles run beside the decode items
   bool prompts_only;  // the caller says every row has more than one query
+  bool few;           // every row's query heads fit one MFMA item per kv head (few_query.hip)
+  int max_q;          // queries per row at most
+  int tokens;
   int prompt_wgs;     // the caller's prompt share of the CUs in an overlap (0: the default)
 };
 struct Route {
@@ -1014,6 +968,33 @@ static int launch_d(const AttnParams& p, int d, int gs, const Shape& s, const St
   }
 }
 
+// A step's kernels after the plan, by its kind: rows of few queries on few_query.hip's items, else by dtype, head dim,
+// lane group, kv heads per item and pages.
+static int launch_step(const AttnParams& p, int d, const Shape& s, const StepKind& k, int dtype, hipStream_t stream,
+                       Route* info) {
+  if (k.few) {
+    Route r;
+    r.decode = LV_KERNEL_DECODE_LIST;
+    // Pairs of kv heads (512-byte pieces of a token's row): where two rounds of workgroups remain without splits (200
+    // rows of 4 queries 1178 -> 1114 us, two layers; 100 rows 631 -> 737), or items are light and fill the CUs.
+    const int64_t items = (int64_t)s.max_decode_items * p.hkv;
+    const bool light = ((int64_t)k.tokens + p.rows - 1) / p.rows * p.group <= 4;  // as plan_shape has it
+    const bool pairs = light ? items >= kFewRound : (int64_t)p.rows * p.hkv >= 2 * kFewRound;
+    r.hp = p.hkv % 2 == 0 && k.max_q * p.group <= 32 && pairs ? 2 : 1;
+    r.decode_grid = s.max_decode_items * (p.hkv / r.hp);
+    r.merge = s.max_splits > 1;
+    if (info) {
+      *info = r;
+      return LV_OK;
+    }
+    launch_few_query(p, d, k.max_q * p.group, r.hp, dtype, s.max_decode_items, stream);
+    LV_LAUNCH_CHECK("few_list_kernel");
+    return LV_OK;
+  }
+  return dtype == LV_DTYPE_BF16 ? launch_d<BF16>(p, d, s.gs, s, k, stream, info)
+                                : launch_d<F16>(p, d, s.gs, s, k, stream, info);
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // The workspace of lv_paged_attention_static: a file-scope device array (each GPU that loads the library holds its
 // own copy until the process ends). Host code must not pass the array's name to a kernel -- in host code it is a
@@ -1060,11 +1041,11 @@ struct PlanSig {
   const void* ws = nullptr;
   const int32_t *cu_q = nullptr, *lens = nullptr, *cu_k = nullptr;
   int64_t rows = 0, tokens = 0, max_k = 0, pieces = 0, qp = 0, max_items = 0, bytes = 0;
-  bool mixed = false, last_first = false;
+  bool mixed = false, last_first = false, few = false;
   bool operator==(const PlanSig& o) const {
     return ws == o.ws && cu_q == o.cu_q && lens == o.lens && cu_k == o.cu_k && rows == o.rows &&
            tokens == o.tokens && max_k == o.max_k && pieces == o.pieces && qp == o.qp && max_items == o.max_items &&
-           bytes == o.bytes && mixed == o.mixed && last_first == o.last_first;
+           bytes == o.bytes && mixed == o.mixed && last_first == o.last_first && few == o.few;
   }
 };
 constexpr int kPlanRecords = 32;
@@ -1135,14 +1116,21 @@ static int check_shape(int32_t num_rows, int32_t num_tokens, int32_t num_heads, 
   return LV_OK;
 }
 
-static StepKind step_kind(int32_t num_rows, bool has_cu_q, int32_t max_seqlen_q, int32_t schedule,
-                          int32_t prompt_workgroups, int32_t flags) {
+static StepKind step_kind(int32_t num_rows, int32_t num_tokens, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
+                          bool has_cu_q, int32_t max_seqlen_q, int32_t schedule, int32_t prompt_workgroups,
+                          int32_t flags) {
+  const int group = num_heads / num_kv_heads;
+  const int few = few_queries(num_rows, num_kv_heads, head_dim, group);
   StepKind k;
   k.mixed = has_cu_q && max_seqlen_q > 1;
   k.listed = num_rows <= kPlanMaxRows;
   k.overlap = schedule != LV_SCHEDULE_SERIAL;
   k.prompts_only = (flags & LV_ATTN_PROMPTS_ONLY) != 0;
   k.prompt_wgs = prompt_workgroups;
+  k.max_q = k.mixed ? max_seqlen_q : 1;
+  k.tokens = num_tokens;
+  k.few = k.listed && k.max_q <= few && num_tokens <= (int64_t)num_rows * few &&
+          (k.mixed || pick_gs(group) != group);
   return k;
 }
 
@@ -1196,8 +1184,10 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   LV_REQUIRE(cache_stride_token >= 0 && (int64_t)kPrefillKeys * cache_stride_token * 2 < (int64_t)1 << 30,
              "paged_attention: cache token stride %lld is negative or too large", (long long)cache_stride_token);
   LV_REQUIRE(scale > 0.f, "paged_attention: the softmax scale must be positive, got %g", (double)scale);
-  const StepKind kind = step_kind(num_rows, cu_seqlens_q != nullptr, max_seqlen_q, schedule, prompt_workgroups, flags);
-  const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed);
+  const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, cu_seqlens_q != nullptr, max_seqlen_q,
+                                  schedule, prompt_workgroups, flags);
+  const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
+                             kind.few);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
   if (static_ws) {
@@ -1262,6 +1252,7 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   sig.max_items = s.max_items;
   sig.bytes = (int64_t)s.bytes;
   sig.mixed = kind.mixed;
+  sig.few = kind.few;
   sig.last_first = kind.prompts_only || !kind.overlap;  // prompt items with the GPU to themselves: last tile first
   bool planned = false;
   if (kind.listed && !plan_is_current(sig, (flags & LV_ATTN_REUSE_PLAN) != 0)) {
@@ -1271,12 +1262,11 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
                       reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kScanThreads), 0, st, kind.mixed ? cu_seqlens_q : nullptr,
                        seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
-                       s.max_decode_items, (int32_t)sig.last_first, (int32_t)s.merges, out);
+                       s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few, (int32_t)s.merges, out);
     LV_LAUNCH_CHECK("plan_kernel");
     planned = true;
   }
-  const int rc = dtype == LV_DTYPE_BF16 ? launch_d<BF16>(p, head_dim, s.gs, s, kind, st, nullptr)
-                                        : launch_d<F16>(p, head_dim, s.gs, s, kind, st, nullptr);
+  const int rc = launch_step(p, head_dim, s, kind, dtype, st, nullptr);
   if (rc != LV_OK) {
     // A failed launch may leave the persistent grid's ticket unreset: the next call on this workspace plans again.
     record_plan(workspace, nullptr);
@@ -1298,7 +1288,11 @@ extern "C" size_t lv_paged_attention_workspace_bytes(int32_t num_rows, int32_t n
     return 0;
   const bool mixed = decode_only == 0;
   const bool listed = mixed || num_rows <= kPlanMaxRows;
-  return plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed).bytes;
+  const size_t bytes = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, false).bytes;
+  // The longest row's queries are not known here: a step whose rows may all have few takes the larger of the two.
+  const int group = num_heads / num_kv_heads;
+  if (!listed || num_tokens > (int64_t)num_rows * few_queries(num_rows, num_kv_heads, head_dim, group) || (!mixed && pick_gs(group) == group)) return bytes;
+  return std::max(bytes, plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, true).bytes);
 }
 
 extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t num_heads,
@@ -1313,15 +1307,16 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
                               has_cu_seqlens_q != 0, max_seqlen_q, max_seqlen_k, schedule, prompt_workgroups, flags,
                               dtype);
   if (rc0 != LV_OK || num_rows == 0 || num_tokens == 0) return rc0;
-  const StepKind kind = step_kind(num_rows, has_cu_seqlens_q != 0, max_seqlen_q, schedule, prompt_workgroups, flags);
-  const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed);
+  const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, has_cu_seqlens_q != 0, max_seqlen_q,
+                                  schedule, prompt_workgroups, flags);
+  const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
+                             kind.few);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
   AttnParams p{};
   shape_params(p, s, num_rows, num_heads, num_kv_heads, block_size, cache_stride_head);
   Route r;
-  const int rc = dtype == LV_DTYPE_BF16 ? launch_d<BF16>(p, head_dim, s.gs, s, kind, nullptr, &r)
-                                        : launch_d<F16>(p, head_dim, s.gs, s, kind, nullptr, &r);
+  const int rc = launch_step(p, head_dim, s, kind, dtype, nullptr, &r);
   if (rc != LV_OK) return rc;
   info->decode_kernel = r.decode;
   info->decode_workgroups = r.decode_grid;
