@@ -7,14 +7,14 @@
 // latents 0 .. L - lq + j.
 //
 // Two schedules, both streaming latents from HBM straight into an LDS ring (global_load_lds_dwordx4):
-//   balanced runs (mla_run_kernel)  pages a multiple of 16 latents: the units' 16-latent stages, end to end, are cut
+//   balanced runs (mla_run_kernel)  pages a multiple of 16 latents: the units' 32-latent stages, end to end, are cut
 //                                   into equal runs, one per workgroup; units cut by run boundaries are merged by
 //                                   log-sum-exp in mla_run_merge_kernel.
 //   split schedule (mla_decode_dma_kernel)  other page sizes, or more units than the runs' in-kernel scan holds:
 //                                   one workgroup per (row, split of <= 4096 latents, query, 16-head tile); split
 //                                   rows are merged by log-sum-exp in mla_merge_kernel.
-// Per 16-latent stage: S^T = Lat Q^T (16 latents x 16 heads, K = 576) on MFMA 16x16x32, the online softmax per
-// head, and O^T += V^T P^T (512 dims x 16 heads) on MFMA 16x16x16 with V^T operands from gfx950's transposing LDS
+// Per 16 latents: S^T = Lat Q^T (16 latents x 16 columns, K = 576) on MFMA 16x16x32, the online softmax per
+// column, and O^T += V^T P^T (512 dims) on MFMA 16x16x32 or 16x16x16 with V^T operands from gfx950's transposing LDS
 // read (ds_read_b64_tr_b16).
 #include <algorithm>
 
@@ -48,9 +48,10 @@ struct MlaParams {
   char* out;
   int64_t o_st, o_sh;  // bytes
   int32_t split, max_splits;
-  float* part_o;    // split schedule: [rows * lq][heads][max_splits][kVDim]; runs: [runs][2][16][kVDim]
-  float* part_lse;  // split schedule: [rows * lq][heads][max_splits]; runs: [runs][2][16]; log2 domain
-  int32_t units;    // runs: (row, query, 16-head tile) units
+  float* part_o;    // split schedule: [rows * lq][heads][max_splits][kVDim]; runs: [runs][2][16 NB][kVDim]
+  float* part_lse;  // split schedule: [rows * lq][heads][max_splits]; runs: [runs][2][16 NB]; log2 domain
+  int32_t units;    // runs: (row, tile of 16 NB (query, head) columns) units
+  int32_t tiles;    // runs: units per row
   int32_t* prefix;  // runs: [units + 2] stage prefix over units, then the stage total and the run length
 };
 
@@ -250,83 +251,114 @@ __global__ __launch_bounds__(256) void mla_decode_dma_kernel(MlaParams p) {
 // ---------------------------------------------------------------------------------------------------------
 // Balanced schedule over equal runs of stages, for pages whose size is a multiple of 16 latents.
 //
-// Unit u = (row, query j, 16-head tile), u = (row * lq + j) * htiles + tile, needs T_u = ceil(L_u / 16) stages
-// of 16 latents (L_u latents seen). Laid end to end (prefix P_u) the units' stages are cut into equal runs, one
-// per workgroup of a grid that fills the GPU once; every workgroup streams its run through the LDS ring of the
-// kernel above, each unit it enters preceded by one stage holding that unit's 16 query rows (the same 16 x 576
-// shape as a latent stage). A unit that lies wholly inside one run is finished in place. A unit cut by run
-// boundaries leaves (o / l, log2 l + m) per head in slot 0 (the run's first unit) or slot 1 (its last unit) of
-// every run it touches, and mla_run_merge_kernel combines them; that kernel also writes the zero output of units
-// that see no latents. Every run does equal work, whatever the spread of row lengths, and partials are written
-// only where a row crosses a run boundary.
+// A row's columns are its (query j, head) pairs, c = j * heads + head. Unit u = (row, tile of 16 NB columns), u = row *
+// tiles + tile, needs T_u = ceil(L_u / 32) stages of 32 latents (L_u: the latents its last query sees; a column of an
+// earlier query masks its last ones). Laid end to end (prefix P_u) the units' stages are cut into equal runs, one per
+// workgroup of a grid that fills the GPU once; every workgroup streams its run through an LDS ring, each unit it enters
+// preceded by a stage holding that unit's query rows. A unit that lies wholly inside one run is finished in place. A unit cut by run boundaries leaves (o / l, log2 l + m) per column in slot 0 (the run's
+// first unit) or slot 1 (its last unit) of every run it touches, and mla_run_merge_kernel combines them; that kernel also
+// writes the zero output of columns that see no latents. Every run does equal work, whatever the spread of row lengths,
+// and partials are written only where a row crosses a run boundary.
 //
-// Each stage's work (the score MFMAs, their exchange, the softmax, P.V) runs between two barriers of one
-// workgroup. On DeepSeek-V2-Lite's step, two workgroups per CU with a two-stage ring (one stage in flight while one
-// is consumed) stream fastest. That is 5% faster than three per CU: their extra runs cut more units, and each cut
-// leaves partials to write and merge. It is 3% faster than two per CU with three stages. One workgroup with five or
-// eight stages is 40% slower.
+// NB is 1 for rows of up to 16 columns, else 2: drafts and heads past 16 share the latents that a workgroup has in LDS
+// instead of streaming them again. (Four blocks spill: 64 heads 1047 us against 458.)
+//
+// One workgroup of 8 waves per CU, a ring of three 36 KB stages, two in flight. Wave (lb, cb) of the first 2 NB computes
+// the scores of 16 latents for 16 columns over the whole K = 576 (its Q^T in registers) and leaves their probabilities in
+// LDS as the P^T operand; the other waves meanwhile issue the stage loads; after a barrier every wave adds P.V for 64 of
+// the 512 output dims and all columns, V^T from the transposing read. Two barriers per 32 latents. The max of a column is
+// shared: a score past it by more than kRescaleSlack makes the workgroup take the stage's maxima from LDS, rescale and
+// write the probabilities again (rare: the first stage of a unit, seldom another).
+//
+// Bound by HBM up to 32 columns (a build without the scores and P.V streams 128 rows of 1024-16384 latents in 201 us,
+// 6.55 TB/s; the scores' serial chain through LDS and the two barriers are what is left). Against the schedule before,
+// two workgroups of 4 waves per CU with a 16-latent stage each, every query and every 16 heads a unit of their own:
+// 128 rows, 16 heads 218 us (217), 32 heads 229 (426), 64 heads 454 (850), 128 heads 890 (1670); two layers of 20 rows,
+// 1024-8192 latents, 16 heads, 2 queries 76 us (108), 3 queries 104 (138), 128 heads 171 (298); 4 rows 57 (70).
 
-constexpr int kRunMin = 16;          // stages per run at least (256 latents)
-constexpr int kRunStages = 2;        // ring depth of a run
-constexpr int kRunsPerCU = 2;        // run workgroups per CU
+constexpr int kRunTile = 32;         // latents per stage
+constexpr int kRunMin = 2;           // stages per run at least
+constexpr int kRunStages = 3;        // ring depth (four stream no faster)
+constexpr int kRunWaves = 8;
+constexpr int kRunsPerCU = 1;        // run workgroups per CU
 constexpr int kRunMaxUnits = 8192;   // units the in-kernel scan serves
+constexpr int kRunRow = kLatent;     // LDS row pitch in elements: no padding, 16-byte chunk c of row r at c ^ (r & 6), so
+                                     // that operand and transposing reads meet no bank conflicts
+constexpr int kRunElems = kRunTile * kRunRow;
+constexpr int kRunLoads = kRunTile * kLatChunks / 64;  // 64-lane loads per stage, 18 per 16 rows
 
-__device__ __forceinline__ int unit_latents(const MlaParams& p, int u) {
-  const int tq = u / p.htiles;  // row * lq + j
-  const int row = tq / p.lq, qj = tq - row * p.lq;
-  return p.lens[row] - p.lq + qj + 1;
+// At most N of this wave's loads outstanding and its LDS reads of the stage before done; then the other waves' are.
+template <int N>
+__device__ __forceinline__ void run_wait() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-__device__ __forceinline__ int unit_latents_uniform(const MlaParams& p, int u) {
-  const int tq = u / p.htiles;
-  const int row = tq / p.lq, qj = tq - row * p.lq;
-  return sload(p.lens + row) - p.lq + qj + 1;
+// Latents that the last query of unit u = (row, tile) sees, from the row's cached latents.
+template <int NB>
+__device__ __forceinline__ int unit_latents(const MlaParams& p, int tile, int len) {
+  const int last = min((tile + 1) * 16 * NB, p.lq * p.heads) - 1;  // the unit's last column
+  return len - p.lq + last / p.heads + 1;
 }
 
+template <int NB>
 __device__ __forceinline__ int unit_stages(const MlaParams& p, int u) {
-  const int lk = unit_latents(p, u);
-  return lk > 0 ? (lk + kDmaTile - 1) / kDmaTile : 0;
+  const int row = u / p.tiles;
+  const int lk = unit_latents<NB>(p, u - row * p.tiles, p.lens[row]);
+  return lk > 0 ? (lk + kRunTile - 1) / kRunTile : 0;
 }
 
-// Position in a run's stage sequence: unit u (prefix pu, tu stages, lk latents), next tile t (-1: its query). The
-// unit's query row tq and head tile ht, its block-table row, and the cache page of the last tile loaded are kept
-// here, so a stage's loads need no division and at most one page lookup per page.
+// Position in a run's stage sequence: unit u (prefix pu, tu stages, lk latents), next tile t (-1: its queries). The
+// unit's row and column tile and its block-table row are kept here, so a stage's loads need no division.
 struct RunCursor {
   int u, pu, tu, lk, t;
-  int tq, ht, pg;
+  int row, len, tile, pg[2];
   const int32_t* table;
-  const char* page;
+  const char* page[2];  // cache pages pg[] of the last stage's two blocks
   bool done;
 };
 
-template <typename T, int STAGES>
-__global__ __launch_bounds__(256) void mla_run_kernel(MlaParams p) {
-  static_assert(STAGES >= 2 && STAGES <= 8, "the stage waits cover up to seven stages in flight");
+template <typename T, int NB>
+__global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p) {
   using E = Elem<T>;
-  __shared__ __attribute__((aligned(16))) uint16_t ring[STAGES * kDmaStageElems];
-  __shared__ f32x4 spart[4][64];  // each wave's partial S^T of the stage
-  __shared__ int wave_tot[4];
-  __shared__ int first[2];
+  constexpr int W = kRunWaves, LB = kRunTile / 16;  // 16-latent blocks of a stage
+  constexpr int DB = kVDim / 16 / W;                // 16-dim output blocks per wave
+  constexpr int SW = LB * NB;                       // waves that compute scores
+  // The other waves load the stages: their cursor and address work runs beside the scores.
+  constexpr int LW = W - SW;
+  constexpr int kPer = kRunLoads / LW;              // loads per stage
+  static_assert(kPer * LW == kRunLoads && kRunStages == 3, "as many for each; one stage ahead of the awaited one");
+  static_assert(SW < W && LB == 2 && NB <= LB, "waves for scores and loads; a stage holds a unit's query rows");
+  __shared__ __attribute__((aligned(16))) uint16_t ring[kRunStages * kRunElems];
+  __shared__ u32x2 s_p[NB][LB][64];      // P^T operands of the stage
+  __shared__ float s_max[NB][LB][16];    // its maxima
+  __shared__ float s_sum[NB][LB][16];    // row sums at a unit's end
+  __shared__ int s_grow[8];
+  __shared__ int wave_tot[W];
+  __shared__ int first[3];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
   const float c = p.scale_log2;
+  const int lb = wave % LB, cb = wave / LB;  // the scores this wave computes (wave < SW)
+  const int columns = p.lq * p.heads;
 
   // Stage counts over units; thread tid sums units [ulo, uhi). Exclusive scan of those sums across the block.
-  const int per_thread = (p.units + 255) / 256;
+  const int per_thread = (p.units + 64 * W - 1) / (64 * W);
   const int ulo = min(tid * per_thread, p.units), uhi = min(ulo + per_thread, p.units);
-  int local = 0;
-  for (int u = ulo; u < uhi; ++u) local += unit_stages(p, u);
-  int x = local;
-  for (int d = 1; d < 64; d <<= 1) {
-    const int y = __shfl_up(x, d, 64);
-    if (lane >= d) x += y;
+  int local = 0, len0 = 0;  // len0: latents of unit ulo's row
+  for (int u = ulo; u < uhi; ++u) {
+    const int row = u / p.tiles, len = p.lens[row];
+    const int lk = unit_latents<NB>(p, u - row * p.tiles, len);
+    local += lk > 0 ? (lk + kRunTile - 1) / kRunTile : 0;
+    len0 = u == ulo ? len : len0;
   }
+  const int x = wave_incl_scan(local);
   if (lane == 63) wave_tot[wave] = x;
+  if (tid < 8) s_grow[tid] = 0;
   __syncthreads();
   int excl = x - local, total = 0;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < W; ++w) {
     excl += w < wave ? wave_tot[w] : 0;
     total += wave_tot[w];
   }
@@ -336,7 +368,7 @@ __global__ __launch_bounds__(256) void mla_run_kernel(MlaParams p) {
     int run = excl;
     for (int u = ulo; u < uhi; ++u) {
       p.prefix[u] = run;
-      run += unit_stages(p, u);
+      run += unit_stages<NB>(p, u);
     }
     if (tid == 0) {
       p.prefix[p.units] = total;
@@ -348,29 +380,32 @@ __global__ __launch_bounds__(256) void mla_run_kernel(MlaParams p) {
   const int end = min(start + per, total);
   if (local > 0 && excl <= start && start < excl + local) {
     int u = ulo, acc = excl;
-    for (int tu = unit_stages(p, u); acc + tu <= start; tu = unit_stages(p, u)) {
-      acc += tu;
-      ++u;
-    }
+    if (per_thread > 1)
+      for (int tu = unit_stages<NB>(p, u); acc + tu <= start; tu = unit_stages<NB>(p, u)) {
+        acc += tu;
+        ++u;
+      }
     first[0] = u;
     first[1] = acc;
+    first[2] = u == ulo ? len0 : p.lens[u / p.tiles];
   }
   __syncthreads();
 
   // Both cursors walk the same sequence: for each unit, its query stage, then its tiles inside [start, end).
-  auto enter = [&](RunCursor& r, int u, int pu) {
-    int lk = unit_latents_uniform(p, u);
-    while (lk <= 0) lk = unit_latents_uniform(p, ++u);  // units without latents hold no stages
+  auto enter = [&](RunCursor& r, int u, int pu, int len = -1) {
+    for (;; ++u) {  // units without latents hold no stages
+      r.row = u / p.tiles;
+      r.tile = u - r.row * p.tiles;
+      r.len = len >= 0 ? len : sload(p.lens + r.row);
+      r.lk = unit_latents<NB>(p, r.tile, r.len);
+      if (r.lk > 0) break;
+    }
     r.u = u;
     r.pu = pu;
-    r.lk = lk;
-    r.tu = (lk + kDmaTile - 1) / kDmaTile;
+    r.tu = (r.lk + kRunTile - 1) / kRunTile;
     r.t = -1;
-    r.tq = u / p.htiles;
-    r.ht = u - r.tq * p.htiles;
-    r.table = p.tables + (int64_t)(r.tq / p.lq) * p.t_stride;
-    r.pg = -1;
-    r.page = nullptr;
+    r.table = p.tables + (int64_t)r.row * p.t_stride;
+    r.pg[0] = r.pg[1] = -1;
     r.done = false;
   };
   auto advance = [&](RunCursor& r) {
@@ -385,139 +420,245 @@ __global__ __launch_bounds__(256) void mla_run_kernel(MlaParams p) {
     }
   };
   RunCursor prod, cons;
-  enter(prod, __builtin_amdgcn_readfirstlane(first[0]), __builtin_amdgcn_readfirstlane(first[1]));
+  enter(prod, __builtin_amdgcn_readfirstlane(first[0]), __builtin_amdgcn_readfirstlane(first[1]),
+        __builtin_amdgcn_readfirstlane(first[2]));
   cons = prod;
 
-  // This wave's loads j = wave + 4 i (i < 5) of a stage's 19: slot 64 j + lane is 16-byte chunk `part` of row r
-  // (latent or head) of the stage. Slots 74 r + 72 and 74 r + 73 of row r are LDS padding, filled with copies of
-  // chunk 71.
-  int lrow[5], lpart[5];
+  // Loader wave lw's loads j = lw + LW i of a stage's 36: each lies in 16-row block j / 18, slot 64 (j % 18) + lane of it
+  // holding position slot % 72 of its row slot / 72, so the chunk that belongs there.
+  const bool loader = wave >= SW;
+  const int lw = loader ? wave - SW : 0;
+  // Whether load i of this wave lies in the second block: known for most i, whatever the wave.
+  auto second = [&](int i) {
+    return LW * i >= kRunLoads / LB || (LW * i + LW > kRunLoads / LB && lw >= kRunLoads / LB - LW * i);
+  };
+  int lrow[kPer], lchunk[kPer];
 #pragma unroll
-  for (int i = 0; i < 5; ++i) {
-    const int slot = min(64 * (wave + 4 * i) + lane, kDmaStageSlots - 1);
-    lrow[i] = slot / kDmaRowSlots;
-    lpart[i] = min(slot - lrow[i] * kDmaRowSlots, kLatChunks - 1) * 16;
+  for (int i = 0; i < kPer; ++i) {
+    const int slot = 64 * ((lw + LW * i) % (kRunLoads / LB)) + lane;
+    lrow[i] = slot / kLatChunks;
+    lchunk[i] = ((slot - lrow[i] * kLatChunks) ^ (lrow[i] & 6)) * 16;
   }
-  // Query stage: head ht 16 + r of the unit's token (heads past the last load the last head; not written).
-  // Latent stage: latents t0 .. t0 + 15 of the row, one page (the page size is a multiple of 16); latents at
+  // Query stage: the 32 columns from the unit's first (columns past the row's last load the last; unused).
+  // Latent stage: latents t0 .. t0 + 31 of the row, each 16 in one page (the page size is a multiple of 16); latents at
   // or past lk load latent lk - 1 instead (finite values; their weight is 0).
   auto fill = [&](RunCursor& r, uint16_t* stage) {
     if (r.t < 0) {
-      const char* qrow = p.q + r.tq * p.q_st;
+      const int c0 = r.tile * NB * 16;
 #pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int j = wave + 4 * i;
-        if (j < kDmaInstr && 64 * j + lane < kDmaStageSlots)
-          lds_dma16(qrow + (int64_t)min(r.ht * 16 + lrow[i], p.heads - 1) * p.q_sh + lpart[i],
-                    lds_addr(stage + 64 * 8 * j));
+      for (int i = 0; i < kPer; ++i) {
+        const int j = lw + LW * i;
+        const int col = min(c0 + (second(i) ? 16 : 0) + lrow[i], columns - 1), qj = col / p.heads;
+        lds_dma16(p.q + (int64_t)(r.row * p.lq + qj) * p.q_st + (int64_t)(col - qj * p.heads) * p.q_sh + lchunk[i],
+                  lds_addr(stage + 64 * 8 * j));
       }
     } else {
-      const int t0 = r.t * kDmaTile;
-      const int pg = (int)p.bs.div(t0);
-      if (pg != r.pg) {
-        r.pg = pg;
-        r.page = p.cache + (int64_t)sload(r.table + pg) * p.c_sb;
+      const int t0 = r.t * kRunTile;
+      const int s0 = t0, s1 = min(t0 + 16, r.lk - 1);  // first latent of either block
+      const int g0 = (int)p.bs.div(s0), g1 = (int)p.bs.div(s1);
+      if (g0 != r.pg[0] || g1 != r.pg[1]) {
+        const int32_t* const where[2] = {r.table + g0, r.table + g1};
+        int page[2];
+        sload_n<2>(where, page);
+        r.pg[0] = g0;
+        r.pg[1] = g1;
+        r.page[0] = p.cache + (int64_t)page[0] * p.c_sb;
+        r.page[1] = p.cache + (int64_t)page[1] * p.c_sb;
       }
-      const char* base = r.page + (int64_t)(t0 - pg * (int)p.bs.d) * p.c_st;
-      const int last = r.lk - 1 - t0;
+      const char* b0 = r.page[0] + (int64_t)(s0 - g0 * (int)p.bs.d) * p.c_st;
+      const char* b1 = r.page[1] + (int64_t)(s1 - g1 * (int)p.bs.d) * p.c_st;
+      const int last0 = r.lk - 1 - s0, last1 = r.lk - 1 - s1;
 #pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const int j = wave + 4 * i;
-        if (j < kDmaInstr && 64 * j + lane < kDmaStageSlots)
-          lds_dma16(base, (uint32_t)(min(lrow[i], last) * (int)p.c_st + lpart[i]), lds_addr(stage + 64 * 8 * j));
+      for (int i = 0; i < kPer; ++i) {
+        const int j = lw + LW * i;
+        lds_dma16(second(i) ? b1 : b0, (uint32_t)(min(lrow[i], second(i) ? last1 : last0) * (int)p.c_st + lchunk[i]),
+                  lds_addr(stage + 64 * 8 * j));
       }
     }
   };
 
-  // S^T = Lat Q^T over K = 576 is split over the waves: wave w takes MFMA k-steps [s0, s0 + ns) of the 18.
-  const int s0 = wave < 2 ? 5 * wave : 4 * wave + 2, ns = wave < 2 ? 5 : 4;
-  u32x4 qb[5];
-  float m = -INFINITY, lsum = 0.f;
-  f32x4 o[8];
+  // Element offsets of this lane's operand reads: scores, k-steps of even and odd index (latent row n, chunk 4 k + g);
+  // values, output block j (latent rows 4 g + n / 4 (+ 16), dims 64 wave + 16 j + 4 (n % 4)).
+  const int kpos[2] = {n * kRunRow + 8 * (g ^ (n & 6)), n * kRunRow + 8 * ((4 + g) ^ (n & 6))};
+  int vpos[DB];
+#pragma unroll
+  for (int j = 0; j < DB; ++j) {
+    const int r = 4 * g + (n >> 2), chunk = 2 * DB * wave + 2 * j + ((n & 3) >> 1);
+    vpos[j] = r * kRunRow + 8 * (chunk ^ (r & 6)) + 4 * (n & 1);
+  }
+
+  u32x4 qb[18];  // Q^T operand: lane holds dims 32 k + 8 g .. + 7 of column n of block cb
+  int sees = 0;  // latents that column sees
+  float m[NB], lsum = 0.f;
+  f32x4 o[NB][DB];
   int issued = 0;
-  for (; issued < STAGES - 1 && !prod.done; ++issued) {
-    fill(prod, ring + issued * kDmaStageElems);
+  for (; loader && issued < kRunStages - 1 && !prod.done; ++issued) {
+    fill(prod, ring + issued * kRunElems);
     advance(prod);
   }
   for (int k = 0; !cons.done; ++k) {
-    dma_stage_barrier(issued - k - 1, wave);  // stage k has landed for every wave
+    // Stage k has landed for every wave (one that loads nothing meets the barrier).
+    const int ahead = issued - k - 1;
+    if (!loader) run_wait<63>();
+    else if (ahead <= 0) run_wait<0>();
+    else run_wait<kPer>();
     // Refill the slot read last iteration (every wave has passed the barrier, so its reads are done).
-    if (!prod.done) {
-      fill(prod, ring + (issued % STAGES) * kDmaStageElems);
+    if (loader && !prod.done) {
+      fill(prod, ring + (issued % kRunStages) * kRunElems);
       advance(prod);
       ++issued;
     }
-    const uint16_t* stage = ring + (k % STAGES) * kDmaStageElems;
+    const uint16_t* stage = ring + (k % kRunStages) * kRunElems;
     if (cons.t < 0) {
-      // Q^T operand of this wave's k-steps: lane holds dims 32 (s0 + i) + 8 g .. + 7 of head n.
-      const uint16_t* qs = stage + n * kMlaPitch + 32 * s0 + 8 * g;
+      if (wave < SW) {
+        const uint16_t* qs = stage + cb * 16 * kRunRow;
 #pragma unroll
-      for (int i = 0; i < 5; ++i)
-        if (i < ns) qb[i] = *reinterpret_cast<const u32x4*>(qs + 32 * i);
-      m = -INFINITY;
-      lsum = 0.f;
+        for (int s = 0; s < 18; ++s) qb[s] = *reinterpret_cast<const u32x4*>(qs + kpos[s & 1] + 64 * (s >> 1));
+        const int col = min((cons.tile * NB + cb) * 16 + n, columns - 1);
+        sees = cons.len - p.lq + col / p.heads + 1;
+        lsum = 0.f;
+      }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] = f32x4{0, 0, 0, 0};
+      for (int nb = 0; nb < NB; ++nb) {
+        m[nb] = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < DB; ++j) o[nb][j] = f32x4{0, 0, 0, 0};
+      }
       advance(cons);
       continue;
     }
-    const int t0 = cons.t * kDmaTile;
-    f32x4 sc = {0, 0, 0, 0};  // latents t0 + 4 g + r of head n
-    const uint16_t* arow = stage + n * kMlaPitch + 32 * s0 + 8 * g;
+    f32x4 sc = {0, 0, 0, 0};  // latents t0 + 16 lb + 4 g + r of column n
+    float mc = 0.f, psum = 0.f;
+    const int t0 = cons.t * kRunTile;
+    // Probabilities of the wave's scores under the column's max, to LDS.
+    auto put_probabilities = [&] {
+      float pr[4];
 #pragma unroll
-    for (int i = 0; i < 5; ++i)
-      if (i < ns) sc = E::mfma16x16x32(*reinterpret_cast<const u32x4*>(arow + 32 * i), qb[i], sc);
-    // Sum the four partials, in the same order in every wave (every wave then holds the same S^T). The barrier
-    // waits for LDS only: the stage loads in flight are not waited for.
-    spart[wave][lane] = sc;
+      for (int r = 0; r < 4; ++r) pr[r] = fast_exp2(fmaf(sc[r], c, -mc));
+      psum = (pr[0] + pr[1]) + (pr[2] + pr[3]);
+      s_p[cb][lb][lane] = u32x2{E::pack(pr[0], pr[1]), E::pack(pr[2], pr[3])};
+    };
+    auto own_max = [&] {
+      float x = m[0];
+#pragma unroll
+      for (int nb = 1; nb < NB; ++nb) x = cb == nb ? m[nb] : x;
+      return x;
+    };
+    // The stage's V^T operands wait for nobody; a wave with scores reads them after those.
+    u32x4 va[DB];
+    auto read_values = [&] {
+#pragma unroll
+      for (int j = 0; j < DB; ++j) {
+        const u32x2 lo = lds_read_tr16(stage + vpos[j]), hi = lds_read_tr16(stage + 16 * kRunRow + vpos[j]);
+        va[j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+    };
+    if (wave >= SW) read_values();
+    if (wave < SW) {
+      const uint16_t* rows = stage + lb * 16 * kRunRow;
+      f32x4 sd = {0, 0, 0, 0};  // two chains
+#pragma unroll
+      for (int s = 0; s < 18; s += 2) {
+        sc = E::mfma16x16x32(*reinterpret_cast<const u32x4*>(rows + kpos[0] + 32 * s), qb[s], sc);
+        sd = E::mfma16x16x32(*reinterpret_cast<const u32x4*>(rows + kpos[1] + 32 * s), qb[s + 1], sd);
+      }
+      // Six operands read ahead of the MFMAs (left alone, the compiler waits for each read in turn).
+      __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+#pragma unroll
+      for (int s = 0; s < 6; ++s) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
+      sc += sd;
+      if (t0 + kRunTile > cons.lk - (p.lq - 1)) {  // else every column sees the stage
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sc[r] = t0 + 16 * lb + 4 * g + r < sees ? sc[r] : -INFINITY;
+      }
+      float mx = vmax(vmax(sc[0], sc[1]), vmax(sc[2], sc[3]));
+      mx = xor32_max(xor16_max(mx));
+      const float mo = own_max();
+      const bool grow = mx > mo && (mo == -INFINITY || (mx - mo) * c > kRescaleSlack);
+      mc = mo == -INFINITY ? 0.f : mo * c;
+      if (g == 0) s_max[cb][lb][n] = mx;
+      if (lane == 0) s_grow[wave] = 0;
+      if (__any(grow)) {
+        if (lane == 0) s_grow[wave] = 1;
+      } else {
+        put_probabilities();
+      }
+      read_values();
+    }
+    // LDS only: the stage loads in flight are not waited for.
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    sc = (spart[0][lane] + spart[1][lane]) + (spart[2][lane] + spart[3][lane]);
-    if (t0 + kDmaTile > cons.lk) {
+    int grown = 0;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sc[r] = t0 + 4 * g + r < cons.lk ? sc[r] : -INFINITY;
+    for (int w = 0; w < SW; ++w) grown |= s_grow[w];
+    u32x4 pb[NB];
+    auto get_probabilities = [&] {
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const u32x2 lo = s_p[nb][0][lane], hi = s_p[nb][1][lane];
+        pb[nb] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      }
+    };
+    get_probabilities();
+    if (__builtin_amdgcn_readfirstlane(grown)) {  // the same in every wave
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const float mn = vmax(m[nb], vmax(s_max[nb][0][n], s_max[nb][1][n]));
+        const float alpha = m[nb] == -INFINITY ? 0.f : fast_exp2((m[nb] - mn) * c);
+        m[nb] = mn;
+        if (cb == nb) lsum *= alpha;
+#pragma unroll
+        for (int j = 0; j < DB; ++j) o[nb][j] *= alpha;
+      }
+      if (wave < SW) {
+        const float mo = own_max();
+        mc = mo == -INFINITY ? 0.f : mo * c;  // a column that has seen no latent
+        put_probabilities();
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      get_probabilities();
     }
-    float mx = vmax(vmax(sc[0], sc[1]), vmax(sc[2], sc[3]));
-    mx = xor32_max(xor16_max(mx));
-    if (__any(mx > m && (m == -INFINITY || (mx - m) * c > kRescaleSlack))) {
-      const float mn = vmax(m, mx);
-      const float alpha = m == -INFINITY ? 0.f : fast_exp2((m - mn) * c);
-      m = mn;
-      lsum *= alpha;
+    lsum += psum;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) o[j] *= alpha;
-    }
-    const float mc = m * c;
-    float pr[4];
+    for (int j = 0; j < DB; ++j)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) pr[r] = fast_exp2(fmaf(sc[r], c, -mc));
-    lsum += (pr[0] + pr[1]) + (pr[2] + pr[3]);
-    const u32x2 pb = {E::pack(pr[0], pr[1]), E::pack(pr[2], pr[3])};
-    const uint16_t* v = stage + (4 * g + (n >> 2)) * kMlaPitch + 128 * wave + 4 * (n & 3);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = E::mfma16x16x16(lds_read_tr16(v + 16 * j), pb, o[j]);
+      for (int nb = 0; nb < NB; ++nb) o[nb][j] = E::mfma16x16x32(va[j], pb[nb], o[nb][j]);
 
     if (cons.t + 1 == cons.tu || cons.pu + cons.t + 1 == end) {  // the unit's last stage in this run
-      const float l = xor32_sum(xor16_sum(lsum));
-      const int tq = cons.tq, head = cons.ht * 16 + n;
-      const float inv = 1.f / l;  // l > 0: each of the run's stages of the unit holds a latent in range
-      if (head < p.heads) {
-        if (cons.pu >= start && cons.pu + cons.tu <= end) {
-          char* dst = p.out + tq * p.o_st + (int64_t)head * p.o_sh;
+      const bool whole = cons.pu >= start && cons.pu + cons.tu <= end;
+      if (wave < SW) {
+        const float l = xor32_sum(xor16_sum(lsum));
+        if (g == 0) s_sum[cb][lb][n] = l;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int d = 128 * wave + 16 * j + 4 * g;
-            const u32x2 val = {E::pack(o[j][0] * inv, o[j][1] * inv), E::pack(o[j][2] * inv, o[j][3] * inv)};
+      for (int nb = 0; nb < NB; ++nb) {
+        const int col = (cons.tile * NB + nb) * 16 + n;
+        if (col >= columns) continue;
+        const float l = s_sum[nb][0][n] + s_sum[nb][1][n];
+        const float inv = l > 0.f || l != l ? 1.f / l : 0.f;  // 0: an earlier query sees none of the run's latents
+        if (whole) {
+          const int qj = col / p.heads;
+          char* dst = p.out + (int64_t)(cons.row * p.lq + qj) * p.o_st + (int64_t)(col - qj * p.heads) * p.o_sh;
+#pragma unroll
+          for (int j = 0; j < DB; ++j) {
+            const int d = 16 * DB * wave + 16 * j + 4 * g;
+            const u32x2 val = {E::pack(o[nb][j][0] * inv, o[nb][j][1] * inv),
+                               E::pack(o[nb][j][2] * inv, o[nb][j][3] * inv)};
             *reinterpret_cast<u32x2*>(dst + d * 2) = val;
           }
         } else {
-          const int slot = (blockIdx.x * 2 + (cons.pu <= start ? 0 : 1)) * 16 + n;
+          const int slot = (blockIdx.x * 2 + (cons.pu <= start ? 0 : 1)) * 16 * NB + 16 * nb + n;
           float* dst = p.part_o + (int64_t)slot * kVDim;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int d = 128 * wave + 16 * j + 4 * g;
-            *reinterpret_cast<f32x4*>(dst + d) = o[j] * inv;
+          for (int j = 0; j < DB; ++j) {
+            const int d = 16 * DB * wave + 16 * j + 4 * g;
+            *reinterpret_cast<f32x4*>(dst + d) = o[nb][j] * inv;
           }
-          if (wave == 0 && g == 0) p.part_lse[slot] = m * c + fast_log2(l);
+          if (wave == 0 && g == 0) p.part_lse[slot] = l > 0.f || l != l ? m[nb] * c + fast_log2(l) : -INFINITY;
         }
       }
     }
@@ -526,13 +667,15 @@ __global__ __launch_bounds__(256) void mla_run_kernel(MlaParams p) {
 }
 
 // Finish units cut by run boundaries (log-sum-exp over the runs that touched them) and zero the output of units
-// that see no latents; units finished in place are left alone. Block (unit, head of its tile), 64 threads.
-template <typename T>
-__global__ __launch_bounds__(64) void mla_run_merge_kernel(MlaParams p) {
+// that see no latents; units finished in place are left alone. Block (unit, four columns of its tile), one wave each.
+template <typename T, int NB>
+__global__ __launch_bounds__(256) void mla_run_merge_kernel(MlaParams p) {
   using E = Elem<T>;
-  const int u = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
-  const int tq = u / p.htiles, head = (u - tq * p.htiles) * 16 + h;
-  if (head >= p.heads) return;
+  const int u = blockIdx.x, lane = threadIdx.x & 63;
+  const int h = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = u / p.tiles, col = (u - row * p.tiles) * 16 * NB + h;
+  if (col >= p.lq * p.heads) return;
+  const int qj = col / p.heads, tq = row * p.lq + qj, head = col - qj * p.heads;
   const int pu = p.prefix[u], tu = p.prefix[u + 1] - pu, per = p.prefix[p.units + 1];
   constexpr int PER = kVDim / 64;
   float o[PER];
@@ -543,7 +686,7 @@ __global__ __launch_bounds__(64) void mla_run_merge_kernel(MlaParams p) {
     if (b0 == b1) return;
     // The runs' partials, kRunMergeBatch at a time with every load of a batch issued before the first is used;
     // the max and the sums carry from batch to batch.
-    constexpr int kRunMergeBatch = 4;
+    constexpr int kRunMergeBatch = 8;
     float m = -INFINITY, den = 0.f;
     for (int c0 = b0; c0 <= b1; c0 += kRunMergeBatch) {
       float ls[kRunMergeBatch];
@@ -555,7 +698,7 @@ __global__ __launch_bounds__(64) void mla_run_merge_kernel(MlaParams p) {
 #pragma unroll
         for (int e = 0; e < PER / 4; ++e) x[i][e] = f32x4{0, 0, 0, 0};
         if (b <= b1) {  // wave-uniform
-          const int slot = (b * 2 + (b == b0 && pu != b0 * per ? 1 : 0)) * 16 + h;
+          const int slot = (b * 2 + (b == b0 && pu != b0 * per ? 1 : 0)) * 16 * NB + h;
           ls[i] = p.part_lse[slot];
           const f32x4* src = reinterpret_cast<const f32x4*>(p.part_o + (int64_t)slot * kVDim + lane * PER);
 #pragma unroll
@@ -631,6 +774,7 @@ __global__ __launch_bounds__(64) void mla_merge_kernel(MlaParams p) {
 struct MlaShape {
   int32_t split, max_splits;  // split schedule
   int32_t runs, units;        // run schedule: workgroups, units
+  int32_t nb, tiles;          // and 16-column blocks per unit, units per row
   size_t lse_off, o_off, prefix_off, bytes;
 };
 
@@ -654,24 +798,35 @@ static MlaShape mla_shape(int32_t rows, int32_t lq, int32_t heads, int32_t max_k
   s.split = (int32_t)split;
   s.max_splits = (int32_t)((keys + split - 1) / split);
   const size_t parts = s.max_splits > 1 ? (size_t)rows * lq * heads * s.max_splits : 0;
-  // Run schedule: two workgroups per CU, fewer when the stages cannot fill runs of kRunMin.
-  const int64_t stages = units * ((keys + kDmaTile - 1) / kDmaTile);
-  s.units = (int32_t)std::min<int64_t>(units, INT32_MAX);
+  // Run schedule: one workgroup per CU, fewer when the stages cannot fill runs of kRunMin.
+  const int64_t columns = (int64_t)lq * heads;
+  s.nb = columns <= 16 ? 1 : 2;
+  const int64_t tiles = (columns + 16 * s.nb - 1) / (16 * s.nb);
+  const int64_t run_units = rows * tiles;
+  const int64_t stages = run_units * ((keys + kRunTile - 1) / kRunTile);
+  s.tiles = (int32_t)std::min<int64_t>(tiles, INT32_MAX);
+  s.units = (int32_t)std::min<int64_t>(run_units, INT32_MAX);
   s.runs = (int32_t)std::max<int64_t>(
       1, std::min<int64_t>(kRunsPerCU * device_cus(), (stages + kRunMin - 1) / kRunMin));
-  const size_t run_parts = (size_t)s.runs * 2 * 16;
+  const size_t run_parts = (size_t)s.runs * 2 * 16 * s.nb;
   const size_t nparts = std::max(parts, run_parts);
   s.lse_off = 0;
   s.o_off = (nparts * sizeof(float) + 255) / 256 * 256;
   s.prefix_off = s.o_off + nparts * kVDim * sizeof(float);
-  s.bytes = s.prefix_off + (size_t)(units + 2) * sizeof(int32_t);
+  s.bytes = s.prefix_off + (size_t)(run_units + 2) * sizeof(int32_t);
   return s;
 }
 
-template <typename T>
+template <typename T, int NB>
 static void launch_runs(const MlaParams& p, int runs, hipStream_t st) {
-  hipLaunchKernelGGL((mla_run_kernel<T, kRunStages>), dim3(runs), dim3(256), 0, st, p);
-  hipLaunchKernelGGL(mla_run_merge_kernel<T>, dim3(p.units, 16), dim3(64), 0, st, p);
+  hipLaunchKernelGGL((mla_run_kernel<T, NB>), dim3(runs), dim3(64 * kRunWaves), 0, st, p);
+  hipLaunchKernelGGL((mla_run_merge_kernel<T, NB>), dim3(p.units, 4 * NB), dim3(256), 0, st, p);
+}
+
+template <typename T>
+static void launch_runs(const MlaParams& p, const MlaShape& s, hipStream_t st) {
+  if (s.nb == 1) launch_runs<T, 1>(p, s.runs, st);
+  else launch_runs<T, 2>(p, s.runs, st);
 }
 
 }  // namespace lv
@@ -746,13 +901,14 @@ extern "C" int lv_mla_decode(const void* q, int64_t q_stride_t, int64_t q_stride
   const int64_t stage_bound = (int64_t)s.units * (((int64_t)std::max(max_seqlen_k, 1) + kDmaTile - 1) / kDmaTile);
   if (one_page && s.units <= kRunMaxUnits && stage_bound < ((int64_t)1 << 30)) {
     p.units = s.units;
+    p.tiles = s.tiles;
     p.part_lse = reinterpret_cast<float*>(ws + s.lse_off);
     p.part_o = reinterpret_cast<float*>(ws + s.o_off);
     p.prefix = reinterpret_cast<int32_t*>(ws + s.prefix_off);
     if (dtype == LV_DTYPE_BF16)
-      launch_runs<BF16>(p, s.runs, st);
+      launch_runs<BF16>(p, s, st);
     else
-      launch_runs<F16>(p, s.runs, st);
+      launch_runs<F16>(p, s, st);
     LV_LAUNCH_CHECK("mla_run_kernel");
     return LV_OK;
   }

@@ -158,3 +158,18 @@ def test_mla_decode_replays_in_a_graph(cuda):
         eager = b.mla_decode(q, cache, VDIM, ctx)
         torch.cuda.synchronize()
         torch.testing.assert_close(out, eager, atol=0, rtol=0)
+
+
+@pytest.mark.parametrize("heads, queries", [(16, 1), (17, 1), (32, 1), (16, 2), (11, 3), (16, 3)])
+@pytest.mark.parametrize("bs", [16, 64])
+def test_columns_and_stages_at_their_edges(cuda, bs, heads, queries):
+    """Columns ((query, head) pairs) that fill one or two 16-column blocks, one more and a second unit; rows of as many
+    latents as queries, of a stage (32) and its neighbours, a long row cut by run boundaries, and enough short rows that
+    a run holds several units."""
+    lens = [queries, 31, 32, 33, 5000, 64 + queries] + [40 + i for i in range(30)]
+    need = [-(-n // bs) for n in lens]
+    width, at, tables = max(need), 0, []
+    for k in need:
+        tables.append(list(range(at, at + k)) + [-1] * (width - k))
+        at += k
+    check_mla(cuda, torch.bfloat16, bs, lens, tables, queries=queries, heads=heads, seed=heads)
