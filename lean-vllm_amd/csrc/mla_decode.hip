@@ -503,11 +503,16 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
     else if (ahead <= 0) run_wait<0>();
     else run_wait<kPer>();
     // Refill the slot read last iteration (every wave has passed the barrier, so its reads are done).
-    if (loader && !prod.done) {
+    auto refill = [&] {
+      if (!loader || prod.done) return;
       fill(prod, ring + (issued % kRunStages) * kRunElems);
       advance(prod);
       ++issued;
-    }
+    };
+    // With the value reads below before it, 128 rows of 16 heads measured 218.5 -> 217.5 us; after it, two column blocks
+    // 77.8 -> 74.8.
+    constexpr bool kValuesFirst = NB == 1;
+    if (cons.t < 0 || !kValuesFirst) refill();
     const uint16_t* stage = ring + (k % kRunStages) * kRunElems;
     if (cons.t < 0) {
       if (wave < SW) {
@@ -553,7 +558,10 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
         va[j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
       }
     };
-    if (wave >= SW) read_values();
+    if (wave >= SW) {
+      read_values();
+      if (kValuesFirst) refill();
+    }
     if (wave < SW) {
       const uint16_t* rows = stage + lb * 16 * kRunRow;
       f32x4 sd = {0, 0, 0, 0};  // two chains
