@@ -52,7 +52,7 @@ struct MlaParams {
   float* part_lse;  // split schedule: [rows * lq][heads][max_splits]; runs: [runs][2][16 NB]; log2 domain
   int32_t units;    // runs: (row, tile of 16 NB (query, head) columns) units
   int32_t tiles;    // runs: units per row
-  int32_t* prefix;  // runs: [units + 2] stage prefix over units, then the stage total and the run length
+  int32_t* prefix;  // runs: [units + 2] prefix of places over units, then their total and the run length
 };
 
 // ---------------------------------------------------------------------------------------------------------
@@ -253,7 +253,8 @@ __global__ __launch_bounds__(256) void mla_decode_dma_kernel(MlaParams p) {
 //
 // A row's columns are its (query j, head) pairs, c = j * heads + head. Unit u = (row, tile of 16 NB columns), u = row *
 // tiles + tile, needs T_u = ceil(L_u / 32) stages of 32 latents (L_u: the latents its last query sees; a column of an
-// earlier query masks its last ones). Laid end to end (prefix P_u) the units' stages are cut into equal runs, one per
+// earlier query masks its last ones), and kRunEnter more places ahead of them for its queries and its output, which cost
+// a run about as much. Laid end to end (prefix P_u) the units' stages are cut into equal runs, one per
 // workgroup of a grid that fills the GPU once; every workgroup streams its run through an LDS ring, each unit it enters
 // preceded by a stage holding that unit's query rows. A unit that lies wholly inside one run is finished in place. A unit cut by run boundaries leaves (o / l, log2 l + m) per column in slot 0 (the run's
 // first unit) or slot 1 (its last unit) of every run it touches, and mla_run_merge_kernel combines them; that kernel also
@@ -273,11 +274,13 @@ __global__ __launch_bounds__(256) void mla_decode_dma_kernel(MlaParams p) {
 // Bound by HBM up to 32 columns (a build without the scores and P.V streams 128 rows of 1024-16384 latents in 201 us,
 // 6.55 TB/s; the scores' serial chain through LDS and the two barriers are what is left). Against the schedule before,
 // two workgroups of 4 waves per CU with a 16-latent stage each, every query and every 16 heads a unit of their own:
-// 128 rows, 16 heads 218 us (217), 32 heads 229 (426), 64 heads 454 (850), 128 heads 890 (1670); two layers of 20 rows,
-// 1024-8192 latents, 16 heads, 2 queries 76 us (108), 3 queries 104 (138), 128 heads 171 (298); 4 rows 57 (70).
+// 128 rows, 16 heads 216 us (215.4), 32 heads 229 (426), 64 heads 454 (850), 128 heads 890 (1670); two layers of 20 rows,
+// 1024-8192 latents, 16 heads, 2 queries 73 us (108), 3 queries 104 (138), 128 heads 171 (298); 4 rows 57 (70).
 
 constexpr int kRunTile = 32;         // latents per stage
-constexpr int kRunMin = 2;           // stages per run at least
+constexpr int kRunEnter = 3;         // places of a unit's start (0 / 1 / 2 / 3: 128 rows 217.5 / 216.4 / 216.9 / 216.0 us, 60 rows
+                                     // 136.6 / 135.1 / 134.4 / 133.2)
+constexpr int kRunMin = 4;           // places per run at least (past a unit's start)
 constexpr int kRunStages = 3;        // ring depth (four stream no faster)
 constexpr int kRunWaves = 8;
 constexpr int kRunsPerCU = 1;        // run workgroups per CU
@@ -300,15 +303,18 @@ __device__ __forceinline__ int unit_latents(const MlaParams& p, int tile, int le
   return len - p.lq + last / p.heads + 1;
 }
 
+// Places of a unit of lk latents in the runs; none without latents.
+__device__ __forceinline__ int stage_places(int lk) {
+  return lk > 0 ? (lk + kRunTile - 1) / kRunTile + kRunEnter : 0;
+}
 template <int NB>
-__device__ __forceinline__ int unit_stages(const MlaParams& p, int u) {
+__device__ __forceinline__ int unit_places(const MlaParams& p, int u) {
   const int row = u / p.tiles;
-  const int lk = unit_latents<NB>(p, u - row * p.tiles, p.lens[row]);
-  return lk > 0 ? (lk + kRunTile - 1) / kRunTile : 0;
+  return stage_places(unit_latents<NB>(p, u - row * p.tiles, p.lens[row]));
 }
 
-// Position in a run's stage sequence: unit u (prefix pu, tu stages, lk latents), next tile t (-1: its queries). The
-// unit's row and column tile and its block-table row are kept here, so a stage's loads need no division.
+// Position in a run's stage sequence: unit u (first stage at place pu, tu stages, lk latents), next tile t (-1: its
+// queries). The unit's row and column tile and its block-table row are kept here, so a stage's loads need no division.
 struct RunCursor {
   int u, pu, tu, lk, t;
   int row, len, tile, pg[2];
@@ -342,14 +348,14 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
   const int lb = wave % LB, cb = wave / LB;  // the scores this wave computes (wave < SW)
   const int columns = p.lq * p.heads;
 
-  // Stage counts over units; thread tid sums units [ulo, uhi). Exclusive scan of those sums across the block.
+  // Places over units; thread tid sums units [ulo, uhi). Exclusive scan of those sums across the block.
   const int per_thread = (p.units + 64 * W - 1) / (64 * W);
   const int ulo = min(tid * per_thread, p.units), uhi = min(ulo + per_thread, p.units);
   int local = 0, len0 = 0;  // len0: latents of unit ulo's row
   for (int u = ulo; u < uhi; ++u) {
     const int row = u / p.tiles, len = p.lens[row];
     const int lk = unit_latents<NB>(p, u - row * p.tiles, len);
-    local += lk > 0 ? (lk + kRunTile - 1) / kRunTile : 0;
+    local += stage_places(lk);
     len0 = u == ulo ? len : len0;
   }
   const int x = wave_incl_scan(local);
@@ -368,7 +374,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
     int run = excl;
     for (int u = ulo; u < uhi; ++u) {
       p.prefix[u] = run;
-      run += unit_stages<NB>(p, u);
+      run += unit_places<NB>(p, u);
     }
     if (tid == 0) {
       p.prefix[p.units] = total;
@@ -381,7 +387,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
   if (local > 0 && excl <= start && start < excl + local) {
     int u = ulo, acc = excl;
     if (per_thread > 1)
-      for (int tu = unit_stages<NB>(p, u); acc + tu <= start; tu = unit_stages<NB>(p, u)) {
+      for (int tu = unit_places<NB>(p, u); acc + tu <= start; tu = unit_places<NB>(p, u)) {
         acc += tu;
         ++u;
       }
@@ -401,7 +407,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       if (r.lk > 0) break;
     }
     r.u = u;
-    r.pu = pu;
+    r.pu = pu + kRunEnter;
     r.tu = (r.lk + kRunTile - 1) / kRunTile;
     r.t = -1;
     r.table = p.tables + (int64_t)r.row * p.t_stride;
@@ -414,7 +420,8 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
     } else if (r.pu + r.t + 1 == end) {
       r.done = true;
     } else if (r.t + 1 == r.tu) {
-      enter(r, r.u + 1, r.pu + r.tu);
+      if (r.pu + r.tu + kRunEnter >= end) r.done = true;  // the next unit's stages lie past the run
+      else enter(r, r.u + 1, r.pu + r.tu);
     } else {
       ++r.t;
     }
@@ -659,7 +666,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
             *reinterpret_cast<u32x2*>(dst + d * 2) = val;
           }
         } else {
-          const int slot = (blockIdx.x * 2 + (cons.pu <= start ? 0 : 1)) * 16 * NB + 16 * nb + n;
+          const int slot = (blockIdx.x * 2 + (cons.pu - kRunEnter <= start ? 0 : 1)) * 16 * NB + 16 * nb + n;
           float* dst = p.part_o + (int64_t)slot * kVDim;
 #pragma unroll
           for (int j = 0; j < DB; ++j) {
@@ -684,7 +691,7 @@ __global__ __launch_bounds__(256) void mla_run_merge_kernel(MlaParams p) {
   const int row = u / p.tiles, col = (u - row * p.tiles) * 16 * NB + h;
   if (col >= p.lq * p.heads) return;
   const int qj = col / p.heads, tq = row * p.lq + qj, head = col - qj * p.heads;
-  const int pu = p.prefix[u], tu = p.prefix[u + 1] - pu, per = p.prefix[p.units + 1];
+  const int at = p.prefix[u], pu = at + kRunEnter, tu = p.prefix[u + 1] - pu, per = p.prefix[p.units + 1];
   constexpr int PER = kVDim / 64;
   float o[PER];
 #pragma unroll
@@ -706,7 +713,7 @@ __global__ __launch_bounds__(256) void mla_run_merge_kernel(MlaParams p) {
 #pragma unroll
         for (int e = 0; e < PER / 4; ++e) x[i][e] = f32x4{0, 0, 0, 0};
         if (b <= b1) {  // wave-uniform
-          const int slot = (b * 2 + (b == b0 && pu != b0 * per ? 1 : 0)) * 16 * NB + h;
+          const int slot = (b * 2 + (b == b0 && at > b0 * per ? 1 : 0)) * 16 * NB + h;
           ls[i] = p.part_lse[slot];
           const f32x4* src = reinterpret_cast<const f32x4*>(p.part_o + (int64_t)slot * kVDim + lane * PER);
 #pragma unroll
@@ -811,7 +818,7 @@ static MlaShape mla_shape(int32_t rows, int32_t lq, int32_t heads, int32_t max_k
   s.nb = columns <= 16 ? 1 : 2;
   const int64_t tiles = (columns + 16 * s.nb - 1) / (16 * s.nb);
   const int64_t run_units = rows * tiles;
-  const int64_t stages = run_units * ((keys + kRunTile - 1) / kRunTile);
+  const int64_t stages = run_units * ((keys + kRunTile - 1) / kRunTile + kRunEnter);
   s.tiles = (int32_t)std::min<int64_t>(tiles, INT32_MAX);
   s.units = (int32_t)std::min<int64_t>(run_units, INT32_MAX);
   s.runs = (int32_t)std::max<int64_t>(
