@@ -862,7 +862,7 @@ static void launch_decode(const AttnParams& p, const Route& r, hipStream_t strea
 
 // A step's kernels after the plan. An overlapped mixed step forks the decode items onto the device's second stream
 // and joins it back into `stream` with events; if the second stream cannot be set up, or the fork's record or wait
-// fails before anything is launched, the step runs serially instead (the same results). A failure after the decode
+// fails before anything is launched, the step runs serially instead (the same results). A failure after the prompt
 // launch leaves the two streams unordered and is returned as LV_EHIP. With `info` set nothing is launched: the
 // route is reported instead.
 template <typename T, int D, int GS, int TP, int HP>
@@ -880,18 +880,20 @@ static int launch(const AttnParams& p, const Shape& s, const StepKind& k, hipStr
     SideStream* side = r.two_streams ? side_stream() : nullptr;
     bool forked = false;
     if (side) {
-      // Decode items go to the second stream first, then the prompt items to the caller's stream: the prompt
-      // workgroups (one per CU) are dispatched as soon as the plan ends, the decode workgroups fill the rest.
+      // The prompt items go first, to the caller's stream, then the decode items to the second one: the prompt
+      // workgroups (one per CU) are dispatched as soon as the plan ends, the decode workgroups fill the rest. On an idle
+      // GPU decode workgroups launched first fill every CU, and the prompt items start when they end: the Qwen3-8B mixed step
+      // alone 4.62 ms, so 2.95; among others 2.97 and 2.93.
       std::lock_guard<std::mutex> g(side->lock);
       if (hipEventRecord(side->fork, stream) == hipSuccess &&
           hipStreamWaitEvent(side->stream, side->fork, 0) == hipSuccess) {
         forked = true;
-        launch_decode<T, D, GS, HP>(p, r, side->stream);
-        LV_LAUNCH_CHECK("decode kernel beside the prompt tiles");
-        LV_HIP_CHECK(hipEventRecord(side->join, side->stream));
         constexpr int pad = std::max(0, kOverlapLds - std::max(1, kRingOf<TP>) * PromptSmem<D, D, (TP > 1)>::kBytes);
         hipLaunchKernelGGL((prompt_overlap_kernel<T, D, TP>), dim3(r.prompt_grid), dim3(256), pad, stream, p);
         LV_LAUNCH_CHECK("prompt_overlap_kernel");
+        launch_decode<T, D, GS, HP>(p, r, side->stream);
+        LV_LAUNCH_CHECK("decode kernel beside the prompt tiles");
+        LV_HIP_CHECK(hipEventRecord(side->join, side->stream));
         LV_HIP_CHECK(hipStreamWaitEvent(stream, side->join, 0));
       } else {
         (void)hipGetLastError();  // the failed record or wait: fall back to the serial schedule
