@@ -187,7 +187,8 @@ int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t
  * into a captured graph. Every call
  * on one GPU shares that GPU's array, which keeps the last call's contents: calls that overlap on one GPU (two
  * streams, two host threads, or a graph replay beside an eager call) race. Results equal lv_paged_attention's for
- * the same arguments. Set-up: the first call on a device resolves the array's address there and creates the
+ * the same arguments, but for the rounding of a step of few prompt tiles, whose keys lv_paged_attention splits over
+ * workgroups where its workspace has room for their partials. Set-up: the first call on a device resolves the array's address there and creates the
  * device's second stream and its two fork/join events (which lv_paged_attention creates at its first overlapped
  * step); no device memory is allocated, and later calls create nothing. A caller that captures graphs makes one
  * call on each device before capturing. */

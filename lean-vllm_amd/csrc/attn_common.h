@@ -48,6 +48,11 @@ struct AttnParams {
   // Split rows (listed steps only): per (row, item head group), the count of its splits that have written their
   // partials (zeroed by the plan kernel); the last to arrive merges them and puts the count back to zero.
   int32_t* merge_count;
+  // Prompt items split over their keys (prompt_split_kernel): pieces per item, and per (item, kv head, piece) the
+  // normalised partial outputs [kPrefillRows][D] and log2-sum-exp2 [kPrefillRows] of its query rows.
+  int32_t pieces;
+  float* piece_o;
+  float* piece_lse;
   // Packed keys only: a row's context keys, seen unmasked before the row's own keys (prefill_item's CTX).
   const char* ctx_k;  // [Tc, Hkv, DQK]
   const char* ctx_v;  // [Tc, Hkv, DV]
@@ -113,12 +118,14 @@ __device__ __forceinline__ int swz(int r, int c) {
 // CTX (packed keys, RING > 0): the row's context keys (p.ctx_k / p.ctx_v, rows p.cu_ctx) come first, every one
 // visible to every query, then the row's own keys under the mask above -- one softmax over both, as the attention
 // over [context; own keys] with the mask aligned to the end.
+// SPLIT (RING > 0): the item's tiles are cut into p.pieces ranges; this call takes range `piece` and leaves its partial
+// in slot `slot`.
 // TP (paged keys, RING > 0): pages per 64-key tile -- 1 for pages of a multiple of 64 keys (one lookup per page,
 // kept across the page's tiles), 2 or 4 for pages of 32 or 16 keys (the tile's pages looked up at every fill, each
 // lane loading from its key's page).
 template <typename T, int DQK, int DV, bool PREFETCH = true, bool OPAQUE_TID = false, int RING = 0, int WAVES = 4,
-          bool CTX = false, int TP = 1>
-__device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, char* smem) {
+          bool CTX = false, int TP = 1, bool SPLIT = false>
+__device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, char* smem, int piece = 0, int slot = 0) {
   using E = Elem<T>;
   constexpr int KS = DQK / 32;  // MFMA k-steps over the q.k width
   constexpr int DB = DV / 16;   // 16-dim blocks of the output
@@ -174,7 +181,11 @@ __device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, c
     lc = p.cu_ctx[row + 1] - cbase;
   }
   const int nc = (lc + kPrefillKeys - 1) / kPrefillKeys;                  // context tiles
-  const int ntiles = nc + (kmax + kPrefillKeys - 1) / kPrefillKeys;       // all tiles of the item
+  const int all_tiles = nc + (kmax + kPrefillKeys - 1) / kPrefillKeys;    // all tiles of the item
+  static_assert(!SPLIT || (RING > 0 && !CTX && WAVES == 4), "split items stream paged keys");
+  const int per_piece = SPLIT ? (all_tiles + p.pieces - 1) / p.pieces : all_tiles;
+  const int tile0 = SPLIT ? min(piece * per_piece, all_tiles) : 0;
+  const int ntiles = SPLIT ? min(tile0 + per_piece, all_tiles) : all_tiles;  // this call's tiles: tile0 .. ntiles - 1
 
   float m[2], l[2];  // raw-score max (held or running) and row sums
   f32x4 o[2][DB];
@@ -452,9 +463,9 @@ __device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, c
     for (int nb = 0; nb < 2; ++nb)
 #pragma unroll
       for (int k = 0; k < KS; ++k) asm volatile("" ::"v"(qb[nb][k]));
-    int issued = 0;
-    for (; issued < RING - 1 && issued < ntiles; ++issued) fill(issued, ring + issued * kStageElems);
-    for (int it = 0; it < ntiles; ++it) {
+    int issued = tile0;
+    for (; issued < tile0 + RING - 1 && issued < ntiles; ++issued) fill(issued, ring + issued % RING * kStageElems);
+    for (int it = tile0; it < ntiles; ++it) {
       // This wave's loads of tile `it` have landed when only the later tiles' are outstanding; the barrier makes
       // every wave's visible and frees the slot read last iteration.
       const int ahead = issued - it - 1;
@@ -468,7 +479,7 @@ __device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, c
       const uint16_t* ks = ring + (it % RING) * kStageElems;
       const bool in_ctx = CTX && it < nc;  // a context tile: every query sees its keys < lc
       const int lcur[2] = {in_ctx ? lc : lim[0], in_ctx ? lc : lim[1]};
-      consume((in_ctx ? it : it - nc) * kPrefillKeys, lcur, ks, ks + kPrefillKeys * KROW, it == 0, running);
+      consume((in_ctx ? it : it - nc) * kPrefillKeys, lcur, ks, ks + kPrefillKeys * KROW, it == tile0, running);
     }
   } else {
     uint16_t* ks = reinterpret_cast<uint16_t*>(smem);  // [64 keys][KROW]
@@ -516,6 +527,13 @@ __device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, c
     const float lsum = xor32_sum(xor16_sum(l[nb]));
     if (!qvalid[nb]) continue;
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    if constexpr (SPLIT) {
+      const int64_t at = (int64_t)slot * kPrefillRows + wave * 32 + nb * 16 + n;
+      if (j4 == 0) p.piece_lse[at] = lsum > 0.f ? m[nb] * c + fast_log2(lsum) : -INFINITY;
+#pragma unroll
+      for (int b = 0; b < DB; ++b) *reinterpret_cast<f32x4*>(p.piece_o + at * DV + b * 16 + 4 * j4) = o[nb][b] * inv;
+      continue;
+    }
     char* dst = p.out + (int64_t)(q0 + qi[nb]) * p.o_st + head[nb] * p.o_sh;
 #pragma unroll
     for (int b = 0; b < DB; ++b) {

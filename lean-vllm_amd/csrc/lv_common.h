@@ -231,37 +231,49 @@ __device__ inline int wave_incl_scan(int x) {
   return x;
 }
 
-// Exclusive prefix sum of a[0, n) in LDS, in place, by a block of kScanThreads threads; a[n] receives the total.
-// wave_tot holds kScanThreads / 64 ints of LDS. Every thread of the block must call it, after a barrier that follows
-// the last write of a[] (a thread's chunk holds entries other threads wrote once n > kScanThreads). Each thread scans its
-// chunk, each wave its threads' chunk totals; every thread then sums the wave totals before its own (16 broadcast
-// LDS reads, issued together) instead of one thread scanning them in sequence between two more barriers.
+// Exclusive prefix sums of N arrays a[i][0, n) in LDS, in place, by a block of kScanThreads threads; a[i][n] receives the
+// total. wave_tot holds kScanThreads / 64 ints of LDS per array. Every thread of the block must call it, after a barrier
+// that follows the last write of the arrays (a thread's chunk holds entries other threads wrote once n > kScanThreads).
+// Each thread scans its chunk, each wave its threads' chunk totals; every thread then sums the wave totals before its own
+// (16 broadcast LDS reads, issued together) instead of one thread scanning them in sequence between two more barriers.
 constexpr int kScanThreads = 1024;
-__device__ inline void block_scan(int* a, int n, int* wave_tot) {
+template <int N>
+__device__ inline void block_scan(int* const (&a)[N], int n, int (&wave_tot)[N][kScanThreads / 64]) {
   const int tid = threadIdx.x;
   const int per = (n + kScanThreads - 1) / kScanThreads;
   const int lo = min(tid * per, n), hi = min(lo + per, n);
-  int local = 0;
-  for (int i = lo; i < hi; ++i) local += a[i];
   const int lane = tid & 63, wave = tid >> 6;
-  const int x = wave_incl_scan(local);  // inclusive scan of the chunk totals across the wave
-  if (lane == 63) wave_tot[wave] = x;
-  __syncthreads();
-  int before = 0, total = 0;
+  int before[N];  // inclusive scan of the chunk totals across the wave, less the thread's own
 #pragma unroll
-  for (int w = 0; w < kScanThreads / 64; ++w) {
-    const int v = wave_tot[w];
-    before += w < wave ? v : 0;
-    total += v;
+  for (int i = 0; i < N; ++i) {
+    int local = 0;
+    for (int j = lo; j < hi; ++j) local += a[i][j];
+    const int x = wave_incl_scan(local);
+    if (lane == 63) wave_tot[i][wave] = x;
+    before[i] = x - local;
   }
-  int run = before + x - local;  // exclusive prefix of this thread's chunk
-  for (int i = lo; i < hi; ++i) {
-    const int v = a[i];
-    a[i] = run;
-    run += v;
-  }
-  if (tid == 0) a[n] = total;
   __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    int run = before[i], total = 0;  // run: exclusive prefix of this thread's chunk
+#pragma unroll
+    for (int w = 0; w < kScanThreads / 64; ++w) {
+      const int v = wave_tot[i][w];
+      run += w < wave ? v : 0;
+      total += v;
+    }
+    for (int j = lo; j < hi; ++j) {
+      const int v = a[i][j];
+      a[i][j] = run;
+      run += v;
+    }
+    if (tid == 0) a[i][n] = total;
+  }
+  __syncthreads();
+}
+__device__ inline void block_scan(int* a, int n, int (&wave_tot)[1][kScanThreads / 64]) {
+  int* const one[1] = {a};
+  block_scan<1>(one, n, wave_tot);
 }
 
 constexpr float kLog2e = 1.4426950408889634f;

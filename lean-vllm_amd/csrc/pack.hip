@@ -27,7 +27,8 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
   __shared__ int cu_q[kPackMaxRows + 1];  // token offsets, batch order
   __shared__ int cu_s[kPackMaxRows + 1];  // slot_mapping offsets (rows with a block list only), batch order
   __shared__ int row_of[kPackMaxRows];    // scheduler row -> batch row (logits only)
-  __shared__ int wave_tot[kPackThreads / 64 + 1];
+  __shared__ int wave_tot[1][kPackThreads / 64];
+  __shared__ int wave_tot2[2][kPackThreads / 64];
   __shared__ int s_cached[kPackMaxRows];    // the per-row inputs, staged once: every later read is from LDS
   __shared__ int s_new[kPackMaxRows];
   __shared__ int s_ptr[kPackMaxRows + 1];
@@ -62,8 +63,8 @@ __global__ __launch_bounds__(kPackThreads) void pack_kernel(
     cu_s[r] = dense_slots || s_ptr[s + 1] > s_ptr[s] ? s_new[s] : 0;
   }
   __syncthreads();
-  block_scan(cu_q, rows, wave_tot);
-  block_scan(cu_s, rows, wave_tot);
+  int* const sums[2] = {cu_q, cu_s};
+  block_scan<2>(sums, rows, wave_tot2);
 
   // 3. Row-level outputs, from one workgroup (cu_seqlens_k last, once cu_q is free to reuse).
   if (blockIdx.x == 0) {

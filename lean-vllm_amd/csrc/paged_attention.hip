@@ -31,6 +31,8 @@ constexpr int kOverlapCusMaxPct = 75;  // at most this percent when the caller s
 constexpr int kDecodeWgs = 2;         // persistent decode workgroups per CU outside the overlap
 constexpr int kOverlapDecodeWgs = 3;  // persistent decode workgroups per CU beside a mixed step's prompt workgroups
                                       // (at most: pair items at D = 128 fit two)
+constexpr int kMaxPromptPieces = 8;   // workgroups a prompt item is split into at most
+constexpr int kPieceKeys = 1024;      // and keys per piece at least, of the longest row
 constexpr int kSplitTarget = 4096;    // decode items (x kv heads x query-head groups) a step with split rows aims for
 constexpr int kMaxRowSplits = 128;    // and splits per row on average at most
 constexpr int kMinSplit = 256;        // keys per decode item at least
@@ -419,6 +421,68 @@ __global__ __launch_bounds__(256, 2) void prompt_list_kernel(AttnParams p) {
   prefill_item<T, D, D, true, false, RING, 4, false, (TP > 0 ? TP : 1)>(p, it.x, -1 - it.y, kvh, smem);
 }
 
+// A few prompt items with long key ranges (a chunk late in a long prompt), each split over its keys into p.pieces
+// workgroups, and the merge of their partials: one thread per four dims of a query row.
+// MFMA-bound, as the unsplit items, but 128 of those leave half the CUs without one and every SIMD of the others with one
+// wave. 32/8 heads, d128, a chunk on a 24,576-token prefix: 512 tokens 505 -> 222 us (412 -> 940 TFLOP/s), 32 tokens
+// 494 -> 84, 1024 tokens 517 -> 417; on 16-token pages 618 -> 235; 256 tokens on 4096 97 -> 47. (Pieces of at least
+// kPieceKeys keys: 512 tokens on 2048 62 -> 53.) A step whose items come to three quarters of the GPU's workgroups stays
+// whole.
+template <typename T, int D, int TP>
+__global__ __launch_bounds__(256, 2) void prompt_split_kernel(AttnParams p) {
+  constexpr int RING = kRingOf<TP>;
+  __shared__ __attribute__((aligned(16))) char smem[RING * PromptSmem<D, D, (TP > 1)>::kBytes];
+  const int f = blockIdx.x / p.hkv, kvh = blockIdx.x - f * p.hkv;
+  const int bx = f / p.pieces, piece = f - bx * p.pieces;
+  if (bx >= p.n_items[kPlanPrompts]) return;
+  const int2 it = p.prompts[bx];
+  prefill_item<T, D, D, true, false, RING, 4, false, TP, true>(p, it.x, -1 - it.y, kvh, smem, piece,
+                                                               (bx * p.hkv + kvh) * p.pieces + piece);
+}
+
+template <typename T, int D>
+__global__ __launch_bounds__(256) void prompt_merge_kernel(AttnParams p) {
+  using E = Elem<T>;
+  constexpr int LPR = D / 4, RPB = 256 / LPR;  // threads per row, rows per workgroup
+  const int item = blockIdx.x / (kPrefillRows / RPB);
+  const int r = (blockIdx.x - item * (kPrefillRows / RPB)) * RPB + threadIdx.x / LPR, d0 = threadIdx.x % LPR * 4;
+  const int bx = item / p.hkv, kvh = item - bx * p.hkv;
+  if (bx >= p.n_items[kPlanPrompts]) return;
+  const int2 it = p.prompts[bx];
+  const int qp = kPrefillRows / p.group;
+  const int q0 = p.cu_q[it.x], lq = p.cu_q[it.x + 1] - q0;
+  const int pos = (-1 - it.y) * qp + r / p.group, head = kvh * p.group + r % p.group;
+  if (r >= qp * p.group || pos >= lq) return;
+  float ls[kMaxPromptPieces];
+  f32x4 x[kMaxPromptPieces];
+  float m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kMaxPromptPieces; ++i) {
+    ls[i] = -INFINITY;
+    x[i] = f32x4{0, 0, 0, 0};
+    if (i < p.pieces) {
+      const int64_t at = ((int64_t)item * p.pieces + i) * kPrefillRows + r;
+      ls[i] = p.piece_lse[at];
+      x[i] = *reinterpret_cast<const f32x4*>(p.piece_o + at * D + d0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kMaxPromptPieces; ++i) m = fmaxf(m, ls[i]);
+  float den = 0.f;
+  f32x4 o = {0, 0, 0, 0};
+  if (m != -INFINITY) {
+#pragma unroll
+    for (int i = 0; i < kMaxPromptPieces; ++i) {
+      const float w = fast_exp2(ls[i] - m);
+      den += w;
+      o += w * x[i];
+    }
+    o *= 1.f / den;
+  }
+  *reinterpret_cast<u32x2*>(p.out + (int64_t)(q0 + pos) * p.o_st + (int64_t)head * p.o_sh + d0 * 2) =
+      u32x2{E::pack(o[0], o[1]), E::pack(o[2], o[3])};
+}
+
 // Prompt items of a mixed step, run at the same time as its decode items: one workgroup per CU, each walking the
 // prompt items blockIdx.x, + gridDim.x, ... in list order. Its LDS request (padded at launch, so the compiler still
 // budgets registers for 2 waves per SIMD) leaves room for no second one, and the decode workgroups take the CU's
@@ -517,7 +581,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   __shared__ int full[kPlanMaxRows + 1];
   __shared__ int slots[kPlanMaxRows + 1];
   __shared__ int bucket[kLenBuckets + 1];
-  __shared__ int wave_tot[kScanThreads / 64 + 1];
+  __shared__ int wave_tot[3][kScanThreads / 64];
   __shared__ int64_t wave_keys[kScanThreads / 64];
   __shared__ int wave_max[kScanThreads / 64];
   const int tid = threadIdx.x;
@@ -565,7 +629,8 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
       slots[r] = n > 1 ? n * lq : 0;
     }
     __syncthreads();
-    block_scan(slots, rows, wave_tot);
+    int* const sums[3] = {pre, full, slots};  // one pass over all: the kernel is its barriers
+    block_scan<3>(sums, rows, wave_tot);
     if (slots[rows] <= max_slots || split >= longest) break;
     split = split < (1 << 29) ? 2 * split : INT32_MAX;
     __syncthreads();  // every thread has read slots[rows]
@@ -587,8 +652,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     bucket[tid] = x - v;
     if (tid == kLenBuckets - 1) bucket[kLenBuckets] = x;
   }
-  block_scan(pre, rows, wave_tot);  // its barriers also publish the bucket offsets
-  block_scan(full, rows, wave_tot);
+  __syncthreads();
   const int npre = pre[rows], nfull = full[rows], npart = bucket[kLenBuckets];
   // Full splits, one thread each (a few long rows hold hundreds: a thread per row would write them one by one).
   for (int i = tid; i < nfull; i += kScanThreads) {
@@ -627,8 +691,9 @@ struct Shape {
   int32_t pieces;      // the plan cuts the decode rows' keys into this many (0: rows are not split)
   int32_t max_splits;  // the most items one row may be split into
   int32_t slots;       // split rows' partial slots
+  int32_t prompt_pieces;  // workgroups per prompt item outside the overlap
   int64_t merges;      // split rows' merge counters (rows x kv heads x query-head groups)
-  size_t items_off, count_off, base_off, lse_off, o_off, merge_off, bytes;
+  size_t items_off, count_off, base_off, lse_off, o_off, merge_off, piece_o_off, piece_lse_off, bytes;
 };
 
 static int pick_gs(int group) {
@@ -648,7 +713,7 @@ static int few_queries(int64_t rows, int32_t hkv, int32_t d, int group) {
 }
 
 static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, int32_t d, int32_t max_k,
-                        bool listed, bool few) {
+                        bool listed, bool few, bool split_prompts) {
   Shape s{};
   const int group = hq / hkv;
   s.gs = pick_gs(group);
@@ -716,6 +781,20 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   s.merges = s.slots > 0 ? (int64_t)rows * per_split : 0;
   s.merge_off = off;
   off += (size_t)s.merges * sizeof(int32_t);
+  // Prompt items that fill less than the GPU's workgroups are split over their keys.
+  const int64_t prompts = (int64_t)s.max_prompt_items * hkv;
+  s.prompt_pieces = 1;
+  if (split_prompts && prompts > 0)
+    s.prompt_pieces = (int32_t)std::max<int64_t>(
+        1, std::min<int64_t>({kMaxPromptPieces, (kFewRound + prompts / 2) / prompts, keys / kPieceKeys}));
+  if (s.prompt_pieces > 1) {
+    const size_t rows_of = (size_t)prompts * s.prompt_pieces * kPrefillRows;
+    off = (off + 255) / 256 * 256;
+    s.piece_lse_off = off;
+    off += rows_of * sizeof(float);
+    s.piece_o_off = off;
+    off += rows_of * d * sizeof(float);
+  }
   s.bytes = off;
   return s;
 }
@@ -820,7 +899,7 @@ static Route route_of(const AttnParams& p, const Shape& s, const StepKind& k) {
   r.merge = s.max_splits > 1 && !k.prompts_only;
   if (k.prompts_only) {
     r.prompt = LV_KERNEL_PROMPT_LIST;
-    r.prompt_grid = (int)pw;
+    r.prompt_grid = (int)pw * (TP > 0 ? s.prompt_pieces : 1);
   } else if (!k.listed) {
     r.decode = LV_KERNEL_DECODE_GRID;
     r.decode_grid = (int)dw;
@@ -839,7 +918,7 @@ static Route route_of(const AttnParams& p, const Shape& s, const StepKind& k) {
   } else {
     if (k.mixed) {
       r.prompt = LV_KERNEL_PROMPT_LIST;
-      r.prompt_grid = (int)pw;
+      r.prompt_grid = (int)pw * (TP > 0 ? s.prompt_pieces : 1);
     }
     r.decode = LV_KERNEL_DECODE_LIST;
     r.decode_grid = (int)dw;
@@ -900,9 +979,18 @@ static int launch(const AttnParams& p, const Shape& s, const StepKind& k, hipStr
       }
     }
     if (!forked) {
-      if (r.prompt != LV_KERNEL_NONE)  // the serial schedule (or its fallback): prompt items on the whole GPU
-        hipLaunchKernelGGL((prompt_list_kernel<T, D, TP>), dim3(s.max_prompt_items * p.hkv), dim3(256), 0, stream,
-                           p);
+      if (r.prompt != LV_KERNEL_NONE) {  // the serial schedule (or its fallback): prompt items on the whole GPU
+        const int items = s.max_prompt_items * p.hkv;
+        if constexpr (TP > 0) {
+          if (s.prompt_pieces > 1) {
+            hipLaunchKernelGGL((prompt_split_kernel<T, D, TP>), dim3(items * s.prompt_pieces), dim3(256), 0, stream, p);
+            hipLaunchKernelGGL((prompt_merge_kernel<T, D>), dim3(items * (kPrefillRows * D / 4 / 256)), dim3(256), 0,
+                               stream, p);
+          }
+        }
+        if (TP == 0 || s.prompt_pieces == 1)
+          hipLaunchKernelGGL((prompt_list_kernel<T, D, TP>), dim3(items), dim3(256), 0, stream, p);
+      }
       if (r.decode != LV_KERNEL_NONE) {
         Route serial = r;
         if (serial.decode == LV_KERNEL_DECODE_BESIDE) {  // the fallback: one workgroup per item
@@ -1189,7 +1277,7 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, cu_seqlens_q != nullptr, max_seqlen_q,
                                   schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
-                             kind.few);
+                             kind.few, kind.mixed && !static_ws);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
   if (static_ws) {
@@ -1235,6 +1323,9 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   p.part_o = s.slots > 0 ? reinterpret_cast<float*>(ws + s.o_off) : nullptr;
   p.prompts = kind.listed ? reinterpret_cast<const int2*>(ws + s.items_off) : nullptr;
   p.items = kind.listed ? p.prompts + s.max_prompt_items : nullptr;
+  p.pieces = s.prompt_pieces;
+  p.piece_o = reinterpret_cast<float*>(ws + s.piece_o_off);
+  p.piece_lse = reinterpret_cast<float*>(ws + s.piece_lse_off);
   p.n_items = kind.listed ? reinterpret_cast<const int32_t*>(ws + s.count_off) : nullptr;
   p.ticket = kind.listed ? reinterpret_cast<int32_t*>(ws + s.count_off) + kPlanTicket : nullptr;
   p.merge_count = s.merges > 0 ? reinterpret_cast<int32_t*>(ws + s.merge_off) : nullptr;
@@ -1290,11 +1381,11 @@ extern "C" size_t lv_paged_attention_workspace_bytes(int32_t num_rows, int32_t n
     return 0;
   const bool mixed = decode_only == 0;
   const bool listed = mixed || num_rows <= kPlanMaxRows;
-  const size_t bytes = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, false).bytes;
+  const size_t bytes = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, false, mixed).bytes;
   // The longest row's queries are not known here: a step whose rows may all have few takes the larger of the two.
   const int group = num_heads / num_kv_heads;
   if (!listed || num_tokens > (int64_t)num_rows * few_queries(num_rows, num_kv_heads, head_dim, group) || (!mixed && pick_gs(group) == group)) return bytes;
-  return std::max(bytes, plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, true).bytes);
+  return std::max(bytes, plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, true, false).bytes);
 }
 
 extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t num_heads,
@@ -1312,7 +1403,7 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
   const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, has_cu_seqlens_q != 0, max_seqlen_q,
                                   schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
-                             kind.few);
+                             kind.few, kind.mixed);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
   AttnParams p{};

@@ -116,3 +116,21 @@ def test_drafts_share_one_plan_over_layers_and_graph_replays(cuda):
         torch.cuda.synchronize()
         for out in outs:
             assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize("new, cached, bs", [([40], [3000], 16), ([33, 20], [2100, 2], 64), ([70], [2500], 256),
+                                              ([17, 1], [4000, 900], 32)])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_few_prompt_items_are_split_over_their_keys(cuda, dtype, dim, new, cached, bs):
+    """Chunks of too few query tiles to fill the GPU, on cached prefixes: each tile's keys are cut into pieces (of a short
+    row's tile some are empty) and merged. One query past a tile, one row beside another, and a decode row."""
+    order = sorted(range(len(new)), key=lambda i: new[i] > 1)
+    new, cached = [new[i] for i in order], [cached[i] for i in order]
+    hq, hkv = (8, 2)
+    info = _run(cuda, (hq, hkv), dim, dtype, new, cached, bs)
+    items = -(-sum(new) // (128 // (hq // hkv))) + len(new)
+    if info["prompt_kernel"] == "prompt_list":
+        assert info["prompt_workgroups"] > items * hkv, info
+    else:  # beside a decode row the schedule may overlap
+        assert min(new) == 1, info
