@@ -220,6 +220,18 @@ __device__ inline float xor32_max(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return vmax(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+// Sum over the 64 lanes of a wave; maximum of ints over them.
+__device__ inline float wave_sum(float x) { return xor32_sum(xor16_sum(group_sum<16>(x))); }
+__device__ inline int wave_max(int x) {
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xf, 0xf, false));
+  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x140, 0xf, 0xf, false));
+  auto r = __builtin_amdgcn_permlane16_swap((uint32_t)x, (uint32_t)x, false, false);
+  x = max((int)r[0], (int)r[1]);
+  r = __builtin_amdgcn_permlane32_swap((uint32_t)x, (uint32_t)x, false, false);
+  return max((int)r[0], (int)r[1]);
+}
 // Inclusive prefix sum over the 64 lanes of a wave.
 __device__ inline int wave_incl_scan(int x) {
   const int lane = threadIdx.x & 63;

@@ -582,47 +582,49 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   __shared__ int slots[kPlanMaxRows + 1];
   __shared__ int bucket[kLenBuckets + 1];
   __shared__ int wave_tot[3][kScanThreads / 64];
-  __shared__ int64_t wave_keys[kScanThreads / 64];
-  __shared__ int wave_max[kScanThreads / 64];
+  __shared__ float wave_keys[kScanThreads / 64];
+  __shared__ int wave_max_of[kScanThreads / 64];
   const int tid = threadIdx.x;
   auto streamed = [&](int lq) { return few ? lq > 0 : lq == 1; };  // a row of decode items
   for (int b = tid; b <= kLenBuckets; b += kScanThreads) bucket[b] = 0;
   for (int i = tid; i < n_merge; i += kScanThreads) out.merge_count[i] = 0;
-  // The decode rows' keys in all and at most.
-  int64_t keys = 0;
+  // Row r's queries and keys; the thread's first row stays in registers.
+  auto load_row = [&](int r) {
+    return make_int2(cu_q ? cu_q[r + 1] - cu_q[r] : 1, lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r]);
+  };
+  const int2 own = tid < rows ? load_row(tid) : make_int2(0, 0);
+  auto row_at = [&](int r) { return r == tid ? own : load_row(r); };
+  // The decode rows' keys in all (fp32 is enough: the count is rounded up past its error) and at most.
+  float keys = 0.f;
   int longest = 1;
   for (int r = tid; r < rows; r += kScanThreads) {
-    const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    if (streamed(lq)) {
-      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
-      keys += max(lk, 0);
-      longest = max(longest, lk);
+    const int2 row = row_at(r);
+    if (streamed(row.x)) {
+      keys += (float)max(row.y, 0);
+      longest = max(longest, row.y);
     }
   }
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) {
-    keys += __shfl_xor(keys, d, 64);
-    longest = max(longest, __shfl_xor(longest, d, 64));
-  }
+  keys = wave_sum(keys);
+  longest = wave_max(longest);
   if ((tid & 63) == 0) {
     wave_keys[tid >> 6] = keys;
-    wave_max[tid >> 6] = longest;
+    wave_max_of[tid >> 6] = longest;
   }
   __syncthreads();
-  keys = 0;
+  keys = 0.f;
   longest = 1;
 #pragma unroll
   for (int w = 0; w < kScanThreads / 64; ++w) {
     keys += wave_keys[w];
-    longest = max(longest, wave_max[w]);
+    longest = max(longest, wave_max_of[w]);
   }
   int64_t want = longest;
-  if (pieces > 0) want = min(want, max((int64_t)kMinSplit, (keys + pieces - 1) / pieces));
+  if (pieces > 0) want = min(want, max((int64_t)kMinSplit, (int64_t)(keys * 1.00001f / (float)pieces) + 1));
   int split = (int)min((want + kSplitStep - 1) / kSplitStep * kSplitStep, (int64_t)INT32_MAX);
   for (;;) {  // every thread leaves together: slots[rows] is the same for all, and split reaches the longest row
     for (int r = tid; r < rows; r += kScanThreads) {
-      const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+      const int2 row = row_at(r);
+      const int lq = row.x, lk = row.y;
       const int n = streamed(lq) ? (lk > split ? (lk + split - 1) / split : 1) : 0;  // the row's decode items
       pre[r] = lq > 1 && !few ? (lq + qp - 1) / qp : 0;
       full[r] = max(n - 1, 0);
@@ -636,9 +638,9 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     __syncthreads();  // every thread has read slots[rows]
   }
   for (int r = tid; r < rows; r += kScanThreads) {
-    const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    if (streamed(lq)) {
-      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+    const int2 row = row_at(r);
+    if (streamed(row.x)) {
+      const int lk = row.y;
       const int n = lk > split ? (lk + split - 1) / split : 1;
       atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
       if (n > 1) out.part_base[r] = slots[r];
@@ -654,21 +656,28 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   }
   __syncthreads();
   const int npre = pre[rows], nfull = full[rows], npart = bucket[kLenBuckets];
-  // Full splits, one thread each (a few long rows hold hundreds: a thread per row would write them one by one).
-  for (int i = tid; i < nfull; i += kScanThreads) {
-    int lo = 0, hi = rows - 1;  // the last row whose first full split is at or before i
+  // Prompt items and full splits, one thread each (a few long rows hold hundreds: a thread per row would write them one by
+  // one, 9 us for seven prompts' 260 items, 5 so).
+  auto row_of = [&](const int* before, int i) {  // the last row with at most i items before its own
+    int lo = 0, hi = rows - 1;
     while (lo < hi) {
       const int mid = (lo + hi + 1) >> 1;
-      if (full[mid] <= i) lo = mid; else hi = mid - 1;
+      if (before[mid] <= i) lo = mid; else hi = mid - 1;
     }
-    if (i < max_items) out.items[i] = make_int2(lo, i - full[lo]);
+    return lo;
+  };
+  for (int i = tid; i < min(npre, max_prompts); i += kScanThreads) {
+    const int r = row_of(pre, i);
+    out.prompts[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
+  }
+  for (int i = tid; i < min(nfull, max_items); i += kScanThreads) {
+    const int r = row_of(full, i);
+    out.items[i] = make_int2(r, i - full[r]);
   }
   for (int r = tid; r < rows; r += kScanThreads) {
-    for (int i = pre[r]; i < pre[r + 1]; ++i)
-      if (i < max_prompts) out.prompts[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
-    const int lq = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
-    if (streamed(lq)) {
-      const int lk = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+    const int2 row = row_at(r);
+    if (streamed(row.x)) {
+      const int lk = row.y;
       const int n = lk > split ? (lk + split - 1) / split : 1;
       const int pos = nfull + atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
       if (pos < max_items) out.items[pos] = make_int2(r, n - 1);
