@@ -76,7 +76,8 @@ class DecodeGraphs:
             raise ValueError("a row's block list does not cover its context")
         n = 3 * bs + 1 + at
         self._inputs[:n].copy_(self._host[:n], non_blocking=True)
-        self._copied = torch.cuda.Event()
+        if self._copied is None:
+            self._copied = torch.cuda.Event()
         self._copied.record(torch.cuda.current_stream(self.device))
 
     # -- the captured step -----------------------------------------------------------------------------------
@@ -123,8 +124,8 @@ class DecodeGraphs:
             raise ValueError(f"no captured graph holds {rows} rows (sizes {self.sizes})")
         tokens = rows * self.query_len
         self._stage(bs, num_cached, block_lists)
-        self.q[:tokens].copy_(q)
-        self.k[:tokens].copy_(k)
-        self.v[:tokens].copy_(v)
+        # One launch for the three copies where their layouts allow (a replay of a few rows is host work and launches:
+        # 3 rows of 16/8 heads 62-71 us with three copies and a new event each time, 57 with one).
+        torch._foreach_copy_([self.q[:tokens], self.k[:tokens], self.v[:tokens]], [q, k, v])
         self.graphs[bs].replay()
         return self.out[:tokens]

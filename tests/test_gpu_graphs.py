@@ -66,3 +66,22 @@ def test_a_step_larger_than_every_graph_is_refused(cuda):
     kv = torch.zeros(3, HKV, DIM, dtype=torch.bfloat16, device=cuda)
     with pytest.raises(ValueError, match="no captured graph"):
         graphs.replay([1, 1, 1], [[0], [1], [2]], q, kv, kv)
+
+
+def test_replay_takes_inputs_of_any_layout(cuda):
+    """Queries, keys and values that are views of one fused tensor, fp32, or on the host replay as plain ones do."""
+    gen = torch.Generator(device=cuda).manual_seed(0)
+
+    def rnd(*shape):
+        return torch.randn(*shape, device=cuda, generator=gen).to(torch.bfloat16)
+
+    kc, vc = rnd(64, 16, 2, 64), rnd(64, 16, 2, 64)
+    graphs = DecodeGraphs(MI355XAttention(8, 64, 0.125, 2), kc, vc, [4], 10)
+    graphs.capture()
+    q, k, v = rnd(3, 8, 64), rnd(3, 2, 64), rnd(3, 2, 64)
+    cached, lists = [40, 20, 3], [[0, 1, 2], [3, 4], [5]]
+    want = graphs.replay(cached, lists, q, k, v).clone()
+    fused = torch.cat([x.flatten(1) for x in (q, k, v)], 1)
+    views = [x.view(3, -1, 64) for x in fused.split([512, 128, 128], 1)]
+    for form in (views, [x.float() for x in (q, k, v)], [x.cpu() for x in (q, k, v)], [q, k.float(), views[2]]):
+        assert torch.equal(graphs.replay(cached, lists, *form), want)
