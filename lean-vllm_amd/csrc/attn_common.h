@@ -529,7 +529,8 @@ __device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, c
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     if constexpr (SPLIT) {
       const int64_t at = (int64_t)slot * kPrefillRows + wave * 32 + nb * 16 + n;
-      if (j4 == 0) p.piece_lse[at] = lsum > 0.f ? m[nb] * c + fast_log2(lsum) : -INFINITY;
+      // Of a NaN sum NaN, so that the merge keeps it where every piece's is one.
+      if (j4 == 0) p.piece_lse[at] = lsum > 0.f || lsum != lsum ? m[nb] * c + fast_log2(lsum) : -INFINITY;
 #pragma unroll
       for (int b = 0; b < DB; ++b) *reinterpret_cast<f32x4*>(p.piece_o + at * DV + b * 16 + 4 * j4) = o[nb][b] * inv;
       continue;

@@ -294,7 +294,7 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
         for (int w = w0; w < kWaves; w += NS) mmax = fmaxf(mmax, wm[w * 16 + i]);
 #pragma unroll
         for (int e = 0; e < N; ++e) x[e] = 0.f;
-        if (mmax == -INFINITY) return mmax;
+        mmax = merge_base(mmax);
 #pragma unroll
         for (int w = w0; w < kWaves; w += NS) {
           const float wt = fast_exp2(wm[w * 16 + i] - mmax);
@@ -302,10 +302,10 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
 #pragma unroll
           for (int e = 0; e < N; ++e) x[e] += wt * wacc[(w * 16 + i) * PITCH + d0 + e];
         }
-        const float inv = 1.f / den;
+        const float inv = inv_sum(den);
 #pragma unroll
         for (int e = 0; e < N; ++e) x[e] *= inv;
-        return mmax + fast_log2(den);
+        return mmax + fast_log2(den);  // no key seen: -inf
       };
       for (int i = threadIdx.x; i < NS * 16 * (D / 4); i += 64 * kWaves) {
         const int row16 = i / (D / 4), d0 = (i % (D / 4)) * 4, w0 = row16 / 16, ri = row16 % 16;

@@ -288,6 +288,13 @@ __device__ inline void block_scan(int* a, int n, int (&wave_tot)[1][kScanThreads
   block_scan<1>(one, n, wave_tot);
 }
 
+// The maximum that partial sums are rescaled to when they merge. Where no partial saw a key every maximum is -inf, and 0
+// stands in for it: each weighs exp2(-inf) = 0. A partial of NaN scores may have a maximum of -inf as well; its NaN sum
+// then reaches the result, which skipping the merge would turn into zeros.
+__device__ __forceinline__ float merge_base(float m) { return m == -INFINITY ? 0.f : m; }
+// 1 / a softmax's denominator: 0 where no key was seen, NaN where a score was not a number.
+__device__ __forceinline__ float inv_sum(float l) { return l > 0.f || l != l ? 1.f / l : 0.f; }
+
 constexpr float kLog2e = 1.4426950408889634f;
 // log2 units by which an online softmax's running max may trail the true max before the accumulators are
 // rescaled: probabilities then stay below 2^kRescaleSlack, well inside bf16 / fp16 and fp32 range.

@@ -244,7 +244,7 @@ __global__ __launch_bounds__(256) void mla_decode_dma_kernel(MlaParams p) {
       const int d = 128 * wave + 16 * j + 4 * g;
       *reinterpret_cast<f32x4*>(dst + d) = o[j] * inv;
     }
-    if (wave == 0 && g == 0) p.part_lse[slot] = lsum > 0.f ? m * c + fast_log2(lsum) : -INFINITY;
+    if (wave == 0 && g == 0) p.part_lse[slot] = lsum > 0.f || lsum != lsum ? m * c + fast_log2(lsum) : -INFINITY;
   }
 }
 
@@ -654,7 +654,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
         const int col = (cons.tile * NB + nb) * 16 + n;
         if (col >= columns) continue;
         const float l = s_sum[nb][0][n] + s_sum[nb][1][n];
-        const float inv = l > 0.f || l != l ? 1.f / l : 0.f;  // 0: an earlier query sees none of the run's latents
+        const float inv = inv_sum(l);  // 0: an earlier query sees none of the run's latents
         if (whole) {
           const int qj = col / p.heads;
           char* dst = p.out + (int64_t)(cons.row * p.lq + qj) * p.o_st + (int64_t)(col - qj * p.heads) * p.o_sh;
@@ -723,14 +723,14 @@ __global__ __launch_bounds__(256) void mla_run_merge_kernel(MlaParams p) {
       float bm = m;
 #pragma unroll
       for (int i = 0; i < kRunMergeBatch; ++i) bm = fmaxf(bm, ls[i]);
-      if (bm == -INFINITY) continue;
-      const float alpha = fast_exp2(m - bm);  // 0 while m is -inf
+      const float base = merge_base(bm);
+      const float alpha = fast_exp2(m - base);  // 0 while m is -inf
       den *= alpha;
 #pragma unroll
       for (int e = 0; e < PER; ++e) o[e] *= alpha;
 #pragma unroll
       for (int i = 0; i < kRunMergeBatch; ++i) {
-        const float w = fast_exp2(ls[i] - bm);  // 0 past the last run
+        const float w = fast_exp2(ls[i] - base);  // 0 past the last run
         den += w;
 #pragma unroll
         for (int e = 0; e < PER / 4; ++e)
@@ -739,7 +739,7 @@ __global__ __launch_bounds__(256) void mla_run_merge_kernel(MlaParams p) {
       }
       m = bm;
     }
-    const float inv = den > 0.f ? 1.f / den : 0.f;
+    const float inv = inv_sum(den);
 #pragma unroll
     for (int e = 0; e < PER; ++e) o[e] *= inv;
   }
@@ -766,20 +766,19 @@ __global__ __launch_bounds__(64) void mla_merge_kernel(MlaParams p) {
 #pragma unroll
   for (int e = 0; e < PER; ++e) o[e] = 0.f;
   float den = 0.f;
-  if (mmax != -INFINITY) {
-    for (int s = 0; s < nsplit; ++s) {
-      const float w = fast_exp2(p.part_lse[slot0 + s] - mmax);
-      den += w;
-      const f32x4* src = reinterpret_cast<const f32x4*>(p.part_o + (slot0 + s) * kVDim + lane * PER);
+  mmax = merge_base(mmax);
+  for (int s = 0; s < nsplit; ++s) {
+    const float w = fast_exp2(p.part_lse[slot0 + s] - mmax);
+    den += w;
+    const f32x4* src = reinterpret_cast<const f32x4*>(p.part_o + (slot0 + s) * kVDim + lane * PER);
 #pragma unroll
-      for (int e = 0; e < PER / 4; ++e) {
-        const f32x4 x = src[e];
+    for (int e = 0; e < PER / 4; ++e) {
+      const f32x4 x = src[e];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[4 * e + r] = fmaf(w, x[r], o[4 * e + r]);
-      }
+      for (int r = 0; r < 4; ++r) o[4 * e + r] = fmaf(w, x[r], o[4 * e + r]);
     }
   }
-  const float inv = den > 0.f ? 1.f / den : 0.f;
+  const float inv = inv_sum(den);
   u32x4 packed;
 #pragma unroll
   for (int w = 0; w < 4; ++w) packed[w] = E::pack(o[2 * w] * inv, o[2 * w + 1] * inv);

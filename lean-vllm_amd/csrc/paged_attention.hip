@@ -280,7 +280,7 @@ __device__ void decode_item(const AttnParams& p, int row, int split, int per, in
     for (int w = 0; w < kWaves; ++w) mmax = fmaxf(mmax, wm[w * HG + g]);
 #pragma unroll
     for (int e = 0; e < N; ++e) o[e] = 0.f;
-    if (mmax == -INFINITY) return mmax;
+    mmax = merge_base(mmax);
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
       const float wt = fast_exp2(wm[w * HG + g] - mmax);
@@ -288,10 +288,10 @@ __device__ void decode_item(const AttnParams& p, int row, int split, int per, in
 #pragma unroll
       for (int e = 0; e < N; ++e) o[e] += wt * wacc[(w * HG + g) * D + d0 + e];
     }
-    const float inv = 1.f / den;
+    const float inv = inv_sum(den);
 #pragma unroll
     for (int e = 0; e < N; ++e) o[e] *= inv;
-    return mmax + fast_log2(den);
+    return mmax + fast_log2(den);  // no key seen: -inf
   };
   auto head_of = [&](int g) { return (kvh + g / GS) * p.group + qg * GS + g % GS; };  // g: hs-major
   if (nsplit <= 1) {
@@ -468,17 +468,16 @@ __global__ __launch_bounds__(256) void prompt_merge_kernel(AttnParams p) {
   }
 #pragma unroll
   for (int i = 0; i < kMaxPromptPieces; ++i) m = fmaxf(m, ls[i]);
+  m = merge_base(m);
   float den = 0.f;
   f32x4 o = {0, 0, 0, 0};
-  if (m != -INFINITY) {
 #pragma unroll
-    for (int i = 0; i < kMaxPromptPieces; ++i) {
-      const float w = fast_exp2(ls[i] - m);
-      den += w;
-      o += w * x[i];
-    }
-    o *= 1.f / den;
+  for (int i = 0; i < kMaxPromptPieces; ++i) {
+    const float w = fast_exp2(ls[i] - m);
+    den += w;
+    o += w * x[i];
   }
+  o *= inv_sum(den);
   *reinterpret_cast<u32x2*>(p.out + (int64_t)(q0 + pos) * p.o_st + (int64_t)head * p.o_sh + d0 * 2) =
       u32x2{E::pack(o[0], o[1]), E::pack(o[2], o[3])};
 }

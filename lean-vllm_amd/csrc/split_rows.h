@@ -94,14 +94,14 @@ __device__ __forceinline__ void merge_split_partials(const AttnParams& p, const 
       float bm = m[q];
 #pragma unroll
       for (int i = 0; i < B; ++i) bm = fmaxf(bm, ls[q][i]);
-      if (bm == -INFINITY) continue;
-      const float alpha = fast_exp2(m[q] - bm);  // 0 while m is -inf
+      const float base = merge_base(bm);
+      const float alpha = fast_exp2(m[q] - base);  // 0 while m is -inf
       den[q] *= alpha;
       o0[q] *= alpha;
       o1[q] *= alpha;
 #pragma unroll
       for (int i = 0; i < B; ++i) {
-        const float w = fast_exp2(ls[q][i] - bm);  // 0 past the last split
+        const float w = fast_exp2(ls[q][i] - base);  // 0 past the last split
         den[q] += w;
         o0[q] = fmaf(w, x[q][i][0], o0[q]);
         o1[q] = fmaf(w, x[q][i][1], o1[q]);
@@ -112,7 +112,7 @@ __device__ __forceinline__ void merge_split_partials(const AttnParams& p, const 
 #pragma unroll
   for (int q = 0; q < NP; ++q) {
     if (pc[q].slot < 0) continue;
-    const float inv = den[q] > 0.f ? 1.f / den[q] : 0.f;
+    const float inv = inv_sum(den[q]);
     *reinterpret_cast<uint32_t*>(p.out + pc[q].tok * p.o_st + pc[q].head * p.o_sh + (int64_t)pc[q].d0 * 2) =
         E::pack(o0[q] * inv, o1[q] * inv);
   }
