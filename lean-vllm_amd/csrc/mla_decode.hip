@@ -284,6 +284,7 @@ constexpr int kRunMin = 4;           // places per run at least (past a unit's s
 constexpr int kRunStages = 3;        // ring depth (four stream no faster)
 constexpr int kRunWaves = 8;
 constexpr int kRunsPerCU = 1;        // run workgroups per CU
+enum : int { kGrow = 1, kUnseen = 2 };
 constexpr int kRunMaxUnits = 8192;   // units the in-kernel scan serves
 constexpr int kRunRow = kLatent;     // LDS row pitch in elements: no padding, 16-byte chunk c of row r at c ^ (r & 6), so
                                      // that operand and transposing reads meet no bank conflicts
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
   __shared__ u32x2 s_p[NB][LB][64];      // P^T operands of the stage
   __shared__ float s_max[NB][LB][16];    // its maxima
   __shared__ float s_sum[NB][LB][16];    // row sums at a unit's end
-  __shared__ int s_grow[8];
+  __shared__ int s_state[8];             // what its score waves found: kGrow, kUnseen
   __shared__ int wave_tot[W];
   __shared__ int first[3];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -360,7 +361,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
   }
   const int x = wave_incl_scan(local);
   if (lane == 63) wave_tot[wave] = x;
-  if (tid < 8) s_grow[tid] = 0;
+  if (tid < 8) s_state[tid] = 0;
   __syncthreads();
   int excl = x - local, total = 0;
 #pragma unroll
@@ -496,6 +497,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
 
   u32x4 qb[18];  // Q^T operand: lane holds dims 32 k + 8 g .. + 7 of column n of block cb
   int sees = 0;  // latents that column sees
+  int later = 0;  // latents that the unit's first query does not see and its last does
   float m[NB], lsum = 0.f;
   f32x4 o[NB][DB];
   int issued = 0;
@@ -522,6 +524,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
     if (cons.t < 0 || !kValuesFirst) refill();
     const uint16_t* stage = ring + (k % kRunStages) * kRunElems;
     if (cons.t < 0) {
+      later = cons.lk - cons.len + p.lq - 1 - (cons.tile > 0 ? cons.tile * NB * 16 / p.heads : 0);
       if (wave < SW) {
         const uint16_t* qs = stage + cb * 16 * kRunRow;
 #pragma unroll
@@ -586,9 +589,14 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       }
       __builtin_amdgcn_sched_group_barrier(0x008, 6, 0);
       sc += sd;
+      bool unseen = false;  // a latent that the column does not see is no number (then its score is none)
       if (t0 + kRunTile > cons.lk - (p.lq - 1)) {  // else every column sees the stage
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sc[r] = t0 + 16 * lb + 4 * g + r < sees ? sc[r] : -INFINITY;
+        for (int r = 0; r < 4; ++r) {
+          const bool in = t0 + 16 * lb + 4 * g + r < sees;
+          unseen |= !in && !__builtin_isfinite(sc[r]);
+          sc[r] = in ? sc[r] : -INFINITY;
+        }
       }
       float mx = vmax(vmax(sc[0], sc[1]), vmax(sc[2], sc[3]));
       mx = xor32_max(xor16_max(mx));
@@ -596,19 +604,17 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       const bool grow = mx > mo && (mo == -INFINITY || (mx - mo) * c > kRescaleSlack);
       mc = mo == -INFINITY ? 0.f : mo * c;
       if (g == 0) s_max[cb][lb][n] = mx;
-      if (lane == 0) s_grow[wave] = 0;
-      if (__any(grow)) {
-        if (lane == 0) s_grow[wave] = 1;
-      } else {
-        put_probabilities();
-      }
+      const bool grows = __any(grow), drafts = __any(unseen);
+      if (lane == 0) s_state[wave] = (grows ? kGrow : 0) | (drafts ? kUnseen : 0);
+      if (!grows) put_probabilities();
       read_values();
     }
     // LDS only: the stage loads in flight are not waited for.
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    int grown = 0;
+    int state = 0;
 #pragma unroll
-    for (int w = 0; w < SW; ++w) grown |= s_grow[w];
+    for (int w = 0; w < SW; ++w) state |= s_state[w];
+    state = __builtin_amdgcn_readfirstlane(state);  // the same in every wave
     u32x4 pb[NB];
     auto get_probabilities = [&] {
 #pragma unroll
@@ -618,7 +624,7 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       }
     };
     get_probabilities();
-    if (__builtin_amdgcn_readfirstlane(grown)) {  // the same in every wave
+    if (state & kGrow) {
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
         const float mn = vmax(m[nb], vmax(s_max[nb][0][n], s_max[nb][1][n]));
@@ -637,10 +643,42 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       get_probabilities();
     }
     lsum += psum;
+    // Latents from `common` on are drafts that the unit's first query does not see. Its weights there are 0, but a value
+    // that is no number would reach its sums all the same: where a stage has one, such latents are left out of the product
+    // and added to the columns that see them one by one.
+    const int common = cons.lk - later;
+    if (state & kUnseen) {
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {  // word w of an operand: latents t0 + 16 (w / 2) + 4 g + 2 (w % 2) and the next
+        const int t = t0 + 16 * (w >> 1) + 4 * g + 2 * (w & 1);
+        const uint32_t keep = t + 1 < common ? 0xffffffffu : t < common ? 0xffffu : 0u;
+#pragma unroll
+        for (int j = 0; j < DB; ++j) va[j][w] &= keep;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < DB; ++j)
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) o[nb][j] = E::mfma16x16x32(va[j], pb[nb], o[nb][j]);
+    if (state & kUnseen) {
+      for (int t = max(t0, common); t < min(t0 + kRunTile, cons.lk); ++t) {
+        const int r = t - t0;
+        // Its first column in the tile: query t - (len - lq) is the first to see it.
+        const int c0 = (t - cons.len + p.lq) * p.heads - cons.tile * NB * 16;
+#pragma unroll
+        for (int j = 0; j < DB; ++j) {
+          const int chunk = 2 * DB * wave + 2 * j + (g >> 1);  // dims 16 DB wave + 16 j + 4 g .. + 3
+          const u32x2 v = *reinterpret_cast<const u32x2*>(stage + r * kRunRow + 8 * (chunk ^ (r & 6)) + 4 * (g & 1));
+#pragma unroll
+          for (int nb = 0; nb < NB; ++nb) {
+            const uint32_t pair = s_p[nb][r >> 4][n + 4 * (r & 12)][(r >> 1) & 1];
+            const float pr = r & 1 ? E::hi(pair) : E::lo(pair);
+            if (16 * nb + n >= c0)
+              o[nb][j] += f32x4{pr * E::lo(v[0]), pr * E::hi(v[0]), pr * E::lo(v[1]), pr * E::hi(v[1])};
+          }
+        }
+      }
+    }
 
     if (cons.t + 1 == cons.tu || cons.pu + cons.t + 1 == end) {  // the unit's last stage in this run
       const bool whole = cons.pu >= start && cons.pu + cons.tu <= end;

@@ -65,8 +65,9 @@ def test_a_query_that_is_not_finite_gives_nan(cuda, step, dim, kind):
     torch.testing.assert_close(out.float().cpu(), want, **TOL)
 
 
-def _mla(cuda, bs, lens, queries, heads, spoil_queries=False):
-    """Random rows of `lens` latents: the step's output and the oracle's."""
+def _mla(cuda, bs, lens, queries, heads, spoil_queries=False, spoil_latents=None):
+    """Random rows of `lens` latents; spoil_latents(row's latents) plants values. The step's output
+    and the oracle's."""
     gen = torch.Generator().manual_seed(5)
     need = [-(-n // bs) for n in lens]
     width, at, tables = max(need), 0, []
@@ -81,6 +82,8 @@ def _mla(cuda, bs, lens, queries, heads, spoil_queries=False):
             _spoil(q[(i + 1) * queries - 1, heads - 1], "inf", latents[i][0])
     cache = torch.zeros(at, bs, LATENT, dtype=torch.bfloat16)
     for lat, table in zip(latents, tables):
+        if spoil_latents is not None:
+            spoil_latents(lat)
         cache.view(-1, LATENT)[torch.tensor(slots_for(table, bs, 0, lat.size(0)))] = lat
     ctx = Context(context_lens=torch.tensor(lens, dtype=torch.int32, device=cuda),
                   block_tables=torch.tensor(tables, dtype=torch.int32, device=cuda))
@@ -102,4 +105,19 @@ def test_a_latent_query_that_is_not_finite_gives_nan(cuda, heads, queries, bs):
     """Rows finished in one run, and rows cut over several."""
     out, want = _mla(cuda, bs, [40, 9000, 700], queries, heads, spoil_queries=True)
     assert want.isnan().any()
+    torch.testing.assert_close(out, want, **TOL)
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+@pytest.mark.parametrize("bs", [64, 40])
+@pytest.mark.parametrize("heads, queries", [(16, 2), (16, 4), (11, 3), (4, 5), (1, 16)])
+def test_a_drafts_latent_reaches_no_earlier_query(cuda, heads, queries, bs, value):
+    """The row's last latents, one per draft, are seen by the queries from their own on; the others' outputs do not
+    change. Row lengths put the drafts at a stage's end, across its border and at a row's start, in one run and in several."""
+    def spoil(lat):
+        lat[-1, :VDIM:7] = value  # the last query's alone
+        lat[-queries // 2, 3] = value
+    lens = [queries, 31, 32, 33, 34, 64 + queries // 2, 5000, 9000]
+    out, want = _mla(cuda, bs, lens, queries, heads, spoil_latents=spoil)
+    assert not want.isfinite().all() and want.isfinite().any()
     torch.testing.assert_close(out, want, **TOL)
