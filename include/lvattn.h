@@ -181,14 +181,14 @@ int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t
  * callers that cannot call hipMalloc -- code under HIP graph capture, tight serving loops, harnesses that forbid
  * allocation. The work list, its counters and the split-K partials live in a static device array of
  * LV_STATIC_WORKSPACE_BYTES that each GPU the library runs on holds until the process ends; a step needing more
- * (lv_paged_attention_workspace_bytes larger than that; the split-K sizing keeps steps of up to 4096 rows at any
- * context length under 9 MiB, of few queries per row under 15 MiB) is refused with LV_EINVAL. The kernels clear what must start at zero themselves
- * (the plan kernel zeroes the persistent grid's ticket and the split rows' merge counters), so no memset is recorded
+ * (the split-K sizing keeps steps of up to 4096 rows at any context length under 9 MiB, of few queries per row under
+ * 15 MiB) is refused with LV_EINVAL; the partials of a step of few prompt tiles, whose keys are split over workgroups, lie
+ * in a second array of 43 MiB, which holds any such step's. The kernels clear what must start at zero themselves (the plan
+ * kernel zeroes the persistent grid's ticket and the split rows' merge counters), so no memset is recorded
  * into a captured graph. Every call
  * on one GPU shares that GPU's array, which keeps the last call's contents: calls that overlap on one GPU (two
  * streams, two host threads, or a graph replay beside an eager call) race. Results equal lv_paged_attention's for
- * the same arguments, but for the rounding of a step of few prompt tiles, whose keys lv_paged_attention splits over
- * workgroups where its workspace has room for their partials. Set-up: the first call on a device resolves the array's address there and creates the
+ * the same arguments. Set-up: the first call on a device resolves the arrays' addresses there and creates the
  * device's second stream and its two fork/join events (which lv_paged_attention creates at its first overlapped
  * step); no device memory is allocated, and later calls create nothing. A caller that captures graphs makes one
  * call on each device before capturing. */

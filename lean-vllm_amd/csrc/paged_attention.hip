@@ -37,6 +37,9 @@ constexpr int kSplitTarget = 4096;    // decode items (x kv heads x query-head g
 constexpr int kMaxRowSplits = 128;    // and splits per row on average at most
 constexpr int kMinSplit = 256;        // keys per decode item at least
 constexpr int kFewRound = 512;        // workgroups that the GPU holds at once, two per CU
+// Pieces of a step's split prompt items at most: n items are cut into (kFewRound + n / 2) / n >= 2 pieces each, so n is at
+// most 2/3 kFewRound, and n pieces of each come to at most kFewRound + n / 2.
+constexpr int kMaxPieces = kFewRound * 4 / 3;
 constexpr int64_t kFewPartBytes = 14 << 20;  // partials of a step of few queries per row at most (within the static workspace)
 constexpr int kSplitStep = 64;        // and a multiple of this: one tile of every wave
 constexpr int kSmallStepRounds = 8;   // a mixed step of at most this many GPU-fulls of workgroups is one launch
@@ -701,7 +704,8 @@ struct Shape {
   int32_t slots;       // split rows' partial slots
   int32_t prompt_pieces;  // workgroups per prompt item outside the overlap
   int64_t merges;      // split rows' merge counters (rows x kv heads x query-head groups)
-  size_t items_off, count_off, base_off, lse_off, o_off, merge_off, piece_o_off, piece_lse_off, bytes;
+  size_t items_off, count_off, base_off, lse_off, o_off, merge_off, bytes;
+  size_t piece_bytes;  // beside them, split prompt items' partials: outputs, then log-sum-exps
 };
 
 static int pick_gs(int group) {
@@ -795,17 +799,14 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   if (split_prompts && prompts > 0)
     s.prompt_pieces = (int32_t)std::max<int64_t>(
         1, std::min<int64_t>({kMaxPromptPieces, (kFewRound + prompts / 2) / prompts, keys / kPieceKeys}));
-  if (s.prompt_pieces > 1) {
-    const size_t rows_of = (size_t)prompts * s.prompt_pieces * kPrefillRows;
-    off = (off + 255) / 256 * 256;
-    s.piece_lse_off = off;
-    off += rows_of * sizeof(float);
-    s.piece_o_off = off;
-    off += rows_of * d * sizeof(float);
-  }
   s.bytes = off;
+  if (s.prompt_pieces > 1) s.piece_bytes = (size_t)prompts * s.prompt_pieces * kPrefillRows * (d + 1) * sizeof(float);
   return s;
 }
+
+// A caller's workspace: the lists and the rows' partials, then the pieces'.
+static size_t piece_off(const Shape& s) { return (s.bytes + 255) / 256 * 256; }
+static size_t workspace_bytes_of(const Shape& s) { return s.piece_bytes > 0 ? piece_off(s) + s.piece_bytes : s.bytes; }
 
 // A second stream per device and the fork/join events that tie it to the caller's stream, created on first use.
 // The mutex makes each call's record / wait / launch sequence atomic against calls from other host threads that
@@ -1094,40 +1095,47 @@ static int launch_step(const AttnParams& p, int d, const Shape& s, const StepKin
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// The workspace of lv_paged_attention_static: a file-scope device array (each GPU that loads the library holds its
-// own copy until the process ends). Host code must not pass the array's name to a kernel -- in host code it is a
-// stand-in, not a device address; its address on the current device comes from hipGetSymbolAddress, resolved once
+// The workspace of lv_paged_attention_static: file-scope device arrays (each GPU that loads the library holds its
+// own copies until the process ends), one for the lists and the rows' partials, one for the pieces of split prompt items
+// (its size covers every step that splits them). Host code must not pass an array's name to a kernel -- in host code it is
+// a stand-in, not a device address; its address on the current device comes from hipGetSymbolAddress, resolved once
 // per device and kept. The same set-up creates the device's second stream and its fork/join events, so that no
 // later call creates anything.
+constexpr size_t kStaticPieceBytes = (size_t)kMaxPieces * kPrefillRows * (128 + 1) * sizeof(float);
 static __device__ __align__(256) char scratch[LV_STATIC_WORKSPACE_BYTES];
+static __device__ __align__(256) char piece_scratch[kStaticPieceBytes];
 
-static void* scratch_on_current_device() {
-  static void* addr[64];
+struct Scratch {
+  void *ws, *pieces;
+};
+static Scratch scratch_on_current_device() {
+  static Scratch addr[64];
   static std::mutex lock;
   int dev = 0;
   const hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) {
     set_error("paged_attention_static: hipGetDevice failed: %s", hipGetErrorString(e));
-    return nullptr;
+    return Scratch{};
   }
   if (dev < 0 || dev >= 64) {
     set_error("paged_attention_static: device %d is past the 64 devices served", dev);
-    return nullptr;
+    return Scratch{};
   }
   std::lock_guard<std::mutex> g(lock);
-  if (!addr[dev]) {
-    void* ptr = nullptr;
-    const hipError_t r = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (r != hipSuccess || !ptr) {
+  if (!addr[dev].ws) {
+    Scratch s{};
+    hipError_t r = hipGetSymbolAddress(&s.ws, HIP_SYMBOL(scratch));
+    if (r == hipSuccess) r = hipGetSymbolAddress(&s.pieces, HIP_SYMBOL(piece_scratch));
+    if (r != hipSuccess || !s.ws || !s.pieces) {
       set_error("paged_attention_static: hipGetSymbolAddress of the static workspace failed on device %d: %s", dev,
                 hipGetErrorString(r));
-      return nullptr;
+      return Scratch{};
     }
     if (!side_stream()) {
       set_error("paged_attention_static: the second stream of device %d could not be created", dev);
-      return nullptr;
+      return Scratch{};
     }
-    addr[dev] = ptr;
+    addr[dev] = s;
   }
   return addr[dev];
 }
@@ -1285,21 +1293,28 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, cu_seqlens_q != nullptr, max_seqlen_q,
                                   schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
-                             kind.few, kind.mixed && !static_ws);
+                             kind.few, kind.mixed);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
+  char* pieces = nullptr;
   if (static_ws) {
     LV_REQUIRE(s.bytes <= (size_t)LV_STATIC_WORKSPACE_BYTES,
                "paged_attention_static: this step needs %zu bytes of workspace; the static workspace holds %zu "
                "(LV_STATIC_WORKSPACE_BYTES): call lv_paged_attention with a workspace instead",
                s.bytes, (size_t)LV_STATIC_WORKSPACE_BYTES);
-    workspace = scratch_on_current_device();
-    if (!workspace) return LV_EHIP;
-    workspace_bytes = LV_STATIC_WORKSPACE_BYTES;
+    LV_REQUIRE(s.piece_bytes <= kStaticPieceBytes, "paged_attention_static: %zu bytes of prompt pieces, more than %zu",
+               s.piece_bytes, kStaticPieceBytes);
+    const Scratch scratch = scratch_on_current_device();
+    if (!scratch.ws) return LV_EHIP;
+    workspace = scratch.ws;
+    pieces = (char*)scratch.pieces;
+  } else {
+    const size_t need = workspace_bytes_of(s);
+    LV_REQUIRE(workspace_bytes >= need && (need == 0 || workspace),
+               "paged_attention: workspace of %zu bytes given, %zu needed", workspace_bytes, need);
+    LV_REQUIRE(aligned(workspace, 256), "paged_attention: workspace must be 256-byte aligned");
+    if (s.piece_bytes > 0) pieces = (char*)workspace + piece_off(s);
   }
-  LV_REQUIRE(workspace_bytes >= s.bytes && (s.bytes == 0 || workspace),
-             "paged_attention: workspace of %zu bytes given, %zu needed", workspace_bytes, s.bytes);
-  LV_REQUIRE(aligned(workspace, 256), "paged_attention: workspace must be 256-byte aligned");
 
   AttnParams p{};
   shape_params(p, s, num_rows, num_heads, num_kv_heads, block_size, cache_stride_head);
@@ -1332,8 +1347,10 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   p.prompts = kind.listed ? reinterpret_cast<const int2*>(ws + s.items_off) : nullptr;
   p.items = kind.listed ? p.prompts + s.max_prompt_items : nullptr;
   p.pieces = s.prompt_pieces;
-  p.piece_o = reinterpret_cast<float*>(ws + s.piece_o_off);
-  p.piece_lse = reinterpret_cast<float*>(ws + s.piece_lse_off);
+  if (s.piece_bytes > 0) {
+    p.piece_o = reinterpret_cast<float*>(pieces);
+    p.piece_lse = p.piece_o + (s.piece_bytes / sizeof(float)) / (head_dim + 1) * head_dim;
+  }
   p.n_items = kind.listed ? reinterpret_cast<const int32_t*>(ws + s.count_off) : nullptr;
   p.ticket = kind.listed ? reinterpret_cast<int32_t*>(ws + s.count_off) + kPlanTicket : nullptr;
   p.merge_count = s.merges > 0 ? reinterpret_cast<int32_t*>(ws + s.merge_off) : nullptr;
@@ -1389,11 +1406,15 @@ extern "C" size_t lv_paged_attention_workspace_bytes(int32_t num_rows, int32_t n
     return 0;
   const bool mixed = decode_only == 0;
   const bool listed = mixed || num_rows <= kPlanMaxRows;
-  const size_t bytes = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, false, mixed).bytes;
+  auto bytes = [&](bool few) {
+    return workspace_bytes_of(plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, few,
+                                         mixed));
+  };
   // The longest row's queries are not known here: a step whose rows may all have few takes the larger of the two.
   const int group = num_heads / num_kv_heads;
-  if (!listed || num_tokens > (int64_t)num_rows * few_queries(num_rows, num_kv_heads, head_dim, group) || (!mixed && pick_gs(group) == group)) return bytes;
-  return std::max(bytes, plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, true, false).bytes);
+  const bool may_be_few = listed && num_tokens <= (int64_t)num_rows * few_queries(num_rows, num_kv_heads, head_dim, group) &&
+                          (mixed || pick_gs(group) != group);
+  return may_be_few ? std::max(bytes(false), bytes(true)) : bytes(false);
 }
 
 extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t num_heads,

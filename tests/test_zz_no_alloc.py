@@ -109,3 +109,26 @@ def test_the_static_workspace_gives_the_same_steps(cuda):
     call("lv_paged_attention_static", b, q2, kc, vc, ctx2, got2, decode=True, schedule=B.SCHEDULE_AUTO)
     assert torch.isfinite(want2).all()
     assert torch.equal(got2, want2)
+
+
+@pytest.mark.parametrize("dim, bs, new, cached", [(128, 256, [300], [9000]), (64, 16, [70, 33], [2500, 3000])])
+def test_the_static_workspace_splits_few_prompt_tiles_alike(cuda, dim, bs, new, cached):
+    """A step of few prompt tiles, whose keys are split over workgroups: the same bits from either entry point."""
+    b = MI355XAttention(32, dim, 1 / math.sqrt(dim), 8)
+    need = [-(-(c + n) // bs) for c, n in zip(cached, new)]
+    width = max(need)
+    tables = [[r * width + j for j in range(k)] + [-1] * (width - k) for r, k in enumerate(need)]
+    qs, kf, vf, kn, vn, kc, vc, slots = paged_step(cached, new, tables, len(new) * width, heads=32, kv_heads=8, dim=dim,
+                                                   bs=bs, device=cuda, dtype=torch.bfloat16)
+    b.store_kvcache(kn, vn, kc, vc, slots)
+    q = torch.cat(qs)
+    ctx = context_for(cached, new, tables, cuda)
+    items = -(-q.size(0) // 32) + len(new)
+    info = route(b, q, kc, ctx, decode=False, schedule=B.SCHEDULE_SERIAL)
+    assert info["prompt_kernel"] == "prompt_list" and info["prompt_workgroups"] > items * 8, info
+    want = torch.full_like(q, float("nan"))
+    got = torch.full_like(q, float("nan"))
+    call("lv_paged_attention", b, q, kc, vc, ctx, want, decode=False, schedule=B.SCHEDULE_SERIAL)
+    call("lv_paged_attention_static", b, q, kc, vc, ctx, got, decode=False, schedule=B.SCHEDULE_SERIAL)
+    assert torch.isfinite(want).all()
+    assert torch.equal(got, want)
