@@ -561,9 +561,17 @@ __device__ inline int len_bucket(int keys, int split) {
 // that a step is cut into about the same number of items whatever its lengths (at most pieces + rows). The caller's
 // bound on key lengths only sizes the buffers: a captured graph's bound is the longest context it may ever serve, and
 // a batch of a few rows far apart in length has most of its keys in one of them. pieces 0: rows are not split, and
-// one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]; a split
-// that needs more slots than there are (lengths past the caller's bound, rows of unequal query counts) is doubled until
-// they fit. few: rows of several queries are streamed as decode items too, one slot per query.
+// one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]. few: rows of
+// several queries are streamed as decode items too, one slot per query and split.
+//
+// few: a row's merge is one workgroup's work, and takes as long as its splits where they hold `least` keys: n splits of lk
+// keys take lk / n keys' stream (12 KB a microsecond) and lq G D n / 512 loads a thread (19 a microsecond), equal at
+// lk / n = sqrt(0.3 lk lq G). One row of 64,000 keys, 128 splits and with this bound: 8/2 heads, d128, 16 queries 160 -> 114
+// us (56 splits); 16/1 heads, 4 queries, two rows 157 -> 113; 40/1 heads, one query 114 -> 91. It is below
+// kMinSplit, and changes nothing, while lk lq G < 218,000 (4 queries of group 4 on 13,000 keys).
+//
+// A split that needs more slots than there are grows until they fit: a long row of more queries than the others (to
+// fewer_pieces first), more queries or lengths than the caller said (by the slots' ratio, a sixteenth at least).
 struct PlanOut {
   int2* prompts;    // the prompt items
   int2* items;      // the decode items
@@ -577,8 +585,8 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
                                                             const int32_t* __restrict__ cu_k, int32_t rows,
                                                             int32_t pieces, int32_t max_slots, int32_t qp,
                                                             int32_t max_prompts, int32_t max_items,
-                                                            int32_t last_first, int32_t few, int32_t n_merge,
-                                                            PlanOut out) {
+                                                            int32_t last_first, int32_t few, int32_t fewer_pieces,
+                                                            int32_t group, int32_t n_merge, PlanOut out) {
   __shared__ int pre[kPlanMaxRows + 1];
   __shared__ int full[kPlanMaxRows + 1];
   __shared__ int slots[kPlanMaxRows + 1];
@@ -586,6 +594,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   __shared__ int wave_tot[3][kScanThreads / 64];
   __shared__ float wave_keys[kScanThreads / 64];
   __shared__ int wave_max_of[kScanThreads / 64];
+  __shared__ int wave_least[kScanThreads / 64];
   const int tid = threadIdx.x;
   auto streamed = [&](int lq) { return few ? lq > 0 : lq == 1; };  // a row of decode items
   for (int b = tid; b <= kLenBuckets; b += kScanThreads) bucket[b] = 0;
@@ -598,19 +607,22 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   auto row_at = [&](int r) { return r == tid ? own : load_row(r); };
   // The decode rows' keys in all (fp32 is enough: the count is rounded up past its error) and at most.
   float keys = 0.f;
-  int longest = 1;
+  int longest = 1, least = kMinSplit;  // least: keys per split at least
   for (int r = tid; r < rows; r += kScanThreads) {
     const int2 row = row_at(r);
     if (streamed(row.x)) {
       keys += (float)max(row.y, 0);
       longest = max(longest, row.y);
+      if (few) least = max(least, (int)sqrtf(0.3f * (float)max(row.y, 0) * (float)(row.x * group)));
     }
   }
   keys = wave_sum(keys);
   longest = wave_max(longest);
+  least = wave_max(least);
   if ((tid & 63) == 0) {
     wave_keys[tid >> 6] = keys;
     wave_max_of[tid >> 6] = longest;
+    wave_least[tid >> 6] = least;
   }
   __syncthreads();
   keys = 0.f;
@@ -619,9 +631,10 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   for (int w = 0; w < kScanThreads / 64; ++w) {
     keys += wave_keys[w];
     longest = max(longest, wave_max_of[w]);
+    least = max(least, wave_least[w]);
   }
   int64_t want = longest;
-  if (pieces > 0) want = min(want, max((int64_t)kMinSplit, (int64_t)(keys * 1.00001f / (float)pieces) + 1));
+  if (pieces > 0) want = min(want, max((int64_t)least, (int64_t)(keys * 1.00001f / (float)pieces) + 1));
   int split = (int)min((want + kSplitStep - 1) / kSplitStep * kSplitStep, (int64_t)INT32_MAX);
   for (;;) {  // every thread leaves together: slots[rows] is the same for all, and split reaches the longest row
     for (int r = tid; r < rows; r += kScanThreads) {
@@ -636,7 +649,13 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     int* const sums[3] = {pre, full, slots};  // one pass over all: the kernel is its barriers
     block_scan<3>(sums, rows, wave_tot);
     if (slots[rows] <= max_slots || split >= longest) break;
-    split = split < (1 << 29) ? 2 * split : INT32_MAX;
+    int64_t grown = max((int64_t)split * slots[rows] / max(max_slots, 1), (int64_t)split + split / 16);
+    if (fewer_pieces > 0) {
+      grown = max((int64_t)split, (int64_t)(keys / (float)fewer_pieces));
+      fewer_pieces = 0;  // the next time by the slots' ratio
+    }
+    grown = (grown + kSplitStep) / kSplitStep * kSplitStep;
+    split = grown <= (1 << 30) ? (int)grown : INT32_MAX;
     __syncthreads();  // every thread has read slots[rows]
   }
   for (int r = tid; r < rows; r += kScanThreads) {
@@ -700,6 +719,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
 struct Shape {
   int32_t max_items, max_prompt_items, max_decode_items, gs;
   int32_t pieces;      // the plan cuts the decode rows' keys into this many (0: rows are not split)
+  int32_t fewer_pieces;  // few queries: and into this many where the partials of those do not fit
   int32_t max_splits;  // the most items one row may be split into
   int32_t slots;       // split rows' partial slots
   int32_t prompt_pieces;  // workgroups per prompt item outside the overlap
@@ -724,8 +744,9 @@ static int few_queries(int64_t rows, int32_t hkv, int32_t d, int group) {
   return std::min(kFewMaxQueries, most / group);
 }
 
+// max_q: queries per row at most, of a step of few queries.
 static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, int32_t d, int32_t max_k,
-                        bool listed, bool few, bool split_prompts) {
+                        bool listed, bool few, int32_t max_q, bool split_prompts) {
   Shape s{};
   const int group = hq / hkv;
   s.gs = pick_gs(group);
@@ -749,12 +770,15 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   // a share / two thirds / one: 12 rows 121 / 117 / 110 us, 24 rows 193 / 192 / 182, 48 rows 346 / 353 / 336; 4 rows with
   // their remainders beside the round 66.7, in it 57.9; 100 rows split by shares 631, unsplit 624.
   const int64_t units = rows * per_split;
-  const int64_t row_queries = few ? ((int64_t)tokens + rows - 1) / rows : 1;  // partial slots per split
+  const int64_t row_queries = few ? ((int64_t)tokens + rows - 1) / rows : 1;  // a row's on average: partial slots per split
+  const int64_t slot_bytes = (int64_t)hq * (d + 1) * (int64_t)sizeof(float);
   const int64_t share = std::max<int64_t>(1, kFewRound / per_split);  // splits of one round of workgroups
   int64_t pieces = std::max<int64_t>(1, share / 2);
-  if (few && row_queries * group > 4) {
-    if (units <= kFewRound) pieces = std::min(share - (8 * rows <= share ? rows : 0), (int64_t)kMaxRowSplits * rows);
-    const int64_t max_slots = kFewPartBytes / ((int64_t)hq * (d + 1) * (int64_t)sizeof(float));
+  const int64_t remainders = 8 * rows <= share ? rows : 0;
+  const bool light = few && row_queries * group <= 4;
+  if (few && !light) {
+    if (units <= kFewRound) pieces = std::min(share - remainders, (int64_t)kMaxRowSplits * rows);
+    const int64_t max_slots = kFewPartBytes / slot_bytes;
     if ((pieces + std::min<int64_t>(rows, pieces)) * row_queries > max_slots) pieces = max_slots / row_queries / 2;
   } else {  // up to four query rows an item weighs no more than a VALU item and splits as one
     const int64_t items = rows <= 2 ? kSplitTarget / 4 : rows <= 16 ? kSplitTarget / 2 : kSplitTarget;
@@ -772,8 +796,24 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   s.max_prompt_items = listed && !few ? sat(((int64_t)tokens + qp - 1) / qp + rows) : 0;
   s.max_decode_items = listed ? sat(splits) : 0;
   s.max_items = sat((int64_t)s.max_prompt_items + s.max_decode_items);
-  // Rows of more than one split hold more keys than a split, so there are at most `pieces` of them.
-  s.slots = s.max_splits > 1 ? sat(std::min(splits, pieces + std::min<int64_t>(rows, pieces)) * row_queries) : 0;
+  // Rows of more than one split hold more keys than a split, so there are at most `pieces` of them, and their splits have
+  // slots for row_queries each. In a step of few queries most keys may be in a row of more than that: slots for max_q each,
+  // where they fit in kFewPartBytes with the counters, at half the pieces (one workgroup per CU streams about as fast and
+  // leaves half the partials to merge), or one round of the light ones. One long row among short ones, us, with the split
+  // doubled until slots for the average row held it (before), and so: 32/8 heads, d128, 8 queries on 64,000 keys among 15 of
+  // one on 300 108.9 -> 74.8; 16 on 60,000 beside 9 on 5000 and two short 214 -> 136.5; 4 on 64,000 beside 7 of one on
+  // 1000 59.9 -> 60.6; 8/8 heads, 8 queries on 64,000 beside 3 of one on 4000 66.2 -> 65.8.
+  const int64_t merges = s.max_splits > 1 ? (int64_t)rows * per_split : 0;
+  if (s.max_splits > 1) {
+    const int64_t split_rows = std::min<int64_t>(rows, pieces);
+    int64_t slots = std::min(splits, pieces + split_rows) * row_queries;
+    if (few) {
+      s.fewer_pieces = (int32_t)std::max<int64_t>(1, light ? share - remainders : pieces / 2);
+      slots = std::max(slots, std::min(std::min(splits, s.fewer_pieces + split_rows) * std::min(max_q, tokens),
+                                       (kFewPartBytes - merges * (int64_t)sizeof(int32_t)) / slot_bytes));
+    }
+    s.slots = sat(slots);
+  }
   size_t off = 0;
   s.items_off = off;
   off += (size_t)s.max_items * sizeof(int2);
@@ -790,7 +830,7 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   s.o_off = off;
   off += parts * d * sizeof(float);
   off = (off + 255) / 256 * 256;
-  s.merges = s.slots > 0 ? (int64_t)rows * per_split : 0;
+  s.merges = merges;
   s.merge_off = off;
   off += (size_t)s.merges * sizeof(int32_t);
   // Prompt items that fill less than the GPU's workgroups are split over their keys.
@@ -1146,12 +1186,13 @@ static Scratch scratch_on_current_device() {
 struct PlanSig {
   const void* ws = nullptr;
   const int32_t *cu_q = nullptr, *lens = nullptr, *cu_k = nullptr;
-  int64_t rows = 0, tokens = 0, max_k = 0, pieces = 0, qp = 0, max_items = 0, bytes = 0;
+  int64_t rows = 0, tokens = 0, max_k = 0, pieces = 0, slots = 0, qp = 0, max_items = 0, merge_off = 0, bytes = 0;
   bool mixed = false, last_first = false, few = false;
   bool operator==(const PlanSig& o) const {
     return ws == o.ws && cu_q == o.cu_q && lens == o.lens && cu_k == o.cu_k && rows == o.rows &&
-           tokens == o.tokens && max_k == o.max_k && pieces == o.pieces && qp == o.qp && max_items == o.max_items &&
-           bytes == o.bytes && mixed == o.mixed && last_first == o.last_first && few == o.few;
+           tokens == o.tokens && max_k == o.max_k && pieces == o.pieces && slots == o.slots && qp == o.qp &&
+           max_items == o.max_items && merge_off == o.merge_off && bytes == o.bytes && mixed == o.mixed &&
+           last_first == o.last_first && few == o.few;
   }
 };
 constexpr int kPlanRecords = 32;
@@ -1293,7 +1334,7 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, cu_seqlens_q != nullptr, max_seqlen_q,
                                   schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
-                             kind.few, kind.mixed);
+                             kind.few, kind.max_q, kind.mixed);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
   char* pieces = nullptr;
@@ -1366,8 +1407,10 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   sig.tokens = num_tokens;
   sig.max_k = max_seqlen_k;
   sig.pieces = s.pieces;
+  sig.slots = s.slots;
   sig.qp = qp;
   sig.max_items = s.max_items;
+  sig.merge_off = (int64_t)s.merge_off;
   sig.bytes = (int64_t)s.bytes;
   sig.mixed = kind.mixed;
   sig.few = kind.few;
@@ -1380,7 +1423,8 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
                       reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kScanThreads), 0, st, kind.mixed ? cu_seqlens_q : nullptr,
                        seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
-                       s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few, (int32_t)s.merges, out);
+                       s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few, s.fewer_pieces,
+                       p.group, (int32_t)s.merges, out);
     LV_LAUNCH_CHECK("plan_kernel");
     planned = true;
   }
@@ -1406,14 +1450,15 @@ extern "C" size_t lv_paged_attention_workspace_bytes(int32_t num_rows, int32_t n
     return 0;
   const bool mixed = decode_only == 0;
   const bool listed = mixed || num_rows <= kPlanMaxRows;
+  const int group = num_heads / num_kv_heads;
+  const int few_q = few_queries(num_rows, num_kv_heads, head_dim, group);
+  const bool may_be_few =
+      listed && num_tokens <= (int64_t)num_rows * few_q && (mixed || pick_gs(group) != group);
   auto bytes = [&](bool few) {
     return workspace_bytes_of(plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, few,
-                                         mixed));
+                                         mixed ? few_q : 1, mixed));
   };
   // The longest row's queries are not known here: a step whose rows may all have few takes the larger of the two.
-  const int group = num_heads / num_kv_heads;
-  const bool may_be_few = listed && num_tokens <= (int64_t)num_rows * few_queries(num_rows, num_kv_heads, head_dim, group) &&
-                          (mixed || pick_gs(group) != group);
   return may_be_few ? std::max(bytes(false), bytes(true)) : bytes(false);
 }
 
@@ -1432,7 +1477,7 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
   const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, has_cu_seqlens_q != 0, max_seqlen_q,
                                   schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
-                             kind.few, kind.mixed);
+                             kind.few, kind.max_q, kind.mixed);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
   if (rg != LV_OK) return rg;
   AttnParams p{};

@@ -73,6 +73,24 @@ def context_for(num_cached, num_new, tables, device, is_prefill=True, host=True)
     )
 
 
+def guarded_workspace(monkeypatch, device, nbytes=64 << 20):
+    """A workspace of its own for the backend's calls in a test, filled with 0x5A."""
+    from lvattn import backend
+
+    ws = backend._Workspace()
+    ws._buf[device] = torch.full((nbytes,), 0x5A, dtype=torch.uint8, device=device)
+    monkeypatch.setattr(backend, "_WORKSPACE", ws)
+    return ws._buf[device]
+
+
+def plan_counts(workspace, max_items):
+    """(decode items, keys per split) of the plan a step left in its workspace: the counts (kPlan* of
+    csrc/attn_common.h) lie behind the work lists' 8-byte items, 256-byte aligned."""
+    at = -(-8 * max_items // 256) * 256
+    counts = workspace[at:at + 20].view(torch.int32).tolist()
+    return counts[0], counts[4]
+
+
 def dense_expected(qs, kf, vf, scale):
     """fp32 textbook attention per row (the reference test oracle), on the CPU."""
     return torch.cat([A.dense_attention(q.cpu().float(), k.cpu().float(), v.cpu().float(), scale)

@@ -10,8 +10,8 @@ import math
 import pytest
 import torch
 
-from helpers import context_for, dense_expected, paged_step
-from lvattn import Context, MI355XAttention
+from helpers import context_for, dense_expected, guarded_workspace, paged_step, plan_counts
+from lvattn import Context, MI355XAttention, _capi
 
 pytestmark = pytest.mark.gpu
 
@@ -62,6 +62,38 @@ def test_few_query_items_match_the_oracle(cuda, dtype, dim, step):
     info = _run(cuda, heads, dim, dtype, new, cached, bs)
     assert info["decode_kernel"] == "decode_list" and info["prompt_kernel"] == "none", info
     assert info["kv_heads_per_item"] == hp, info
+
+
+# id: (query heads, kv heads), head dim, queries of each row, keys before them, max_seqlen_q if not theirs, and the number of
+# splits of the longest row, within a split's rounding
+UNEQUAL = {
+    # Half the even share (of 512 workgroups 64 per kv head, less the rows' remainders), 15 and 14 for the average row.
+    "8-queries-beside-decodes": ((32, 8), 128, [8] + [1] * 15, [64_000] + [300] * 15, None, (28, 32)),
+    "two-of-many-queries": ((32, 8), 128, [9, 1, 16, 2], [5000, 3, 60_000, 900], None, (25, 30)),
+    # As many as the merge pays for, lk / sqrt(0.3 lk lq G); 26 for the average row.
+    "merge-bound-d64": ((8, 2), 64, [16] + [1] * 7, [64_000] + [10] * 7, None, (53, 58)),
+    "merge-bound-d128": ((8, 2), 128, [1] * 7 + [16], [10] * 7 + [64_000], None, (53, 58)),
+    "merge-bound-wide-group": ((40, 1), 64, [1], [64_000], None, (70, 74)),
+    # Slots for 4 queries a row at most: grown twice.
+    "more-queries-than-the-step-says": ((8, 2), 64, [1] * 9 + [16] + [1] * 6, [10] * 9 + [64_000] + [20] * 6, 4, (32, 34)),
+}
+
+
+@pytest.mark.parametrize("case", list(UNEQUAL))
+def test_a_long_row_of_more_queries_than_the_others_is_spread(cuda, monkeypatch, case):
+    """Partials have room for the splits of a long row that has more queries than the step's average, and a row has no more
+    splits than its merge is worth. Nothing is written past the workspace that the step asked for."""
+    (hq, hkv), dim, new, cached, max_q, (least, most) = UNEQUAL[case]
+    ws = guarded_workspace(monkeypatch, cuda)
+    info = _run(cuda, (hq, hkv), dim, torch.bfloat16, new, cached, 16, max_q=max_q)
+    assert info["decode_kernel"] == "decode_list" and info["prompt_kernel"] == "none", info
+    lens = [c + n for c, n in zip(cached, new)]
+    need = _capi.query("lv_paged_attention_workspace_bytes", len(new), sum(new), hq, hkv, dim, 16 * (-(-max(lens) // 16) + 1),
+                       int(max(new) == 1))
+    assert (ws[need:] == 0x5A).all()
+    items, split = plan_counts(ws, info["decode_workgroups"] * info["kv_heads_per_item"] // hkv)
+    assert items == sum(-(-n // split) for n in lens)
+    assert least <= -(-max(lens) // split) <= most
 
 
 @pytest.mark.parametrize("layout", ["NHD", "HND"])
