@@ -1421,8 +1421,10 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
     int2* lists = reinterpret_cast<int2*>(ws + s.items_off);
     const PlanOut out{lists, lists + s.max_prompt_items, reinterpret_cast<int32_t*>(ws + s.count_off),
                       reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kScanThreads), 0, st, kind.mixed ? cu_seqlens_q : nullptr,
-                       seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
+    // Few-query items take a row's queries from cu_seqlens_q, so its partial slots are counted from there too, also in a
+    // step that was said to have one query a row.
+    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kScanThreads), 0, st,
+                       kind.mixed || kind.few ? cu_seqlens_q : nullptr, seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
                        s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few, s.fewer_pieces,
                        p.group, (int32_t)s.merges, out);
     LV_LAUNCH_CHECK("plan_kernel");

@@ -74,6 +74,9 @@ UNEQUAL = {
     "merge-bound-d64": ((8, 2), 64, [16] + [1] * 7, [64_000] + [10] * 7, None, (53, 58)),
     "merge-bound-d128": ((8, 2), 128, [1] * 7 + [16], [10] * 7 + [64_000], None, (53, 58)),
     "merge-bound-wide-group": ((40, 1), 64, [1], [64_000], None, (70, 74)),
+    # A row of 7 queries in a step said to have one a row: its items attend all seven, and 79 splits of them (the
+    # bound of one) have no room.
+    "queries-of-a-one-query-step": ((6, 2), 64, [7] + [1] * 6, [20_000] + [5] * 6, 1, (51, 55)),
     # Slots for 4 queries a row at most: grown twice.
     "more-queries-than-the-step-says": ((8, 2), 64, [1] * 9 + [16] + [1] * 6, [10] * 9 + [64_000] + [20] * 6, 4, (32, 34)),
 }
@@ -89,7 +92,7 @@ def test_a_long_row_of_more_queries_than_the_others_is_spread(cuda, monkeypatch,
     assert info["decode_kernel"] == "decode_list" and info["prompt_kernel"] == "none", info
     lens = [c + n for c, n in zip(cached, new)]
     need = _capi.query("lv_paged_attention_workspace_bytes", len(new), sum(new), hq, hkv, dim, 16 * (-(-max(lens) // 16) + 1),
-                       int(max(new) == 1))
+                       int(max_q == 1 or max(new) == 1))
     assert (ws[need:] == 0x5A).all()
     items, split = plan_counts(ws, info["decode_workgroups"] * info["kv_heads_per_item"] // hkv)
     assert items == sum(-(-n // split) for n in lens)
