@@ -166,7 +166,8 @@ typedef struct lv_launch_info {
   int32_t prompt_workgroups;
   int32_t kv_heads_per_item;  /* 1, or 2: a decode item reads two adjacent kv heads of each token */
   int32_t two_streams;
-  int32_t keys_per_split;     /* keys per decode item at least (the plan sizes them from the rows' lengths) */
+  int32_t keys_per_split;     /* keys per decode item of a step whose rows all have one query (few-query items: as many
+                                 as the longest) and max_seqlen_k keys; the plan sizes them from the rows' lengths */
   int32_t max_splits;         /* the most decode items one row may be split into */
   int32_t splitk_merge;       /* 1: rows are split over several items; each row's last split to finish merges
                                  them (log-sum-exp) inside the decode launch */

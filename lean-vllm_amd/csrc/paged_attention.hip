@@ -572,6 +572,20 @@ __device__ inline int len_bucket(int keys, int split) {
 //
 // A split that needs more slots than there are grows until they fit: a long row of more queries than the others (to
 // fewer_pieces first), more queries or lengths than the caller said (by the slots' ratio, a sixteenth at least).
+__host__ __device__ inline int least_split(int lk, int query_rows) {
+  return (int)sqrtf(0.3f * (float)(lk > 0 ? lk : 0) * (float)query_rows);
+}
+__host__ __device__ inline int split_keys(float keys, int longest, int least, int pieces) {
+  int64_t want = longest;
+  if (pieces > 0) {
+    int64_t share = (int64_t)(keys * 1.00001f / (float)pieces) + 1;
+    share = share > least ? share : least;
+    want = want < share ? want : share;
+  }
+  want = (want + kSplitStep - 1) / kSplitStep * kSplitStep;
+  return want < INT32_MAX ? (int)want : INT32_MAX;
+}
+
 struct PlanOut {
   int2* prompts;    // the prompt items
   int2* items;      // the decode items
@@ -613,7 +627,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     if (streamed(row.x)) {
       keys += (float)max(row.y, 0);
       longest = max(longest, row.y);
-      if (few) least = max(least, (int)sqrtf(0.3f * (float)max(row.y, 0) * (float)(row.x * group)));
+      if (few) least = max(least, least_split(row.y, row.x * group));
     }
   }
   keys = wave_sum(keys);
@@ -633,9 +647,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     longest = max(longest, wave_max_of[w]);
     least = max(least, wave_least[w]);
   }
-  int64_t want = longest;
-  if (pieces > 0) want = min(want, max((int64_t)least, (int64_t)(keys * 1.00001f / (float)pieces) + 1));
-  int split = (int)min((want + kSplitStep - 1) / kSplitStep * kSplitStep, (int64_t)INT32_MAX);
+  int split = split_keys(keys, longest, least, pieces);
   for (;;) {  // every thread leaves together: slots[rows] is the same for all, and split reaches the longest row
     for (int r = tid; r < rows; r += kScanThreads) {
       const int2 row = row_at(r);
@@ -1493,7 +1505,9 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
   info->prompt_workgroups = r.prompt_grid;
   info->kv_heads_per_item = r.hp;
   info->two_streams = r.two_streams;
-  info->keys_per_split = kMinSplit;
+  const int least = kind.few ? least_split(max_seqlen_k, std::min(kind.max_q, num_tokens) * p.group) : 0;
+  info->keys_per_split = split_keys((float)num_rows * (float)max_seqlen_k, std::max(max_seqlen_k, 1),
+                                    std::max(kMinSplit, least), s.pieces);
   info->max_splits = s.max_splits;
   info->splitk_merge = r.merge;
   return LV_OK;

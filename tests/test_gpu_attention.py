@@ -9,7 +9,8 @@ import math
 import pytest
 import torch
 
-from helpers import context_for, dense_expected, paged_step, randn, slots_for
+from helpers import (context_for, dense_expected, guarded_workspace, paged_step, plan_counts, randn,
+                     slots_for)
 from lvattn import Context, MI355XAttention
 from oracle import attention as A
 
@@ -763,3 +764,28 @@ def test_splits_are_sized_from_the_rows_lengths(cuda, lens):
     want = dense_expected([q[i:i + 1] for i in live], [kf[i] for i in live], [vf[i] for i in live], 1 / math.sqrt(dim))
     torch.testing.assert_close(out[live].float().cpu(), want, atol=2e-2, rtol=1e-2)
     assert not out[[i for i, n in enumerate(lens) if not n]].any()
+
+
+@pytest.mark.parametrize("heads, rows, keys", [((8, 2), 1, 40_000), ((8, 2), 3, 40_000), ((32, 8), 20, 3008), ((8, 2), 600, 64),
+                                               ((40, 1), 1, 64_000)],
+                         ids=["one-row", "three-rows", "20-rows", "unsplit", "wide-group"])
+def test_launch_info_tells_the_keys_per_split(cuda, monkeypatch, heads, rows, keys):
+    """lv_launch_info.keys_per_split is what the plan takes for rows of max_seqlen_k keys each."""
+    (hq, hkv), bs, dim = heads, 64, 64
+    ws = guarded_workspace(monkeypatch, cuda)
+    b = MI355XAttention(hq, dim, 1 / math.sqrt(dim), hkv)
+    kc, vc = (torch.zeros(keys // bs, bs, hkv, dim, dtype=torch.bfloat16, device=cuda) for _ in range(2))
+    ctx = Context(context_lens=torch.full((rows,), keys, dtype=torch.int32, device=cuda),
+                  block_tables=torch.arange(keys // bs, dtype=torch.int32, device=cuda).repeat(rows, 1))
+    b.launch_trace = []
+    b.decode(torch.zeros(rows, hq, dim, dtype=torch.bfloat16, device=cuda), kc, vc, ctx)
+    torch.cuda.synchronize()
+    info = b.launch_trace[-1]
+    group = hq // hkv
+    lanes = next(g for g in (4, 2, 1) if group % g == 0)
+    few = group not in (1, 2, 4)
+    groups = 1 if few else group // lanes
+    listed = 0 if few else -(-rows // (128 // group)) + rows
+    items, split = plan_counts(ws, listed + info["decode_workgroups"] * info["kv_heads_per_item"] // hkv // groups)
+    assert items == rows * -(-keys // split)
+    assert info["keys_per_split"] == split
