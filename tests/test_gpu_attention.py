@@ -738,11 +738,12 @@ def test_huge_values_with_scores_above_the_first_tile(cuda, dim):
 
 @pytest.mark.parametrize("lens", [[40_000], [3, 20_000], [5_000, 0, 9_000] + [700] * 13, [12_000] + [257] * 16],
                          ids=["one-row", "two-rows", "16-rows", "17-rows"])
-def test_splits_are_sized_from_the_rows_lengths(cuda, lens):
+def test_splits_are_sized_from_the_rows_lengths(cuda, monkeypatch, lens):
     """Decode rows far apart in length, under a table twice as wide as the longest needs: the plan sizes the splits
     from the keys there are. The row counts sit on both sides of the rules that bound the number of splits (2 and 16
     rows; one row's splits capped). Against the oracle."""
     bs, heads, kv_heads, dim = 16, 8, 2, 64
+    ws = guarded_workspace(monkeypatch, cuda)
     need = [-(-n // bs) for n in lens]
     width, at, tables = 2 * max(need), 0, []
     for k in need:
@@ -760,7 +761,17 @@ def test_splits_are_sized_from_the_rows_lengths(cuda, lens):
     b.launch_trace = []
     out = b.decode(q, kc, vc, ctx)
     torch.cuda.synchronize()
-    assert b.launch_trace[-1]["splitk_merge"]
+    info = b.launch_trace[-1]
+    assert info["splitk_merge"]
+    # The plan itself: all keys over 4096 items (2048 up to 16 rows, 1024 up to 2; 128 splits a row at most) of two kv heads,
+    # less the rows' remainders; one query lane group of four heads.
+    rows = len(lens)
+    pieces = min((1024 if rows <= 2 else 2048 if rows <= 16 else 4096) // kv_heads, 128 * rows) - rows
+    listed = -(-rows // (128 // (heads // kv_heads))) + rows  # room for prompt items ahead of the decode items
+    items, split = plan_counts(ws, listed + info["decode_workgroups"] * info["kv_heads_per_item"] // kv_heads)
+    even = max(256, -(-(sum(lens) // pieces + 1) // 64) * 64)
+    assert split == even
+    assert items == sum(max(1, -(-n // split)) for n in lens)
     want = dense_expected([q[i:i + 1] for i in live], [kf[i] for i in live], [vf[i] for i in live], 1 / math.sqrt(dim))
     torch.testing.assert_close(out[live].float().cpu(), want, atol=2e-2, rtol=1e-2)
     assert not out[[i for i, n in enumerate(lens) if not n]].any()
