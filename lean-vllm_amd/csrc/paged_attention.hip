@@ -543,10 +543,9 @@ __global__ __launch_bounds__(256) void decode_grid_kernel(AttnParams p) {
 }
 
 constexpr int kLenBuckets = 64;
-// Bucket of a split of `keys` keys out of `split`: longer splits get smaller buckets (dispatched first).
-__device__ inline int len_bucket(int keys, int split) {
-  const int b = (int)(((int64_t)(split - keys) * kLenBuckets) / split);
-  return b < kLenBuckets - 1 ? b : kLenBuckets - 1;
+// Bucket of a split that is `short_of` keys short of a whole one: longer splits get smaller buckets (dispatched first).
+__device__ inline int len_bucket(int short_of, float per_key) {
+  return min(max((int)((float)short_of * per_key), 0), kLenBuckets - 1);
 }
 
 // Work lists of a step, longest work first: the prompt items (row, -1 - tile); and the decode items, every full split
@@ -594,6 +593,11 @@ struct PlanOut {
   int32_t* merge_count;
 };
 
+// ROWS: rows a thread at most. The kernel is its barriers, its round trips to memory and its code, which a step's one plan meets
+// cold: the rows' loads are issued together, once, and all that is known of a row stays in registers. 3 / 256 / 1024 / 4096
+// rows of a decode step 6.0 / 6.4 / 7.4 / 12.8 us with later rows loaded again in each pass and 64-bit bucket divisions, 5.4
+// / 5.9 / 6.6 / 10.4 so (with splits of a size fixed on the host 5.6 / 4.5 / 5.0 / 8.9).
+template <int ROWS>
 __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __restrict__ cu_q,
                                                             const int32_t* __restrict__ lens_k,
                                                             const int32_t* __restrict__ cu_k, int32_t rows,
@@ -601,38 +605,41 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
                                                             int32_t max_prompts, int32_t max_items,
                                                             int32_t last_first, int32_t few, int32_t fewer_pieces,
                                                             int32_t group, int32_t n_merge, PlanOut out) {
-  __shared__ int pre[kPlanMaxRows + 1];
-  __shared__ int full[kPlanMaxRows + 1];
-  __shared__ int slots[kPlanMaxRows + 1];
+  __shared__ int pre[ROWS * kScanThreads + 1];
+  __shared__ int full[ROWS * kScanThreads + 1];
+  __shared__ int slots[ROWS * kScanThreads + 1];
   __shared__ int bucket[kLenBuckets + 1];
   __shared__ int wave_tot[3][kScanThreads / 64];
   __shared__ float wave_keys[kScanThreads / 64];
   __shared__ int wave_max_of[kScanThreads / 64];
   __shared__ int wave_least[kScanThreads / 64];
   const int tid = threadIdx.x;
-  auto streamed = [&](int lq) { return few ? lq > 0 : lq == 1; };  // a row of decode items
+  int lq[ROWS], lk[ROWS], n[ROWS];  // of rows tid, tid + kScanThreads, ...: queries, keys, decode items
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int r = tid + i * kScanThreads;
+    lq[i] = lk[i] = n[i] = 0;
+    if (r < rows) {
+      lq[i] = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
+      lk[i] = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
+    }
+  }
+  auto streamed = [&](int i) { return few ? lq[i] > 0 : lq[i] == 1; };  // a row of decode items
   for (int b = tid; b <= kLenBuckets; b += kScanThreads) bucket[b] = 0;
   for (int i = tid; i < n_merge; i += kScanThreads) out.merge_count[i] = 0;
-  // Row r's queries and keys; the thread's first row stays in registers.
-  auto load_row = [&](int r) {
-    return make_int2(cu_q ? cu_q[r + 1] - cu_q[r] : 1, lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r]);
-  };
-  const int2 own = tid < rows ? load_row(tid) : make_int2(0, 0);
-  auto row_at = [&](int r) { return r == tid ? own : load_row(r); };
   // The decode rows' keys in all (fp32 is enough: the count is rounded up past its error) and at most.
   float keys = 0.f;
   int longest = 1, least = kMinSplit;  // least: keys per split at least
-  for (int r = tid; r < rows; r += kScanThreads) {
-    const int2 row = row_at(r);
-    if (streamed(row.x)) {
-      keys += (float)max(row.y, 0);
-      longest = max(longest, row.y);
-      if (few) least = max(least, least_split(row.y, row.x * group));
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i)
+    if (streamed(i)) {
+      keys += (float)max(lk[i], 0);
+      longest = max(longest, lk[i]);
+      if (few) least = max(least, least_split(lk[i], lq[i] * group));
     }
-  }
   keys = wave_sum(keys);
   longest = wave_max(longest);
-  least = wave_max(least);
+  if (few) least = wave_max(least);
   if ((tid & 63) == 0) {
     wave_keys[tid >> 6] = keys;
     wave_max_of[tid >> 6] = longest;
@@ -640,7 +647,6 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   }
   __syncthreads();
   keys = 0.f;
-  longest = 1;
 #pragma unroll
   for (int w = 0; w < kScanThreads / 64; ++w) {
     keys += wave_keys[w];
@@ -649,16 +655,17 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   }
   int split = split_keys(keys, longest, least, pieces);
   for (;;) {  // every thread leaves together: slots[rows] is the same for all, and split reaches the longest row
-    for (int r = tid; r < rows; r += kScanThreads) {
-      const int2 row = row_at(r);
-      const int lq = row.x, lk = row.y;
-      const int n = streamed(lq) ? (lk > split ? (lk + split - 1) / split : 1) : 0;  // the row's decode items
-      pre[r] = lq > 1 && !few ? (lq + qp - 1) / qp : 0;
-      full[r] = max(n - 1, 0);
-      slots[r] = n > 1 ? n * lq : 0;
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      const int r = tid + i * kScanThreads;
+      if (r >= rows) break;
+      n[i] = streamed(i) ? (lk[i] > split ? (lk[i] + split - 1) / split : 1) : 0;
+      pre[r] = lq[i] > 1 && !few ? (lq[i] + qp - 1) / qp : 0;
+      full[r] = max(n[i] - 1, 0);
+      slots[r] = n[i] > 1 ? n[i] * lq[i] : 0;
     }
     __syncthreads();
-    int* const sums[3] = {pre, full, slots};  // one pass over all: the kernel is its barriers
+    int* const sums[3] = {pre, full, slots};  // one pass over all
     block_scan<3>(sums, rows, wave_tot);
     if (slots[rows] <= max_slots || split >= longest) break;
     int64_t grown = max((int64_t)split * slots[rows] / max(max_slots, 1), (int64_t)split + split / 16);
@@ -670,15 +677,16 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     split = grown <= (1 << 30) ? (int)grown : INT32_MAX;
     __syncthreads();  // every thread has read slots[rows]
   }
-  for (int r = tid; r < rows; r += kScanThreads) {
-    const int2 row = row_at(r);
-    if (streamed(row.x)) {
-      const int lk = row.y;
-      const int n = lk > split ? (lk + split - 1) / split : 1;
-      atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
-      if (n > 1) out.part_base[r] = slots[r];
+  const float per_key = (float)kLenBuckets / (float)split;
+  int at[ROWS];  // the bucket of a row's last split
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i)
+    if (n[i] > 0) {
+      const int r = tid + i * kScanThreads;
+      at[i] = len_bucket(split - (lk[i] - (n[i] - 1) * split), per_key);
+      atomicAdd(&bucket[at[i]], 1);
+      if (n[i] > 1) out.part_base[r] = slots[r];
     }
-  }
   __syncthreads();
   if (tid < kLenBuckets) {  // wave 0: the bucket counts to offsets (one bucket per lane)
     static_assert(kLenBuckets == 64, "one wave scans the buckets");
@@ -707,15 +715,12 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     const int r = row_of(full, i);
     out.items[i] = make_int2(r, i - full[r]);
   }
-  for (int r = tid; r < rows; r += kScanThreads) {
-    const int2 row = row_at(r);
-    if (streamed(row.x)) {
-      const int lk = row.y;
-      const int n = lk > split ? (lk + split - 1) / split : 1;
-      const int pos = nfull + atomicAdd(&bucket[len_bucket(lk - (n - 1) * split, split)], 1);
-      if (pos < max_items) out.items[pos] = make_int2(r, n - 1);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i)
+    if (n[i] > 0) {
+      const int pos = nfull + atomicAdd(&bucket[at[i]], 1);
+      if (pos < max_items) out.items[pos] = make_int2(tid + i * kScanThreads, n[i] - 1);
     }
-  }
   if (tid == 0) {
     out.counts[kPlanDecodes] = min(nfull + npart, max_items);
     out.counts[kPlanPrompts] = min(npre, max_prompts);
@@ -1435,7 +1440,8 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
                       reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
     // Few-query items take a row's queries from cu_seqlens_q, so its partial slots are counted from there too, also in a
     // step that was said to have one query a row.
-    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(kScanThreads), 0, st,
+    auto* const plan = num_rows <= kScanThreads ? &plan_kernel<1> : &plan_kernel<kPlanMaxRows / kScanThreads>;
+    hipLaunchKernelGGL(plan, dim3(1), dim3(kScanThreads), 0, st,
                        kind.mixed || kind.few ? cu_seqlens_q : nullptr, seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
                        s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few, s.fewer_pieces,
                        p.group, (int32_t)s.merges, out);

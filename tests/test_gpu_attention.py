@@ -800,3 +800,34 @@ def test_launch_info_tells_the_keys_per_split(cuda, monkeypatch, heads, rows, ke
     items, split = plan_counts(ws, listed + info["decode_workgroups"] * info["kv_heads_per_item"] // hkv // groups)
     assert items == rows * -(-keys // split)
     assert info["keys_per_split"] == split
+
+
+@pytest.mark.parametrize("rows", [1, 63, 1023, 1024, 1025, 2049, 4096])
+def test_the_plan_lists_every_split_once_longest_first(cuda, monkeypatch, rows):
+    """Row counts on both sides of the plan's rows per thread: the decode items it left in the workspace are every split of
+    every row once, whole splits first and the others by decreasing length, a sixty-fourth of a split apart at most."""
+    hq, hkv, dim, bs = 8, 2, 64, 64
+    ws = guarded_workspace(monkeypatch, cuda)
+    gen = torch.Generator().manual_seed(rows)
+    lens = torch.randint(0, 700, (rows,), generator=gen, dtype=torch.int32)
+    lens[rows // 2] = 6400  # split up to 1024 rows
+    b = MI355XAttention(hq, dim, 1 / math.sqrt(dim), hkv)
+    kc, vc = (torch.zeros(100, bs, hkv, dim, dtype=torch.bfloat16, device=cuda) for _ in range(2))
+    ctx = Context(context_lens=lens.to(cuda),
+                  block_tables=torch.arange(100, dtype=torch.int32, device=cuda).expand(rows, 100).contiguous())
+    b.launch_trace = []
+    b.decode(torch.zeros(rows, hq, dim, dtype=torch.bfloat16, device=cuda), kc, vc, ctx)
+    torch.cuda.synchronize()
+    info = b.launch_trace[-1]
+    listed = -(-rows // 32) + rows
+    count, split = plan_counts(ws, listed + info["decode_workgroups"] * info["kv_heads_per_item"] // hkv)
+    items = ws[8 * listed:8 * (listed + count)].view(torch.int32).view(-1, 2).cpu()
+    splits = [max(1, -(-n // split)) for n in lens.tolist()]
+    assert sorted(map(tuple, items.tolist())) == [(r, s) for r, n in enumerate(splits) for s in range(n)]
+    keys = (lens[items[:, 0].long()] - items[:, 1] * split).clamp(max=split)
+    # A row's last split follows all whole ones, whatever its length.
+    last = items[:, 1] == torch.tensor(splits)[items[:, 0].long()] - 1
+    first_last = int(last.nonzero()[0])
+    assert last[first_last:].all()
+    lasts = keys[first_last:]
+    assert (lasts[1:] - lasts[:-1]).max() <= split / 64 + 1 if rows > 1 else True
