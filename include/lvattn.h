@@ -78,7 +78,8 @@ int lv_pack(const int32_t* num_cached, const int32_t* num_new, const int32_t* bl
 
 /* ---------------------------------------------------------------------------------------------------------
  * Scatter new keys/values into the paged cache. Replaces AttentionBackend.store_kvcache
- * (lean_vllm/attention/abstract.py:107-116; Triton store_kvcache_kernel, lean_vllm/attention/triton_cache.py:9-37,58-81).
+ * (lean_vllm/attention/abstract.py:107-116; Triton store_kvcache_kernel,
+ * lean_vllm/attention/triton_cache.py:9-37,58-81).
  * key/value: [T, Hkv, D] with unit dim stride and head stride D; row strides key_stride_t / value_stride_t.
  * Caches: logical (block, token, head, dim) addressed by their strides (an HND cache's transposed view works),
  * unit dim stride. slot_mapping[T]: slot = block * block_size + offset; -1 skips the token. Bit-exact copy. */
@@ -109,7 +110,9 @@ int lv_store_latents(const void* latent, int64_t latent_stride_t, int32_t num_to
  * split-K grid and workspace so a captured graph needs no length read back (the splits themselves are sized on the
  * device, from the lengths). num_tokens is T (it sizes the work list).
  * workspace: caller-owned device memory of at least lv_paged_attention_workspace_bytes(...) bytes for the same
- * arguments; its contents need no initialisation.
+ * arguments; its contents need no initialisation. The query knows neither the schedule nor the longest row's queries:
+ * it covers the partials of split prompt tiles (up to 43 MiB) and of few-query items (up to 14 MiB) where the shape may
+ * take them.
  * schedule (a step with prompt rows): LV_SCHEDULE_OVERLAP runs the prompt tiles on part of the CUs beside the
  * decode rows' streaming (a second stream, joined back into `stream` by events); LV_SCHEDULE_SERIAL runs the
  * prompt tiles on the whole GPU, then the decode rows -- the faster choice when the decode rows' bytes take less
@@ -155,7 +158,7 @@ int lv_paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h, co
 #define LV_KERNEL_NONE 0
 #define LV_KERNEL_DECODE_LIST 1    /* one workgroup per decode item of the work list */
 #define LV_KERNEL_DECODE_BESIDE 2  /* persistent grid taking decode items by ticket, beside prompt_overlap */
-#define LV_KERNEL_DECODE_GRID 3    /* one workgroup per (row, kv head, head group), unsplit; no work list (> 4096 rows) */
+#define LV_KERNEL_DECODE_GRID 3    /* one workgroup per (row, kv head, head group), unsplit; no list (> 4096 rows) */
 #define LV_KERNEL_PROMPT_LIST 4    /* one workgroup per prompt item, on the whole GPU */
 #define LV_KERNEL_PROMPT_OVERLAP 5 /* persistent prompt workgroups on part of the CUs, beside the decode items */
 #define LV_KERNEL_MIXED_SMALL 6    /* prompt and decode items of a small mixed step in one launch */
@@ -182,17 +185,16 @@ int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_tokens, int32_t
  * callers that cannot call hipMalloc -- code under HIP graph capture, tight serving loops, harnesses that forbid
  * allocation. The work list, its counters and the split-K partials live in a static device array of
  * LV_STATIC_WORKSPACE_BYTES that each GPU the library runs on holds until the process ends; a step needing more
- * (the split-K sizing keeps steps of up to 4096 rows at any context length under 9 MiB, of few queries per row under
- * 15 MiB) is refused with LV_EINVAL; the partials of a step of few prompt tiles, whose keys are split over workgroups, lie
- * in a second array of 43 MiB, which holds any such step's. The kernels clear what must start at zero themselves (the plan
- * kernel zeroes the persistent grid's ticket and the split rows' merge counters), so no memset is recorded
- * into a captured graph. Every call
- * on one GPU shares that GPU's array, which keeps the last call's contents: calls that overlap on one GPU (two
- * streams, two host threads, or a graph replay beside an eager call) race. Results equal lv_paged_attention's for
- * the same arguments. Set-up: the first call on a device resolves the arrays' addresses there and creates the
- * device's second stream and its two fork/join events (which lv_paged_attention creates at its first overlapped
- * step); no device memory is allocated, and later calls create nothing. A caller that captures graphs makes one
- * call on each device before capturing. */
+ * (the split-K sizing keeps steps of up to 4096 rows at any context length under 9 MiB, of few queries per row
+ * under 15 MiB) is refused with LV_EINVAL; the partials of a step of few prompt tiles, whose keys are split over
+ * workgroups, lie in a second array of 43 MiB, which holds any such step's. The kernels clear what must start at
+ * zero themselves (the plan kernel zeroes the persistent grid's ticket and the split rows' merge counters), so no
+ * memset is recorded into a captured graph. Every call on one GPU shares that GPU's array, which keeps the last
+ * call's contents: calls that overlap on one GPU (two streams, two host threads, or a graph replay beside an eager
+ * call) race. Results equal lv_paged_attention's for the same arguments. Set-up: the first call on a device
+ * resolves the arrays' addresses there and creates the device's second stream and its two fork/join events (which
+ * lv_paged_attention creates at its first overlapped step); no device memory is allocated, and later calls create
+ * nothing. A caller that captures graphs makes one call on each device before capturing. */
 #define LV_STATIC_WORKSPACE_BYTES (16u << 20)
 int lv_paged_attention_static(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_cache,
                               const void* v_cache, int64_t cache_stride_block, int64_t cache_stride_token,

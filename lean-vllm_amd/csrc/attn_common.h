@@ -125,7 +125,8 @@ __device__ __forceinline__ int swz(int r, int c) {
 // lane loading from its key's page).
 template <typename T, int DQK, int DV, bool PREFETCH = true, bool OPAQUE_TID = false, int RING = 0, int WAVES = 4,
           bool CTX = false, int TP = 1, bool SPLIT = false>
-__device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, char* smem, int piece = 0, int slot = 0) {
+__device__ void prefill_item(const AttnParams& p, int row, int qtile, int kvh, char* smem, int piece = 0,
+                             int slot = 0) {
   using E = Elem<T>;
   constexpr int KS = DQK / 32;  // MFMA k-steps over the q.k width
   constexpr int DB = DV / 16;   // 16-dim blocks of the output

@@ -1,11 +1,11 @@
 // Paged attention of rows with few queries on MFMA: drafted tokens (2 to 16 queries a row), and decode rows whose GQA
 // group is not 1, 2 or 4 query heads.
 //
-// An item is (row, split, kv head): all of the row's (position, head) query rows of one GQA group, up to 64, against the
-// keys [split * S, (split + 1) * S) of the row, so the keys and values are read from memory once. Bound by HBM: 16 to 64
-// query rows do 16 to 64 flops a byte. The VALU decode item takes one query and 1, 2 or 4 heads of a group, and would
-// read the keys once for each such share; the MFMA prompt item holds 128 query rows and walks the row's keys in one
-// workgroup, which leaves most of the chip idle on a few long rows.
+// An item is (row, split, kv head): all of the row's (position, head) query rows of one GQA group, up to 64, against
+// the keys [split * S, (split + 1) * S) of the row, so the keys and values are read from memory once. Bound by HBM:
+// 16 to 64 query rows do 16 to 64 flops a byte. The VALU decode item takes one query and 1, 2 or 4 heads of a group,
+// and would read the keys once for each such share; the MFMA prompt item holds 128 query rows and walks the row's
+// keys in one workgroup, which leaves most of the chip idle on a few long rows.
 //
 // Each of a workgroup's four waves takes every 4th tile of the item's keys through a private two-stage LDS ring, filled
 // straight from memory; no barrier until the waves merge. A tile's keys are refilled as soon as their scores are in
@@ -90,7 +90,8 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
 
   // Pages of the wave's next 64 tiles, one tile per lane (a 16-key block lies in one page).
   int pages[KB];
-  auto block_start = [&](int t0, int b) { return t0 + 16 * b < kend ? t0 + 16 * b : t0; };  // a block past the end: block 0
+  // A block past the end: block 0.
+  auto block_start = [&](int t0, int b) { return t0 + 16 * b < kend ? t0 + 16 * b : t0; };
   auto load_pages = [&](int t) {
     const int t0 = min(k0 + KT * WT * (t + lane), kend - 1);
 #pragma unroll
@@ -106,8 +107,8 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
     for (int b = 0; b < KB; ++b) {
       const int s = block_start(t0, b);
       const int pg = (int)p.bs.div(s);
-      off[b] = (int64_t)__builtin_amdgcn_readlane(pages[b], t & 63) * p.c_sb + (int64_t)(s - pg * (int)p.bs.d) * p.c_st +
-               (int64_t)wh * p.c_sh;
+      off[b] = (int64_t)__builtin_amdgcn_readlane(pages[b], t & 63) * p.c_sb +
+               (int64_t)(s - pg * (int)p.bs.d) * p.c_st + (int64_t)wh * p.c_sh;
     }
   };
   // The keys or the values of tile t, located before. Keys past the item's end load its last key (finite; weight 0).
@@ -127,7 +128,8 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
     }
   };
 
-  for (int q0 = 0; q0 < qrows; q0 += 16 * NB + SET_ROWS) {  // one pass, unless the row has more query rows than the launch expects
+  // One pass, unless the row has more query rows than the launch expects.
+  for (int q0 = 0; q0 < qrows; q0 += 16 * NB + SET_ROWS) {
     // Query rows q0 + SET_ROWS set + 16 nb + n: Q^T operands (dims 32 k + 8 j4 .. + 7) and the keys each sees.
     int lim[NB];
     u32x4 qb[NB][KS];
@@ -220,8 +222,9 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
         }
       }
       // P^T operands: k slots 4 j4 .. + 3 (and, of 32 keys, 16 + 4 j4 .. + 3). Probabilities as a sum of two 16-bit
-      // numbers, the second MFMA being free beside the stream: one alone would leave a rounding as large as the output's
-      // (against 64 bits 2.3e-3 in bf16, where the VALU item, whose maxima are exactly 1, has 2.1e-3; so 1.7e-3).
+      // numbers, the second MFMA being free beside the stream: one alone would leave a rounding as large as the
+      // output's (against 64 bits 2.3e-3 in bf16, where the VALU item, whose maxima are exactly 1, has 2.1e-3; so
+      // 1.7e-3).
       uint32_t pb[NB][2 * KB], pl[NB][2 * KB];
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) {
@@ -256,8 +259,10 @@ __device__ __forceinline__ void few_item(const AttnParams& p, int row, int split
           const u32x4 a = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll
           for (int nb = 0; nb < NB; ++nb) {
-            o[nb][b] = E::mfma16x16x32(a, u32x4{pb[nb][0], pb[nb][1], pb[nb][2 * KB - 2], pb[nb][2 * KB - 1]}, o[nb][b]);
-            o[nb][b] = E::mfma16x16x32(a, u32x4{pl[nb][0], pl[nb][1], pl[nb][2 * KB - 2], pl[nb][2 * KB - 1]}, o[nb][b]);
+            const u32x4 ph = {pb[nb][0], pb[nb][1], pb[nb][2 * KB - 2], pb[nb][2 * KB - 1]};
+            const u32x4 pr = {pl[nb][0], pl[nb][1], pl[nb][2 * KB - 2], pl[nb][2 * KB - 1]};
+            o[nb][b] = E::mfma16x16x32(a, ph, o[nb][b]);
+            o[nb][b] = E::mfma16x16x32(a, pr, o[nb][b]);
           }
         }
       }

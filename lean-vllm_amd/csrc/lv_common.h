@@ -243,11 +243,12 @@ __device__ inline int wave_incl_scan(int x) {
   return x;
 }
 
-// Exclusive prefix sums of N arrays a[i][0, n) in LDS, in place, by a block of kScanThreads threads; a[i][n] receives the
-// total. wave_tot holds kScanThreads / 64 ints of LDS per array. Every thread of the block must call it, after a barrier
-// that follows the last write of the arrays (a thread's chunk holds entries other threads wrote once n > kScanThreads).
-// Each thread scans its chunk, each wave its threads' chunk totals; every thread then sums the wave totals before its own
-// (16 broadcast LDS reads, issued together) instead of one thread scanning them in sequence between two more barriers.
+// Exclusive prefix sums of N arrays a[i][0, n) in LDS, in place, by a block of kScanThreads threads; a[i][n] receives
+// the total. wave_tot holds kScanThreads / 64 ints of LDS per array. Every thread of the block must call it, after a
+// barrier that follows the last write of the arrays (a thread's chunk holds entries other threads wrote once n >
+// kScanThreads). Each thread scans its chunk, each wave its threads' chunk totals; every thread then sums the wave
+// totals before its own (16 broadcast LDS reads, issued together) instead of one thread scanning them in sequence
+// between two more barriers.
 constexpr int kScanThreads = 1024;
 template <int N>
 __device__ inline void block_scan(int* const (&a)[N], int n, int (&wave_tot)[N][kScanThreads / 64]) {
@@ -288,9 +289,9 @@ __device__ inline void block_scan(int* a, int n, int (&wave_tot)[1][kScanThreads
   block_scan<1>(one, n, wave_tot);
 }
 
-// The maximum that partial sums are rescaled to when they merge. Where no partial saw a key every maximum is -inf, and 0
-// stands in for it: each weighs exp2(-inf) = 0. A partial of NaN scores may have a maximum of -inf as well; its NaN sum
-// then reaches the result, which skipping the merge would turn into zeros.
+// The maximum that partial sums are rescaled to when they merge. Where no partial saw a key every maximum is -inf,
+// and 0 stands in for it: each weighs exp2(-inf) = 0. A partial of NaN scores may have a maximum of -inf as well; its
+// NaN sum then reaches the result, which skipping the merge would turn into zeros.
 __device__ __forceinline__ float merge_base(float m) { return m == -INFINITY ? 0.f : m; }
 // 1 / a softmax's denominator: 0 where no key was seen, NaN where a score was not a number.
 __device__ __forceinline__ float inv_sum(float l) { return l > 0.f || l != l ? 1.f / l : 0.f; }

@@ -67,10 +67,10 @@ constexpr int kDmaRowSlots = kLatChunks + 2;            // 16-byte slots per LDS
 constexpr int kDmaStageSlots = kDmaTile * kDmaRowSlots;  // 1184
 constexpr int kDmaInstr = (kDmaStageSlots + 63) / 64;   // 64-lane loads per stage: 19, 5 per wave (4 for wave 3)
 constexpr int kDmaStageElems = kDmaStageSlots * 8;
-static_assert(kDmaRowSlots * 8 == kMlaPitch, "one LDS row pitch for both variants");
+static_assert(kDmaRowSlots * 8 == kMlaPitch, "the slots make up the LDS row pitch");
 static_assert(kDmaInstr == 19, "the stage waits count 5 loads for waves 0-2 and 4 for wave 3");
 
-// Wait until at most `ahead` (<= 6) stages of this wave's loads (5 per stage, 4 for wave 3) are outstanding, then meet
+// Wait until at most `ahead` (<= 2) stages of this wave's loads (5 per stage, 4 for wave 3) are outstanding, then meet
 // the other waves. No fence: the stage's LDS writes are exactly the loads waited for, and a fence would wait for
 // the stages still in flight as well.
 #define LV_WAIT_BARRIER(N) asm volatile("s_waitcnt vmcnt(" #N ")\n\ts_barrier" ::: "memory")
@@ -79,21 +79,13 @@ __device__ __forceinline__ void dma_stage_barrier(int ahead, int wave) {
     switch (ahead) {
       case 0: LV_WAIT_BARRIER(0); break;
       case 1: LV_WAIT_BARRIER(5); break;
-      case 2: LV_WAIT_BARRIER(10); break;
-      case 3: LV_WAIT_BARRIER(15); break;
-      case 4: LV_WAIT_BARRIER(20); break;
-      case 5: LV_WAIT_BARRIER(25); break;
-      default: LV_WAIT_BARRIER(30); break;
+      default: LV_WAIT_BARRIER(10); break;
     }
   } else {
     switch (ahead) {
       case 0: LV_WAIT_BARRIER(0); break;
       case 1: LV_WAIT_BARRIER(4); break;
-      case 2: LV_WAIT_BARRIER(8); break;
-      case 3: LV_WAIT_BARRIER(12); break;
-      case 4: LV_WAIT_BARRIER(16); break;
-      case 5: LV_WAIT_BARRIER(20); break;
-      default: LV_WAIT_BARRIER(24); break;
+      default: LV_WAIT_BARRIER(8); break;
     }
   }
 }
@@ -251,43 +243,46 @@ __global__ __launch_bounds__(256) void mla_decode_dma_kernel(MlaParams p) {
 // ---------------------------------------------------------------------------------------------------------
 // Balanced schedule over equal runs of stages, for pages whose size is a multiple of 16 latents.
 //
-// A row's columns are its (query j, head) pairs, c = j * heads + head. Unit u = (row, tile of 16 NB columns), u = row *
-// tiles + tile, needs T_u = ceil(L_u / 32) stages of 32 latents (L_u: the latents its last query sees; a column of an
-// earlier query masks its last ones), and kRunEnter more places ahead of them for its queries and its output, which cost
-// a run about as much. Laid end to end (prefix P_u) the units' stages are cut into equal runs, one per
-// workgroup of a grid that fills the GPU once; every workgroup streams its run through an LDS ring, each unit it enters
-// preceded by a stage holding that unit's query rows. A unit that lies wholly inside one run is finished in place. A unit cut by run boundaries leaves (o / l, log2 l + m) per column in slot 0 (the run's
-// first unit) or slot 1 (its last unit) of every run it touches, and mla_run_merge_kernel combines them; that kernel also
-// writes the zero output of columns that see no latents. Every run does equal work, whatever the spread of row lengths,
-// and partials are written only where a row crosses a run boundary.
+// A row's columns are its (query j, head) pairs, c = j * heads + head. Unit u = (row, tile of 16 NB columns), u = row
+// * tiles + tile, needs T_u = ceil(L_u / 32) stages of 32 latents (L_u: the latents its last query sees; a column of
+// an earlier query masks its last ones), and kRunEnter more places ahead of them for its queries and its output,
+// which cost a run about as much. Laid end to end (prefix P_u) the units' stages are cut into equal runs, one per
+// workgroup of a grid that fills the GPU once; every workgroup streams its run through an LDS ring, each unit it
+// enters preceded by a stage holding that unit's query rows. A unit that lies wholly inside one run is finished in
+// place. A unit cut by run boundaries leaves (o / l, log2 l + m) per column in slot 0 (the run's first unit) or slot
+// 1 (its last unit) of every run it touches, and mla_run_merge_kernel combines them; that kernel also writes the zero
+// output of columns that see no latents. Every run does equal work, whatever the spread of row lengths, and partials
+// are written only where a row crosses a run boundary.
 //
 // NB is 1 for rows of up to 16 columns, else 2: drafts and heads past 16 share the latents that a workgroup has in LDS
 // instead of streaming them again. (Four blocks spill: 64 heads 1047 us against 458.)
 //
-// One workgroup of 8 waves per CU, a ring of three 36 KB stages, two in flight. Wave (lb, cb) of the first 2 NB computes
-// the scores of 16 latents for 16 columns over the whole K = 576 (its Q^T in registers) and leaves their probabilities in
-// LDS as the P^T operand; the other waves meanwhile issue the stage loads; after a barrier every wave adds P.V for 64 of
-// the 512 output dims and all columns, V^T from the transposing read. Two barriers per 32 latents. The max of a column is
-// shared: a score past it by more than kRescaleSlack makes the workgroup take the stage's maxima from LDS, rescale and
-// write the probabilities again (rare: the first stage of a unit, seldom another).
+// One workgroup of 8 waves per CU, a ring of three 36 KB stages, two in flight. Wave (lb, cb) of the first 2 NB
+// computes the scores of 16 latents for 16 columns over the whole K = 576 (its Q^T in registers) and leaves their
+// probabilities in LDS as the P^T operand; the other waves meanwhile issue the stage loads; after a barrier every
+// wave adds P.V for 64 of the 512 output dims and all columns, V^T from the transposing read. Two barriers per 32
+// latents. The max of a column is shared: a score past it by more than kRescaleSlack makes the workgroup take the
+// stage's maxima from LDS, rescale and write the probabilities again (rare: the first stage of a unit, seldom
+// another).
 //
 // Bound by HBM up to 32 columns (a build without the scores and P.V streams 128 rows of 1024-16384 latents in 201 us,
-// 6.55 TB/s; the scores' serial chain through LDS and the two barriers are what is left). Against the schedule before,
-// two workgroups of 4 waves per CU with a 16-latent stage each, every query and every 16 heads a unit of their own:
-// 128 rows, 16 heads 216 us (215.4), 32 heads 229 (426), 64 heads 454 (850), 128 heads 890 (1670); two layers of 20 rows,
-// 1024-8192 latents, 16 heads, 2 queries 73 us (108), 3 queries 104 (138), 128 heads 171 (298); 4 rows 57 (70).
+// 6.55 TB/s; the scores' serial chain through LDS and the two barriers are what is left). Against the schedule
+// before, two workgroups of 4 waves per CU with a 16-latent stage each, every query and every 16 heads a unit of
+// their own: 128 rows, 16 heads 216 us (215.4), 32 heads 229 (426), 64 heads 454 (850), 128 heads 890 (1670); two
+// layers of 20 rows, 1024-8192 latents, 16 heads, 2 queries 73 us (108), 3 queries 104 (138), 128 heads 171 (298); 4
+// rows 57 (70).
 
 constexpr int kRunTile = 32;         // latents per stage
-constexpr int kRunEnter = 3;         // places of a unit's start (0 / 1 / 2 / 3: 128 rows 217.5 / 216.4 / 216.9 / 216.0 us, 60 rows
-                                     // 136.6 / 135.1 / 134.4 / 133.2)
+constexpr int kRunEnter = 3;         // places of a unit's start (0 / 1 / 2 / 3: 60 rows 136.6 / 135.1 / 134.4 / 133.2
+                                     // us, 128 rows 217.5 / 216.4 / 216.9 / 216.0, within the spread of runs)
 constexpr int kRunMin = 4;           // places per run at least (past a unit's start)
 constexpr int kRunStages = 3;        // ring depth (four stream no faster)
 constexpr int kRunWaves = 8;
 constexpr int kRunsPerCU = 1;        // run workgroups per CU
 enum : int { kGrow = 1, kUnseen = 2 };
 constexpr int kRunMaxUnits = 8192;   // units the in-kernel scan serves
-constexpr int kRunRow = kLatent;     // LDS row pitch in elements: no padding, 16-byte chunk c of row r at c ^ (r & 6), so
-                                     // that operand and transposing reads meet no bank conflicts
+constexpr int kRunRow = kLatent;     // LDS row pitch in elements: no padding, 16-byte chunk c of row r at c ^ (r & 6),
+                                     // so that operand and transposing reads meet no bank conflicts
 constexpr int kRunElems = kRunTile * kRunRow;
 constexpr int kRunLoads = kRunTile * kLatChunks / 64;  // 64-lane loads per stage, 18 per 16 rows
 
@@ -432,8 +427,8 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
         __builtin_amdgcn_readfirstlane(first[2]));
   cons = prod;
 
-  // Loader wave lw's loads j = lw + LW i of a stage's 36: each lies in 16-row block j / 18, slot 64 (j % 18) + lane of it
-  // holding position slot % 72 of its row slot / 72, so the chunk that belongs there.
+  // Loader wave lw's loads j = lw + LW i of a stage's 36: each lies in 16-row block j / 18, slot 64 (j % 18) + lane
+  // of it holding position slot % 72 of its row slot / 72, so the chunk that belongs there.
   const bool loader = wave >= SW;
   const int lw = loader ? wave - SW : 0;
   // Whether load i of this wave lies in the second block: known for most i, whatever the wave.
@@ -518,8 +513,8 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       advance(prod);
       ++issued;
     };
-    // With the value reads below before it, 128 rows of 16 heads measured 218.5 -> 217.5 us; after it, two column blocks
-    // 77.8 -> 74.8.
+    // With the value reads below before it, one column block: 128 rows of 16 heads 207.7 -> 205.0 us, 60 rows 98.2 ->
+    // 97.1, 256 shorter rows 121.8 -> 120.9, 20 rows 30.2 -> 30.4; after it, two column blocks: 77.8 -> 74.8.
     constexpr bool kValuesFirst = NB == 1;
     if (cons.t < 0 || !kValuesFirst) refill();
     const uint16_t* stage = ring + (k % kRunStages) * kRunElems;
@@ -643,9 +638,9 @@ __global__ __launch_bounds__(64 * kRunWaves, 2) void mla_run_kernel(MlaParams p)
       get_probabilities();
     }
     lsum += psum;
-    // Latents from `common` on are drafts that the unit's first query does not see. Its weights there are 0, but a value
-    // that is no number would reach its sums all the same: where a stage has one, such latents are left out of the product
-    // and added to the columns that see them one by one.
+    // Latents from `common` on are drafts that the unit's first query does not see. Its weights there are 0, but a
+    // value that is no number would reach its sums all the same: where a stage has one, such latents are left out of
+    // the product and added to the columns that see them one by one.
     const int common = cons.lk - later;
     if (state & kUnseen) {
 #pragma unroll
@@ -949,9 +944,10 @@ extern "C" int lv_mla_decode(const void* q, int64_t q_stride_t, int64_t q_stride
 
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const bool one_page = block_size % kDmaTile == 0 && p.c_st * kDmaTile < ((int64_t)1 << 31);
-  // The run schedule counts stages in 32 bits on the device.
-  const int64_t stage_bound = (int64_t)s.units * (((int64_t)std::max(max_seqlen_k, 1) + kDmaTile - 1) / kDmaTile);
-  if (one_page && s.units <= kRunMaxUnits && stage_bound < ((int64_t)1 << 30)) {
+  // The run schedule counts places in 32 bits on the device.
+  const int64_t keys = std::max(max_seqlen_k, 1);
+  const int64_t places = (int64_t)s.units * ((keys + kRunTile - 1) / kRunTile + kRunEnter);
+  if (one_page && s.units <= kRunMaxUnits && places < ((int64_t)1 << 30)) {
     p.units = s.units;
     p.tiles = s.tiles;
     p.part_lse = reinterpret_cast<float*>(ws + s.lse_off);

@@ -22,7 +22,7 @@
 
 namespace lv {
 
-constexpr int kTile = 16;          // decode tokens per tile; block sizes are multiples of 16, so a tile sits in one block
+constexpr int kTile = 16;           // decode tokens per tile; block sizes are multiples of it: a tile is in one block
 constexpr int kPlanMaxRows = 4096;  // rows of a step with prompts (the work-list scan lives in LDS)
 
 constexpr int kPromptRing = 2;        // LDS stages of the prompt tiles' ring
@@ -36,12 +36,13 @@ constexpr int kPieceKeys = 1024;      // and keys per piece at least, of the lon
 constexpr int kSplitTarget = 4096;    // decode items (x kv heads x query-head groups) a step with split rows aims for
 constexpr int kMaxRowSplits = 128;    // and splits per row on average at most
 constexpr int kMinSplit = 256;        // keys per decode item at least
-constexpr int kFewRound = 512;        // workgroups that the GPU holds at once, two per CU
-// Pieces of a step's split prompt items at most: n items are cut into (kFewRound + n / 2) / n >= 2 pieces each, so n is at
-// most 2/3 kFewRound, and n pieces of each come to at most kFewRound + n / 2.
-constexpr int kMaxPieces = kFewRound * 4 / 3;
-constexpr int64_t kFewPartBytes = 14 << 20;  // partials of a step of few queries per row at most (within the static workspace)
 constexpr int kSplitStep = 64;        // and a multiple of this: one tile of every wave
+constexpr int kFewRound = 512;        // workgroups that an MI355X holds at once, two per CU (kMaxPieces is its bound)
+// Pieces of a step's split prompt items at most: n items are cut into (kFewRound + n / 2) / n >= 2 pieces each, so n
+// is at most 2/3 kFewRound, and n pieces of each come to at most kFewRound + n / 2.
+constexpr int kMaxPieces = kFewRound * 4 / 3;
+// Partials of a step of few queries per row at most (within the static workspace).
+constexpr int64_t kFewPartBytes = 14 << 20;
 constexpr int kSmallStepRounds = 8;   // a mixed step of at most this many GPU-fulls of workgroups is one launch
 
 // ---------------------------------------------------------------------------------------------------------
@@ -425,12 +426,12 @@ __global__ __launch_bounds__(256, 2) void prompt_list_kernel(AttnParams p) {
 }
 
 // A few prompt items with long key ranges (a chunk late in a long prompt), each split over its keys into p.pieces
-// workgroups, and the merge of their partials: one thread per four dims of a query row.
-// MFMA-bound, as the unsplit items, but 128 of those leave half the CUs without one and every SIMD of the others with one
-// wave. 32/8 heads, d128, a chunk on a 24,576-token prefix: 512 tokens 505 -> 222 us (412 -> 940 TFLOP/s), 32 tokens
-// 494 -> 84, 1024 tokens 517 -> 417; on 16-token pages 618 -> 235; 256 tokens on 4096 97 -> 47. (Pieces of at least
-// kPieceKeys keys: 512 tokens on 2048 62 -> 53.) A step whose items come to three quarters of the GPU's workgroups stays
-// whole.
+// workgroups, and the merge of their partials: one thread per four dims of a query row. MFMA-bound, as the unsplit
+// items, but 128 of those leave half the CUs without one and every SIMD of the others with one wave. 32/8 heads,
+// d128, a chunk on a 24,576-token prefix: 512 tokens 505 -> 222 us (412 -> 940 TFLOP/s), 32 tokens 494 -> 84, 1024
+// tokens 517 -> 417; on 16-token pages 618 -> 235; 256 tokens on 4096 97 -> 47. (Pieces of at least kPieceKeys keys:
+// 512 tokens on 2048 62 -> 53.) The number of pieces is the step's, by its longest row; a piece is that part of its
+// own item's tiles, so a short row's or an early tile's pieces are shorter, or empty.
 template <typename T, int D, int TP>
 __global__ __launch_bounds__(256, 2) void prompt_split_kernel(AttnParams p) {
   constexpr int RING = kRingOf<TP>;
@@ -560,14 +561,14 @@ __device__ inline int len_bucket(int short_of, float per_key) {
 // that a step is cut into about the same number of items whatever its lengths (at most pieces + rows). The caller's
 // bound on key lengths only sizes the buffers: a captured graph's bound is the longest context it may ever serve, and
 // a batch of a few rows far apart in length has most of its keys in one of them. pieces 0: rows are not split, and
-// one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]. few: rows of
-// several queries are streamed as decode items too, one slot per query and split.
+// one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]. few: rows
+// of several queries are streamed as decode items too, one slot per query and split.
 //
-// few: a row's merge is one workgroup's work, and takes as long as its splits where they hold `least` keys: n splits of lk
-// keys take lk / n keys' stream (12 KB a microsecond) and lq G D n / 512 loads a thread (19 a microsecond), equal at
-// lk / n = sqrt(0.3 lk lq G). One row of 64,000 keys, 128 splits and with this bound: 8/2 heads, d128, 16 queries 160 -> 114
-// us (56 splits); 16/1 heads, 4 queries, two rows 157 -> 113; 40/1 heads, one query 114 -> 91. It is below
-// kMinSplit, and changes nothing, while lk lq G < 218,000 (4 queries of group 4 on 13,000 keys).
+// few: a row's merge is one workgroup's work, and takes as long as its splits where they hold `least` keys: n splits
+// of lk keys take lk / n keys' stream (12 KB a microsecond) and lq G D n / 512 loads a thread (19 a microsecond),
+// equal at lk / n = sqrt(0.3 lk lq G). One row of 64,000 keys, 128 splits and with this bound: 8/2 heads, d128, 16
+// queries 160 -> 114 us (56 splits); 16/1 heads, 4 queries, two rows 157 -> 113; 40/1 heads, one query 114 -> 91. It
+// is below kMinSplit, and changes nothing, while lk lq G < 218,000 (4 queries of group 4 on 13,000 keys).
 //
 // A split that needs more slots than there are grows until they fit: a long row of more queries than the others (to
 // fewer_pieces first), more queries or lengths than the caller said (by the slots' ratio, a sixteenth at least).
@@ -593,10 +594,10 @@ struct PlanOut {
   int32_t* merge_count;
 };
 
-// ROWS: rows a thread at most. The kernel is its barriers, its round trips to memory and its code, which a step's one plan meets
-// cold: the rows' loads are issued together, once, and all that is known of a row stays in registers. 3 / 256 / 1024 / 4096
-// rows of a decode step 6.0 / 6.4 / 7.4 / 12.8 us with later rows loaded again in each pass and 64-bit bucket divisions, 5.4
-// / 5.9 / 6.6 / 10.4 so (with splits of a size fixed on the host 5.6 / 4.5 / 5.0 / 8.9).
+// ROWS: rows a thread at most. The kernel is its barriers, its round trips to memory and its code, which a step's one
+// plan meets cold: the rows' loads are issued together, once, and all that is known of a row stays in registers. 3 /
+// 256 / 1024 / 4096 rows of a decode step 6.0 / 6.4 / 7.4 / 12.8 us with later rows loaded again in each pass and
+// 64-bit bucket divisions, 5.4 / 5.9 / 6.6 / 10.4 so (with splits of a size fixed on the host 5.6 / 4.5 / 5.0 / 8.9).
 template <int ROWS>
 __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __restrict__ cu_q,
                                                             const int32_t* __restrict__ lens_k,
@@ -697,8 +698,8 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   }
   __syncthreads();
   const int npre = pre[rows], nfull = full[rows], npart = bucket[kLenBuckets];
-  // Prompt items and full splits, one thread each (a few long rows hold hundreds: a thread per row would write them one by
-  // one, 9 us for seven prompts' 260 items, 5 so).
+  // Prompt items and full splits, one thread each (a few long rows hold hundreds: a thread per row would write them
+  // one by one, 9 us for seven prompts' 260 items, 5 so).
   auto row_of = [&](const int* before, int i) {  // the last row with at most i items before its own
     int lo = 0, hi = rows - 1;
     while (lo < hi) {
@@ -751,11 +752,19 @@ static int pick_gs(int group) {
   return 1;
 }
 
-// Queries per row that a step of few queries may have (0: the GQA group is too wide). Past 32 query rows per kv head an
-// item at D = 128 streams its keys into LDS twice, and the prompt items (128 query rows, unsplit) are as fast once they
-// fill the GPU: 16 queries a row of 32/8 heads, two layers, 8 rows 162 against 398 us, 48 rows 758 against 492. At D = 64
-// it stays with one copy: 48 rows 231 against 308 us, 8 rows 83 against 256. (A decode row of a group that wide is a few-query
-// row all the same: the VALU items would read its keys once per four heads.)
+// Queries per row that a step of few queries may have (0: the GQA group is too wide). Past 32 query rows per kv head
+// an item at D = 128 streams its keys into LDS twice; its steps are few-query steps while rows x kv heads are at most
+// a quarter of the GPU's workgroups. At D = 64 it stays with one copy: two layers, 16 queries a row of 32/8 heads, 48
+// rows 231 against 308 us on the prompt items, 8 rows 83 against 256 (unsplit).
+//
+// What the line weighs, D = 128, 16 queries a row of 32/8 heads, us a layer, few-query items / split prompt items,
+// contexts of 2K, 8K, 32K: 1 row 29 / 55, 53 / 42, 94 / 114; 4 rows 33 / 55, 71 / 45, 223 / 122; 8 rows 46 / 56, 121
+// / 76, 423 / 243; 16 rows 70 / 57, 221 / 123, 830 / 426. One row of 64,000 keys among short ones (8/2 heads): 114 /
+// 212. Few-query items win on short contexts and where the long rows are one or two; a step of equal rows past 4K
+// would be faster on the prompt items, but the host knows the bound on the contexts, not the contexts.
+//
+// (A decode row of a group that wide is a few-query row all the same: the VALU items would read its keys once per
+// four heads.)
 static int few_queries(int64_t rows, int32_t hkv, int32_t d, int group) {
   const int most = d == 64 || group > 32 || rows * hkv <= kFewRound / 4 ? kFewMaxRows : kFewMaxRows / 2;
   return std::min(kFewMaxQueries, most / group);
@@ -772,22 +781,24 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   // Rows split only in a listed step (whose workspace holds the partial slots and merge counters). The number of pieces
   // weighs the list's balance against the merge of a row, its round trips past the L2 after its last split.
   //
-  // Where unsplit items fill the GPU (VALU: more than half the items aimed for; few queries: more than one round), the
-  // longest-first list balances them as they are, and only a row of more than two workgroups' share of all keys is split.
+  // Where unsplit items fill the GPU (VALU: more than half the items aimed for; few queries: more than one round),
+  // the longest-first list balances them as they are, and only a row of more than two workgroups' share of all keys
+  // is split.
   //
   // VALU decode items: 4096 one-head items for many rows, fewer for a few long ones. 32/8 heads, d128, contexts
-  // U[32K, 128K], 1024 / 2048 / 3072 / 4096 items (before, 4096 of sizes set by the longest row): 1 row
-  // 93 / 113 / 125 / 132 us (166), 2 rows 174 / 181 / 192 / 190 (219), 3 rows 252 / 250 / 256 / 261 (272), 8 rows
-  // 594 / 557 / 567 / 569 (585), 24 rows 1494 / 1399 / 1372 / 1384 (1452); 48 rows U[4K, 64K] 1431 / 1283 / 1237 / 1241 (1309).
+  // U[32K, 128K], 1024 / 2048 / 3072 / 4096 items (before, 4096 of sizes set by the longest row): 1 row 93 / 113 /
+  // 125 / 132 us (166), 2 rows 174 / 181 / 192 / 190 (219), 3 rows 252 / 250 / 256 / 261 (272), 8 rows 594 / 557 /
+  // 567 / 569 (585), 24 rows 1494 / 1399 / 1372 / 1384 (1452); 48 rows U[4K, 64K] 1431 / 1283 / 1237 / 1241 (1309):
+  // the lines at 2 and 16 rows lie between measured counts, and 3072 items for more rows would be within 1%.
   //
-  // Steps of few queries (few_query.hip, two workgroups per CU whatever the group): a full piece is one workgroup's share
-  // of all keys, so the full pieces run in one round and the rows' remainders pack beside them; up to kFewRound / 8
-  // rows' remainders are counted in, so that all run at once. More pieces cost more than they balance, their partials
-  // being several query rows each. 32/8 heads, d128, 4 queries a row, contexts U[512, 8192], two layers, pieces of half
-  // a share / two thirds / one: 12 rows 121 / 117 / 110 us, 24 rows 193 / 192 / 182, 48 rows 346 / 353 / 336; 4 rows with
-  // their remainders beside the round 66.7, in it 57.9; 100 rows split by shares 631, unsplit 624.
+  // Steps of few queries (few_query.hip, two workgroups per CU whatever the group): a full piece is one workgroup's
+  // share of all keys, so the full pieces run in one round and the rows' remainders pack beside them; up to kFewRound
+  // / 8 rows' remainders are counted in, so that all run at once. More pieces cost more than they balance, their
+  // partials being several query rows each. 32/8 heads, d128, 4 queries a row, contexts U[512, 8192], two layers,
+  // pieces of half a share / two thirds / one: 12 rows 121 / 117 / 110 us, 24 rows 193 / 192 / 182, 48 rows 346 / 353
+  // / 336; 4 rows with their remainders beside the round 66.7, in it 57.9; 100 rows split by shares 631, unsplit 624.
   const int64_t units = rows * per_split;
-  const int64_t row_queries = few ? ((int64_t)tokens + rows - 1) / rows : 1;  // a row's on average: partial slots per split
+  const int64_t row_queries = few ? ((int64_t)tokens + rows - 1) / rows : 1;  // a row's on average
   const int64_t slot_bytes = (int64_t)hq * (d + 1) * (int64_t)sizeof(float);
   const int64_t share = std::max<int64_t>(1, kFewRound / per_split);  // splits of one round of workgroups
   int64_t pieces = std::max<int64_t>(1, share / 2);
@@ -813,13 +824,14 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   s.max_prompt_items = listed && !few ? sat(((int64_t)tokens + qp - 1) / qp + rows) : 0;
   s.max_decode_items = listed ? sat(splits) : 0;
   s.max_items = sat((int64_t)s.max_prompt_items + s.max_decode_items);
-  // Rows of more than one split hold more keys than a split, so there are at most `pieces` of them, and their splits have
-  // slots for row_queries each. In a step of few queries most keys may be in a row of more than that: slots for max_q each,
-  // where they fit in kFewPartBytes with the counters, at half the pieces (one workgroup per CU streams about as fast and
-  // leaves half the partials to merge), or one round of the light ones. One long row among short ones, us, with the split
-  // doubled until slots for the average row held it (before), and so: 32/8 heads, d128, 8 queries on 64,000 keys among 15 of
-  // one on 300 108.9 -> 74.8; 16 on 60,000 beside 9 on 5000 and two short 214 -> 136.5; 4 on 64,000 beside 7 of one on
-  // 1000 59.9 -> 60.6; 8/8 heads, 8 queries on 64,000 beside 3 of one on 4000 66.2 -> 65.8.
+  // Rows of more than one split hold more keys than a split, so there are at most `pieces` of them, and their splits
+  // have slots for row_queries each. In a step of few queries most keys may be in a row of more than that: slots for
+  // max_q each, where they fit in kFewPartBytes with the counters, at half the pieces (one workgroup per CU streams
+  // about as fast and leaves half the partials to merge), or one round of the light ones. One long row among short
+  // ones, us, with the split doubled until slots for the average row held it (before), and so: 32/8 heads, d128, 8
+  // queries on 64,000 keys among 15 of one on 300 108.9 -> 74.8; 16 on 60,000 beside 9 on 5000 and two short 214 ->
+  // 136.5; 4 on 64,000 beside 7 of one on 1000 59.9 -> 60.6; 8/8 heads, 8 queries on 64,000 beside 3 of one on 4000
+  // 66.2 -> 65.8.
   const int64_t merges = s.max_splits > 1 ? (int64_t)rows * per_split : 0;
   if (s.max_splits > 1) {
     const int64_t split_rows = std::min<int64_t>(rows, pieces);
@@ -850,7 +862,9 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   s.merges = merges;
   s.merge_off = off;
   off += (size_t)s.merges * sizeof(int32_t);
-  // Prompt items that fill less than the GPU's workgroups are split over their keys.
+  // Prompt items that fill at most two thirds of the GPU's workgroups are split over their keys, into as many pieces
+  // as come nearest to one round. Their bound counts a tile per decode row too, so a serial step's chunk beside many
+  // decode rows stays whole (512 tokens beside 32 rows of 32/8 heads: 128 items, 400 counted).
   const int64_t prompts = (int64_t)s.max_prompt_items * hkv;
   s.prompt_pieces = 1;
   if (split_prompts && prompts > 0)
@@ -1007,7 +1021,8 @@ static void launch_decode(const AttnParams& p, const Route& r, hipStream_t strea
 
 // A step's kernels after the plan. An overlapped mixed step forks the decode items onto the device's second stream
 // and joins it back into `stream` with events; if the second stream cannot be set up, or the fork's record or wait
-// fails before anything is launched, the step runs serially instead (the same results). A failure after the prompt
+// fails before anything is launched, the step runs serially instead (the same results, but for the rounding where
+// the serial schedule splits few prompt items). A failure after the prompt
 // launch leaves the two streams unordered and is returned as LV_EHIP. With `info` set nothing is launched: the
 // route is reported instead.
 template <typename T, int D, int GS, int TP, int HP>
@@ -1026,9 +1041,9 @@ static int launch(const AttnParams& p, const Shape& s, const StepKind& k, hipStr
     bool forked = false;
     if (side) {
       // The prompt items go first, to the caller's stream, then the decode items to the second one: the prompt
-      // workgroups (one per CU) are dispatched as soon as the plan ends, the decode workgroups fill the rest. On an idle
-      // GPU decode workgroups launched first fill every CU, and the prompt items start when they end: the Qwen3-8B mixed step
-      // alone 4.62 ms, so 2.95; among others 2.97 and 2.93.
+      // workgroups (one per CU) are dispatched as soon as the plan ends, the decode workgroups fill the rest. On an
+      // idle GPU decode workgroups launched first fill every CU, and the prompt items start when they end: the
+      // Qwen3-8B mixed step alone 4.62 ms, so 2.95; among others 2.97 and 2.93.
       std::lock_guard<std::mutex> g(side->lock);
       if (hipEventRecord(side->fork, stream) == hipSuccess &&
           hipStreamWaitEvent(side->stream, side->fork, 0) == hipSuccess) {
@@ -1151,12 +1166,12 @@ static int launch_step(const AttnParams& p, int d, const Shape& s, const StepKin
                                 : launch_d<F16>(p, d, s.gs, s, k, stream, info);
 }
 
-// ---------------------------------------------------------------------------------------------------------
-// The workspace of lv_paged_attention_static: file-scope device arrays (each GPU that loads the library holds its
-// own copies until the process ends), one for the lists and the rows' partials, one for the pieces of split prompt items
-// (its size covers every step that splits them). Host code must not pass an array's name to a kernel -- in host code it is
-// a stand-in, not a device address; its address on the current device comes from hipGetSymbolAddress, resolved once
-// per device and kept. The same set-up creates the device's second stream and its fork/join events, so that no
+// --------------------------------------------------------------------------------------------------------- The
+// workspace of lv_paged_attention_static: file-scope device arrays (each GPU that loads the library holds its own
+// copies until the process ends), one for the lists and the rows' partials, one for the pieces of split prompt items
+// (its size covers every step that splits them). Host code must not pass an array's name to a kernel -- in host code
+// it is a stand-in, not a device address; its address on the current device comes from hipGetSymbolAddress, resolved
+// once per device and kept. The same set-up creates the device's second stream and its fork/join events, so that no
 // later call creates anything.
 constexpr size_t kStaticPieceBytes = (size_t)kMaxPieces * kPrefillRows * (128 + 1) * sizeof(float);
 static __device__ __align__(256) char scratch[LV_STATIC_WORKSPACE_BYTES];
@@ -1280,9 +1295,9 @@ static int check_shape(int32_t num_rows, int32_t num_tokens, int32_t num_heads, 
   return LV_OK;
 }
 
-static StepKind step_kind(int32_t num_rows, int32_t num_tokens, int32_t num_heads, int32_t num_kv_heads, int32_t head_dim,
-                          bool has_cu_q, int32_t max_seqlen_q, int32_t schedule, int32_t prompt_workgroups,
-                          int32_t flags) {
+static StepKind step_kind(int32_t num_rows, int32_t num_tokens, int32_t num_heads, int32_t num_kv_heads,
+                          int32_t head_dim, bool has_cu_q, int32_t max_seqlen_q, int32_t schedule,
+                          int32_t prompt_workgroups, int32_t flags) {
   const int group = num_heads / num_kv_heads;
   const int few = few_queries(num_rows, num_kv_heads, head_dim, group);
   StepKind k;
@@ -1348,8 +1363,8 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   LV_REQUIRE(cache_stride_token >= 0 && (int64_t)kPrefillKeys * cache_stride_token * 2 < (int64_t)1 << 30,
              "paged_attention: cache token stride %lld is negative or too large", (long long)cache_stride_token);
   LV_REQUIRE(scale > 0.f, "paged_attention: the softmax scale must be positive, got %g", (double)scale);
-  const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, cu_seqlens_q != nullptr, max_seqlen_q,
-                                  schedule, prompt_workgroups, flags);
+  const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, cu_seqlens_q != nullptr,
+                                  max_seqlen_q, schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
                              kind.few, kind.max_q, kind.mixed);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);
@@ -1438,13 +1453,13 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
     int2* lists = reinterpret_cast<int2*>(ws + s.items_off);
     const PlanOut out{lists, lists + s.max_prompt_items, reinterpret_cast<int32_t*>(ws + s.count_off),
                       reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
-    // Few-query items take a row's queries from cu_seqlens_q, so its partial slots are counted from there too, also in a
-    // step that was said to have one query a row.
+    // Few-query items take a row's queries from cu_seqlens_q, so its partial slots are counted from there too, also
+    // in a step that was said to have one query a row.
     auto* const plan = num_rows <= kScanThreads ? &plan_kernel<1> : &plan_kernel<kPlanMaxRows / kScanThreads>;
     hipLaunchKernelGGL(plan, dim3(1), dim3(kScanThreads), 0, st,
-                       kind.mixed || kind.few ? cu_seqlens_q : nullptr, seqlens_k, cu_seqlens_k, num_rows, s.pieces, s.slots, qp, s.max_prompt_items,
-                       s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few, s.fewer_pieces,
-                       p.group, (int32_t)s.merges, out);
+                       kind.mixed || kind.few ? cu_seqlens_q : nullptr, seqlens_k, cu_seqlens_k, num_rows, s.pieces,
+                       s.slots, qp, s.max_prompt_items, s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few,
+                       s.fewer_pieces, p.group, (int32_t)s.merges, out);
     LV_LAUNCH_CHECK("plan_kernel");
     planned = true;
   }
@@ -1475,8 +1490,8 @@ extern "C" size_t lv_paged_attention_workspace_bytes(int32_t num_rows, int32_t n
   const bool may_be_few =
       listed && num_tokens <= (int64_t)num_rows * few_q && (mixed || pick_gs(group) != group);
   auto bytes = [&](bool few) {
-    return workspace_bytes_of(plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, listed, few,
-                                         mixed ? few_q : 1, mixed));
+    return workspace_bytes_of(plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k,
+                                         listed, few, mixed ? few_q : 1, mixed));
   };
   // The longest row's queries are not known here: a step whose rows may all have few takes the larger of the two.
   return may_be_few ? std::max(bytes(false), bytes(true)) : bytes(false);
@@ -1494,8 +1509,8 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
                               has_cu_seqlens_q != 0, max_seqlen_q, max_seqlen_k, schedule, prompt_workgroups, flags,
                               dtype);
   if (rc0 != LV_OK || num_rows == 0 || num_tokens == 0) return rc0;
-  const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, has_cu_seqlens_q != 0, max_seqlen_q,
-                                  schedule, prompt_workgroups, flags);
+  const StepKind kind = step_kind(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, has_cu_seqlens_q != 0,
+                                  max_seqlen_q, schedule, prompt_workgroups, flags);
   const Shape s = plan_shape(num_rows, num_tokens, num_heads, num_kv_heads, head_dim, max_seqlen_k, kind.listed,
                              kind.few, kind.max_q, kind.mixed);
   const int rg = check_grids(s, num_rows, num_heads, num_kv_heads);

@@ -1,5 +1,5 @@
-// Shared by the kernels that stream a row's keys in splits (paged_attention.hip, few_query.hip): the decode work list, and
-// the merge of a split row inside the launch that attends it.
+// Shared by the kernels that stream a row's keys in splits (paged_attention.hip, few_query.hip): the decode work
+// list, and the merge of a split row inside the launch that attends it.
 #pragma once
 
 #include "attn_common.h"
@@ -12,8 +12,8 @@ constexpr int kWaves = 4;  // waves per workgroup
 // query rows per kv head -- what one item's accumulators hold at two workgroups per CU.
 constexpr int kFewMaxQueries = 16;
 constexpr int kFewMaxRows = 64;
-// Launches the decode list (at most `items` items of hp kv heads each), rows of at most query_rows (position, head) query
-// rows per kv head in one pass over their keys (rows of more take several).
+// Launches the decode list (at most `items` items of hp kv heads each), rows of at most query_rows (position, head)
+// query rows per kv head in one pass over their keys (rows of more take several).
 void launch_few_query(const AttnParams& p, int d, int query_rows, int hp, int dtype, int items, hipStream_t stream);
 
 // Decode item i (below the launch's bound, so inside the list's memory), the number of decode items and the keys per
@@ -25,7 +25,8 @@ struct DecodeWork {
 __device__ __forceinline__ DecodeWork decode_work(const AttnParams& p, int i) {
   DecodeWork w;
   int64_t item;
-  asm volatile("s_load_dwordx2 %0, %3, 0x0\n\ts_load_dword %1, %4, %5\n\ts_load_dword %2, %4, %6\n\ts_waitcnt lgkmcnt(0)"
+  asm volatile("s_load_dwordx2 %0, %3, 0x0\n\ts_load_dword %1, %4, %5\n\ts_load_dword %2, %4, %6\n\t"
+               "s_waitcnt lgkmcnt(0)"
                : "=&s"(item), "=&s"(w.count), "=&s"(w.per)
                : "s"(p.items + i), "s"(p.n_items), "n"(4 * kPlanDecodes), "n"(4 * kPlanSplit));
   w.row = (int)(uint32_t)item;
@@ -54,12 +55,12 @@ __device__ __forceinline__ void coherent_load2(const float* ptr, float& a, float
   b = __uint_as_float((uint32_t)(v >> 32));
 }
 
-// Merge of a split row's partial outputs: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M). A piece is two adjacent dims of
-// one query head's output (its partials in slots slot, slot + stride, ...); a thread merges NP pieces at once, reading
-// kMergeLoads / NP splits of each at a time, every load issued before the first is used, with the max and the sums
-// carried from batch to batch. The merge is the serial end of a row's step: one round trip past the L2 per batch, and
-// one set of them per kMergeLoads loads a thread has to make. Each output element's arithmetic depends only on its own
-// head, dim and NP, so any spread of the pieces over threads gives the same bits.
+// Merge of a split row's partial outputs: o = sum_s 2^(lse_s - M) o_s / sum_s 2^(lse_s - M). A piece is two adjacent
+// dims of one query head's output (its partials in slots slot, slot + stride, ...); a thread merges NP pieces at
+// once, reading kMergeLoads / NP splits of each at a time, every load issued before the first is used, with the max
+// and the sums carried from batch to batch. The merge is the serial end of a row's step: one round trip past the L2
+// per batch, and one set of them per kMergeLoads loads a thread has to make. Each output element's arithmetic depends
+// only on its own head, dim and NP, so any spread of the pieces over threads gives the same bits.
 constexpr int kMergeLoads = 32;
 struct MergePiece {
   int slot, tok, head, d0;  // slot < 0: no piece
@@ -118,8 +119,8 @@ __device__ __forceinline__ void merge_split_partials(const AttnParams& p, const 
   }
 }
 
-// All pieces of an item, `pieces` of them (piece_of(i): piece i), by its workgroup of 64 kWaves threads; up to four at a
-// time per thread where there are that many.
+// All pieces of an item, `pieces` of them (piece_of(i): piece i), by its workgroup of 64 kWaves threads; up to four
+// at a time per thread where there are that many.
 template <typename T, int D, int NP, typename F>
 __device__ __forceinline__ void merge_pieces(const AttnParams& p, int pieces, int stride, int nsplit, F&& piece_of) {
   constexpr int NT = 64 * kWaves;
