@@ -109,6 +109,16 @@ def test_many_rows_of_drafts_take_kv_head_pairs(cuda, layout):
     assert info["kv_heads_per_item"] == 2 and info["prompt_kernel"] == "none" and info["splitk_merge"], info
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_pairs_of_two_row_blocks(cuda, dtype, dim):
+    """Items of a pair of kv heads whose query rows fill a 16-row block and spill into the next: 5 heads, up to 4 queries."""
+    new = [3, 2, 1, 4] * 65
+    cached = [(37 * i) % 90 for i in range(259)] + [6000]
+    info = _run(cuda, (20, 4), dim, dtype, new, cached, 16)
+    assert info["kv_heads_per_item"] == 2 and info["prompt_kernel"] == "none" and info["splitk_merge"], info
+
+
 def test_a_row_of_more_queries_than_the_step_says(cuda):
     """max_seqlen_q sizes the item; a row of more query rows than it holds takes several passes over its keys."""
     info = _run(cuda, (8, 2), 64, torch.bfloat16, [7, 1, 1, 1], [900, 3, 4, 5], 16, max_q=3)
