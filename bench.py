@@ -425,8 +425,6 @@ def attention_op(wl) -> str:
         return "lv_varlen_context_attention (varlen_kernel over prefix then causal new keys, one softmax)"
     if wl.is_mla:
         return "lv_mla_decode (mla_run_kernel + mla_run_merge_kernel)"
-    if all(n > 1 for n in wl.num_new):  # a step of prompts: the serial schedule, prompt tiles on the whole GPU
-        return "lv_paged_attention (plan_kernel + prompt_list_kernel)"
     # The paged steps' kernels as the committed kernel trace of this workload names them.
     f = ROOT / "profiles" / f"traffic_{wl.name}.json"
     if f.exists():
