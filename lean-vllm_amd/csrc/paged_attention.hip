@@ -738,6 +738,7 @@ struct Shape {
   int32_t max_items, max_prompt_items, max_decode_items, gs;
   int32_t pieces;      // the plan cuts the decode rows' keys into this many (0: rows are not split)
   int32_t fewer_pieces;  // few queries: and into this many where the partials of those do not fit
+  int32_t route_items; // decode items by which a mixed step's route is chosen
   int32_t max_splits;  // the most items one row may be split into
   int32_t slots;       // split rows' partial slots
   int32_t prompt_pieces;  // workgroups per prompt item outside the overlap
@@ -813,6 +814,8 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
     const int64_t splits = std::min<int64_t>((items + per_split - 1) / per_split, (int64_t)kMaxRowSplits * rows);
     if (2 * (int64_t)rows <= splits) pieces = splits - rows;
   }
+  int64_t route_split = kMinSplit;
+  while (route_split < keys && units * ((keys + route_split - 1) / route_split) > kSplitTarget) route_split *= 2;
   if (!listed || keys <= kMinSplit) pieces = 0;
   s.pieces = (int32_t)pieces;
   const int64_t most = pieces > 0 ? (keys + kMinSplit - 1) / kMinSplit : 1;  // splits of one row
@@ -824,6 +827,7 @@ static Shape plan_shape(int32_t rows, int32_t tokens, int32_t hq, int32_t hkv, i
   s.max_prompt_items = listed && !few ? sat(((int64_t)tokens + qp - 1) / qp + rows) : 0;
   s.max_decode_items = listed ? sat(splits) : 0;
   s.max_items = sat((int64_t)s.max_prompt_items + s.max_decode_items);
+  s.route_items = sat(rows * ((keys + route_split - 1) / route_split));
   // Rows of more than one split hold more keys than a split, so there are at most `pieces` of them, and their splits
   // have slots for row_queries each. In a step of few queries most keys may be in a row of more than that: slots for
   // max_q each, where they fit in kFewPartBytes with the counters, at half the pieces (one workgroup per CU streams
@@ -961,7 +965,10 @@ static int prompt_grid(const Shape& s, const AttnParams& p, int requested) {
 // - a step of prompts: its prompt items one workgroup each on the whole GPU;
 // - more rows than the work list holds (decode only): one workgroup per (row, split, item head group), no list;
 // - a mixed step under the overlapped schedule whose workgroups (bounds: prompt bounds past a row's queries exit at
-//   once) fill the GPU at most kSmallStepRounds times: prompt and decode items in one launch (mixed_small_kernel);
+//   once; decode items at a power of two of keys, the largest number up to kSplitTarget: by the finer splits that the
+//   plan may make, a step of few rows with long contexts would be a large one, 235 rows of 16/8 heads beside a 1154-token
+//   chunk 151 us a layer here and 206 there, 23 rows of 12/1 heads 61 and 80) fill the GPU at most kSmallStepRounds
+//   times: prompt and decode items in one launch (mixed_small_kernel);
 // - a larger one: prompt items on a persistent share of the CUs, decode items beside them on a second stream, on the
 //   persistent ticket grid where the item bound gives each of its workgroups at least eight items (else one
 //   workgroup per item: few short items finish sooner all at once than in rounds);
@@ -975,6 +982,7 @@ static Route route_of(const AttnParams& p, const Shape& s, const StepKind& k) {
   const int ny = p.hkv / HP * p.qgroups;
   const int cus = device_cus();
   const int64_t pw = k.listed && k.mixed ? (int64_t)s.max_prompt_items * p.hkv : 0;
+  const int64_t rw = (int64_t)s.route_items * ny;
   const int64_t dw = k.listed ? (int64_t)s.max_decode_items * ny : (int64_t)p.rows * ny;
   r.merge = s.max_splits > 1 && !k.prompts_only;
   if (k.prompts_only) {
@@ -984,7 +992,7 @@ static Route route_of(const AttnParams& p, const Shape& s, const StepKind& k) {
     r.decode = LV_KERNEL_DECODE_GRID;
     r.decode_grid = (int)dw;
   } else if (k.mixed && k.overlap &&
-             pw + dw <= (int64_t)kSmallStepRounds * resident_per_cu<mixed_small_kernel<T, D, GS, TP, HP>>() * cus) {
+             pw + rw <= (int64_t)kSmallStepRounds * resident_per_cu<mixed_small_kernel<T, D, GS, TP, HP>>() * cus) {
     r.prompt = r.decode = LV_KERNEL_MIXED_SMALL;
     r.prompt_grid = (int)pw;
     r.decode_grid = (int)dw;
@@ -993,7 +1001,7 @@ static Route route_of(const AttnParams& p, const Shape& s, const StepKind& k) {
     r.prompt = LV_KERNEL_PROMPT_OVERLAP;
     r.prompt_grid = prompt_grid(s, p, k.prompt_wgs);
     const int grid = std::min(kOverlapDecodeWgs, resident_per_cu<decode_beside_kernel<T, D, GS, HP>>()) * cus;
-    r.decode = dw >= 8 * (int64_t)grid ? LV_KERNEL_DECODE_BESIDE : LV_KERNEL_DECODE_LIST;
+    r.decode = rw >= 8 * (int64_t)grid ? LV_KERNEL_DECODE_BESIDE : LV_KERNEL_DECODE_LIST;
     r.decode_grid = r.decode == LV_KERNEL_DECODE_BESIDE ? grid : (int)dw;
   } else {
     if (k.mixed) {

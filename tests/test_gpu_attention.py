@@ -831,3 +831,17 @@ def test_the_plan_lists_every_split_once_longest_first(cuda, monkeypatch, rows):
     assert last[first_last:].all()
     lasts = keys[first_last:]
     assert (lasts[1:] - lasts[:-1]).max() <= split / 64 + 1 if rows > 1 else True
+
+
+@pytest.mark.parametrize("hq, hkv, bs, rows, tokens, max_q, max_k", [(16, 8, 64, 235, 1498, 1154, 5906),
+                                                                     (12, 1, 16, 23, 388, 305, 19_352),
+                                                                     (16, 2, 16, 48, 245, 198, 12_559)])
+def test_a_mixed_step_of_few_rows_is_one_launch_whatever_its_contexts(cuda, hq, hkv, bs, rows, tokens, max_q, max_k):
+    """The route of a mixed step goes by the work that its bounds allow, not by the finer splits that the plan may make: the
+    overlapped form of these steps takes 1.2 to 1.4 times as long."""
+    from lvattn import _capi
+    from lvattn import backend as B
+
+    info = _capi.launch_info(rows, tokens, hq, hkv, 128, bs, 128, 1, max_q, max_k, B.SCHEDULE_OVERLAP, 0, 0,
+                             _capi.DTYPES[torch.bfloat16])
+    assert info["prompt_kernel"] == info["decode_kernel"] == "mixed_small" and not info["two_streams"], info
