@@ -557,12 +557,12 @@ __device__ inline int len_bucket(int short_of, float per_key) {
 // faster than first tile first. Beside the decode rows (the overlapped schedule) the order made no measurable
 // difference, and the first tile goes first there as before. The split rows' merge counters start at zero.
 //
-// Keys per decode split: the decode rows' own keys over `pieces`, at least kMinSplit and a multiple of kSplitStep, so
-// that a step is cut into about the same number of items whatever its lengths (at most pieces + rows). The caller's
-// bound on key lengths only sizes the buffers: a captured graph's bound is the longest context it may ever serve, and
-// a batch of a few rows far apart in length has most of its keys in one of them. pieces 0: rows are not split, and
-// one split holds the longest row. The partials of split rows lie in consecutive slots from part_base[row]. few: rows
-// of several queries are streamed as decode items too, one slot per query and split.
+// Keys per decode split: the decode rows' own keys over `pieces`, at least kMinSplit (or two) and a multiple of
+// kSplitStep, so that a step is cut into about the same number of items whatever its lengths (at most pieces + rows).
+// The caller's bound on key lengths only sizes the buffers: a captured graph's bound is the longest context it may
+// ever serve, and a batch of a few rows far apart in length has most of its keys in one of them. pieces 0: rows are
+// not split, and one split holds the longest row. The partials of split rows lie in consecutive slots from
+// part_base[row]. few: rows of several queries are streamed as decode items too, one slot per query and split.
 //
 // few: a row's merge is one workgroup's work, and takes as long as its splits where they hold `least` keys: n splits
 // of lk keys take lk / n keys' stream (12 KB a microsecond) and lq G D n / 512 loads a thread (19 a microsecond),
@@ -575,7 +575,11 @@ __device__ inline int len_bucket(int short_of, float per_key) {
 __host__ __device__ inline int least_split(int lk, int query_rows) {
   return (int)sqrtf(0.3f * (float)(lk > 0 ? lk : 0) * (float)query_rows);
 }
-__host__ __device__ inline int split_keys(float keys, int longest, int least, int pieces) {
+// VALU items (few: kv_heads 0): two kMinSplit where that still gives every CU an item of its own kv head. Over 80
+// decode steps of random shapes 3% faster than kMinSplit everywhere (one to nine long rows of one or two kv heads
+// 15-35%), over 120 mixed steps 1%; one row of 8K keys of 8 kv heads, below the line, 34.6 us against 40.1 with it.
+__host__ __device__ inline int split_keys(float keys, int longest, int least, int pieces, int kv_heads) {
+  if (keys * (float)kv_heads >= 2.f * kMinSplit * (kFewRound / 2) && least < 2 * kMinSplit) least = 2 * kMinSplit;
   int64_t want = longest;
   if (pieces > 0) {
     int64_t share = (int64_t)(keys * 1.00001f / (float)pieces) + 1;
@@ -605,7 +609,8 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
                                                             int32_t pieces, int32_t max_slots, int32_t qp,
                                                             int32_t max_prompts, int32_t max_items,
                                                             int32_t last_first, int32_t few, int32_t fewer_pieces,
-                                                            int32_t group, int32_t n_merge, PlanOut out) {
+                                                            int32_t group, int32_t kv_heads, int32_t n_merge,
+                                                            PlanOut out) {
   __shared__ int pre[ROWS * kScanThreads + 1];
   __shared__ int full[ROWS * kScanThreads + 1];
   __shared__ int slots[ROWS * kScanThreads + 1];
@@ -654,7 +659,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
     longest = max(longest, wave_max_of[w]);
     least = max(least, wave_least[w]);
   }
-  int split = split_keys(keys, longest, least, pieces);
+  int split = split_keys(keys, longest, least, pieces, few ? 0 : kv_heads);
   for (;;) {  // every thread leaves together: slots[rows] is the same for all, and split reaches the longest row
 #pragma unroll
     for (int i = 0; i < ROWS; ++i) {
@@ -966,9 +971,9 @@ static int prompt_grid(const Shape& s, const AttnParams& p, int requested) {
 // - more rows than the work list holds (decode only): one workgroup per (row, split, item head group), no list;
 // - a mixed step under the overlapped schedule whose workgroups (bounds: prompt bounds past a row's queries exit at
 //   once; decode items at a power of two of keys, the largest number up to kSplitTarget: by the finer splits that the
-//   plan may make, a step of few rows with long contexts would be a large one, 235 rows of 16/8 heads beside a 1154-token
-//   chunk 151 us a layer here and 206 there, 23 rows of 12/1 heads 61 and 80) fill the GPU at most kSmallStepRounds
-//   times: prompt and decode items in one launch (mixed_small_kernel);
+//   plan may make, a step of few rows with long contexts would be a large one, 235 rows of 16/8 heads beside a
+//   1154-token chunk 151 us a layer here and 206 there, 23 rows of 12/1 heads 61 and 80) fill the GPU at most
+//   kSmallStepRounds times: prompt and decode items in one launch (mixed_small_kernel);
 // - a larger one: prompt items on a persistent share of the CUs, decode items beside them on a second stream, on the
 //   persistent ticket grid where the item bound gives each of its workgroups at least eight items (else one
 //   workgroup per item: few short items finish sooner all at once than in rounds);
@@ -1467,7 +1472,7 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
     hipLaunchKernelGGL(plan, dim3(1), dim3(kScanThreads), 0, st,
                        kind.mixed || kind.few ? cu_seqlens_q : nullptr, seqlens_k, cu_seqlens_k, num_rows, s.pieces,
                        s.slots, qp, s.max_prompt_items, s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few,
-                       s.fewer_pieces, p.group, (int32_t)s.merges, out);
+                       s.fewer_pieces, p.group, p.hkv, (int32_t)s.merges, out);
     LV_LAUNCH_CHECK("plan_kernel");
     planned = true;
   }
@@ -1536,7 +1541,7 @@ extern "C" int lv_paged_attention_launch_info(int32_t num_rows, int32_t num_toke
   info->two_streams = r.two_streams;
   const int least = kind.few ? least_split(max_seqlen_k, std::min(kind.max_q, num_tokens) * p.group) : 0;
   info->keys_per_split = split_keys((float)num_rows * (float)max_seqlen_k, std::max(max_seqlen_k, 1),
-                                    std::max(kMinSplit, least), s.pieces);
+                                    std::max(kMinSplit, least), s.pieces, kind.few ? 0 : num_kv_heads);
   info->max_splits = s.max_splits;
   info->splitk_merge = r.merge;
   return LV_OK;

@@ -845,3 +845,24 @@ def test_a_mixed_step_of_few_rows_is_one_launch_whatever_its_contexts(cuda, hq, 
     info = _capi.launch_info(rows, tokens, hq, hkv, 128, bs, 128, 1, max_q, max_k, B.SCHEDULE_OVERLAP, 0, 0,
                              _capi.DTYPES[torch.bfloat16])
     assert info["prompt_kernel"] == info["decode_kernel"] == "mixed_small" and not info["two_streams"], info
+
+
+@pytest.mark.parametrize("keys, least", [(1984, 256), (2048, 512)])
+def test_decode_items_hold_512_keys_where_they_fill_the_gpu(cuda, monkeypatch, keys, least):
+    """32 rows of two kv heads: 256 items of 512 keys, or just less, where items hold 256."""
+    rows, hq, hkv, dim, bs = 32, 8, 2, 64, 64
+    ws = guarded_workspace(monkeypatch, cuda)
+    b = MI355XAttention(hq, dim, 1 / math.sqrt(dim), hkv)
+    kc, vc = (torch.randn(keys // bs, bs, hkv, dim, device=cuda).to(torch.bfloat16) for _ in range(2))
+    ctx = Context(context_lens=torch.full((rows,), keys, dtype=torch.int32, device=cuda),
+                  block_tables=torch.arange(keys // bs, dtype=torch.int32, device=cuda).repeat(rows, 1))
+    q = torch.randn(rows, hq, dim, device=cuda).to(torch.bfloat16)
+    b.launch_trace = []
+    out = b.decode(q, kc, vc, ctx)
+    torch.cuda.synchronize()
+    info = b.launch_trace[-1]
+    items, split = plan_counts(ws, 1 + rows + info["decode_workgroups"] * info["kv_heads_per_item"] // hkv)
+    assert split == info["keys_per_split"] == least and items == rows * -(-keys // split)
+    want = dense_expected([q[i:i + 1] for i in range(rows)], [kc.flatten(0, 1)] * rows, [vc.flatten(0, 1)] * rows,
+                          1 / math.sqrt(dim))
+    torch.testing.assert_close(out.float().cpu(), want, atol=2e-2, rtol=1e-2)
