@@ -602,7 +602,10 @@ struct PlanOut {
 // plan meets cold: the rows' loads are issued together, once, and all that is known of a row stays in registers. 3 /
 // 256 / 1024 / 4096 rows of a decode step 6.0 / 6.4 / 7.4 / 12.8 us with later rows loaded again in each pass and
 // 64-bit bucket divisions, 5.4 / 5.9 / 6.6 / 10.4 so (with splits of a size fixed on the host 5.6 / 4.5 / 5.0 / 8.9).
-template <int ROWS>
+// PROMPTS: the caller says that no row is a decode row (LV_ATTN_PROMPTS_ONLY), so no split is sized and no decode item
+// listed: a step of one or two short prompts, whose layers take 9 us each, 2.5 us instead of 4.9 (1100
+// rows 4.4 instead of 7.8).
+template <int ROWS, bool PROMPTS>
 __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __restrict__ cu_q,
                                                             const int32_t* __restrict__ lens_k,
                                                             const int32_t* __restrict__ cu_k, int32_t rows,
@@ -629,6 +632,40 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
       lq[i] = cu_q ? cu_q[r + 1] - cu_q[r] : 1;
       lk[i] = lens_k ? lens_k[r] : cu_k[r + 1] - cu_k[r];
     }
+  }
+  // Prompt items and full splits, one thread each (a few long rows hold hundreds: a thread per row would write them
+  // one by one, 9 us for seven prompts' 260 items, 5 so).
+  auto row_of = [&](const int* before, int i) {  // the last row with at most i items before its own
+    int lo = 0, hi = rows - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (before[mid] <= i) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+  };
+  auto list_prompts = [&] {
+    for (int i = tid; i < min(pre[rows], max_prompts); i += kScanThreads) {
+      const int r = row_of(pre, i);
+      out.prompts[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
+    }
+  };
+  if constexpr (PROMPTS) {
+    __shared__ int prompt_tot[1][kScanThreads / 64];
+    for (int i = tid; i < n_merge; i += kScanThreads) out.merge_count[i] = 0;
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i)
+      if (tid + i * kScanThreads < rows) pre[tid + i * kScanThreads] = lq[i] > 1 ? (lq[i] + qp - 1) / qp : 0;
+    __syncthreads();
+    block_scan(pre, rows, prompt_tot);
+    list_prompts();
+    if (tid == 0) {
+      out.counts[kPlanDecodes] = 0;
+      out.counts[kPlanPrompts] = min(pre[rows], max_prompts);
+      out.counts[kPlanTicket] = 0;
+      out.counts[kPlanDone] = 0;
+      out.counts[kPlanSplit] = kSplitStep;
+    }
+    return;
   }
   auto streamed = [&](int i) { return few ? lq[i] > 0 : lq[i] == 1; };  // a row of decode items
   for (int b = tid; b <= kLenBuckets; b += kScanThreads) bucket[b] = 0;
@@ -703,20 +740,7 @@ __global__ __launch_bounds__(kScanThreads) void plan_kernel(const int32_t* __res
   }
   __syncthreads();
   const int npre = pre[rows], nfull = full[rows], npart = bucket[kLenBuckets];
-  // Prompt items and full splits, one thread each (a few long rows hold hundreds: a thread per row would write them
-  // one by one, 9 us for seven prompts' 260 items, 5 so).
-  auto row_of = [&](const int* before, int i) {  // the last row with at most i items before its own
-    int lo = 0, hi = rows - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (before[mid] <= i) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-  };
-  for (int i = tid; i < min(npre, max_prompts); i += kScanThreads) {
-    const int r = row_of(pre, i);
-    out.prompts[i] = make_int2(r, -1 - (last_first ? pre[r + 1] - 1 - i : i - pre[r]));
-  }
+  list_prompts();
   for (int i = tid; i < min(nfull, max_items); i += kScanThreads) {
     const int r = row_of(full, i);
     out.items[i] = make_int2(r, i - full[r]);
@@ -1232,12 +1256,12 @@ struct PlanSig {
   const void* ws = nullptr;
   const int32_t *cu_q = nullptr, *lens = nullptr, *cu_k = nullptr;
   int64_t rows = 0, tokens = 0, max_k = 0, pieces = 0, slots = 0, qp = 0, max_items = 0, merge_off = 0, bytes = 0;
-  bool mixed = false, last_first = false, few = false;
+  bool mixed = false, last_first = false, few = false, prompts = false;
   bool operator==(const PlanSig& o) const {
     return ws == o.ws && cu_q == o.cu_q && lens == o.lens && cu_k == o.cu_k && rows == o.rows &&
            tokens == o.tokens && max_k == o.max_k && pieces == o.pieces && slots == o.slots && qp == o.qp &&
            max_items == o.max_items && merge_off == o.merge_off && bytes == o.bytes && mixed == o.mixed &&
-           last_first == o.last_first && few == o.few;
+           last_first == o.last_first && few == o.few && prompts == o.prompts;
   }
 };
 constexpr int kPlanRecords = 32;
@@ -1459,6 +1483,7 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
   sig.bytes = (int64_t)s.bytes;
   sig.mixed = kind.mixed;
   sig.few = kind.few;
+  sig.prompts = kind.prompts_only && !kind.few;
   sig.last_first = kind.prompts_only || !kind.overlap;  // prompt items with the GPU to themselves: last tile first
   bool planned = false;
   if (kind.listed && !plan_is_current(sig, (flags & LV_ATTN_REUSE_PLAN) != 0)) {
@@ -1468,7 +1493,10 @@ static int paged_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h
                       reinterpret_cast<int32_t*>(ws + s.base_off), p.merge_count};
     // Few-query items take a row's queries from cu_seqlens_q, so its partial slots are counted from there too, also
     // in a step that was said to have one query a row.
-    auto* const plan = num_rows <= kScanThreads ? &plan_kernel<1> : &plan_kernel<kPlanMaxRows / kScanThreads>;
+    constexpr int kMany = kPlanMaxRows / kScanThreads;
+    const bool many = num_rows > kScanThreads;
+    auto* const plan = sig.prompts ? (many ? &plan_kernel<kMany, true> : &plan_kernel<1, true>)
+                                   : (many ? &plan_kernel<kMany, false> : &plan_kernel<1, false>);
     hipLaunchKernelGGL(plan, dim3(1), dim3(kScanThreads), 0, st,
                        kind.mixed || kind.few ? cu_seqlens_q : nullptr, seqlens_k, cu_seqlens_k, num_rows, s.pieces,
                        s.slots, qp, s.max_prompt_items, s.max_decode_items, (int32_t)sig.last_first, (int32_t)kind.few,

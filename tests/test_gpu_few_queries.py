@@ -179,3 +179,21 @@ def test_few_prompt_items_are_split_over_their_keys(cuda, dtype, dim, new, cache
         assert info["prompt_workgroups"] > items * hkv, info
     else:  # beside a decode row the schedule may overlap
         assert min(new) == 1, info
+
+
+@pytest.mark.parametrize("rows", [1, 1024, 1025, 1300])
+def test_a_step_of_prompts_lists_every_tile_once(cuda, monkeypatch, rows):
+    """Rows of more queries than few-query items take, on both sides of the plan's rows per thread: the prompt tiles that the
+    plan left in the workspace, last tile of a row first, no decode item, and the step's outputs against the oracle."""
+    hq, hkv, dim, bs = 8, 1, 64, 16
+    new = [17 + (7 * r) % 20 for r in range(rows)]
+    ws = guarded_workspace(monkeypatch, cuda)
+    info = _run(cuda, (hq, hkv), dim, torch.bfloat16, new, [0] * rows, bs)
+    assert info["prompt_kernel"] == "prompt_list" and info["decode_kernel"] == "none", info
+    qp = 128 // hq
+    listed = -(-sum(new) // qp) + rows
+    tiles = [(r, -1 - t) for r, n in enumerate(new) for t in reversed(range(-(-n // qp)))]
+    assert ws[:8 * len(tiles)].view(torch.int32).view(-1, 2).tolist() == [list(t) for t in tiles]
+    # The decode items' room behind the prompt items': one unsplit item a row.
+    items, _ = plan_counts(ws, listed + rows)
+    assert items == 0
